@@ -16,10 +16,10 @@
 //                        (ReLU, bfloat16 weights, FP32 accumulation), RS = RS_prev e^y,
 //                        rule value where the fallback flag is set, h2 written into the
 //                        regf i-block.
-//  * rsnet_grad_kernel / rsnet_sum_kernel / rsnet_adam_kernel   training: per-block
-//                        forward + backward of 64 samples with activations in LDS,
-//                        a fixed-order sum of the block partials, Adam on FP32 master
-//                        weights with a bfloat16 copy for the forward pass.
+//  * rsnet_grad_kernel / rsnet_sum_kernel   training: per-block forward + backward of
+//                        64 samples with activations in LDS; a fixed-order sum of the
+//                        block partials, and Adam on FP32 master weights with a bfloat16
+//                        copy for the forward pass.
 #include "nb6_internal.h"
 
 #include <hipcub/hipcub.hpp>
@@ -67,15 +67,31 @@ struct SW {
     float w1[NH * NF], b1[NH], w2[NH * (NH + 1)], b2[NH], w3[NH], b3;
 };
 
+// bfloat16 weights (two per 32-bit load) into LDS by BS threads: every load is in flight
+// before the first is used
+template <int BS>
 __device__ __forceinline__ void load_weights(SW &s, const uint16_t *__restrict__ w) {
-    for (int k = threadIdx.x; k < NPARAM; k += blockDim.x) {
-        const float v = bf16_to_f32(w[k]);
-        if (k < OFF_B1) s.w1[k] = v;
-        else if (k < OFF_W2) s.b1[k - OFF_B1] = v;
-        else if (k < OFF_B2) { const int q = k - OFF_W2; s.w2[(q / NH) * (NH + 1) + q % NH] = v; }
-        else if (k < OFF_W3) s.b2[k - OFF_B2] = v;
-        else if (k < OFF_B3) s.w3[k - OFF_W3] = v;
-        else s.b3 = v;
+    constexpr int NW = (NPARAM + 1) / 2, PER = (NW + BS - 1) / BS;
+    const uint32_t *w2 = reinterpret_cast<const uint32_t *>(w);   // (NPARAM + 1 allocated)
+    uint32_t v[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int k = q * BS + (int)threadIdx.x;
+        v[q] = k < NW ? w2[k] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int k = 2 * (q * BS + (int)threadIdx.x) + h;
+            const float f = bf16_to_f32((uint16_t)(h ? v[q] >> 16 : v[q]));
+            if (k < OFF_B1) s.w1[k] = f;
+            else if (k < OFF_W2) s.b1[k - OFF_B1] = f;
+            else if (k < OFF_B2) { const int m = k - OFF_W2; s.w2[(m / NH) * (NH + 1) + m % NH] = f; }
+            else if (k < OFF_W3) s.b2[k - OFF_B2] = f;
+            else if (k < OFF_B3) s.w3[k - OFF_W3] = f;
+            else if (k == OFF_B3) s.b3 = f;
+        }
     }
 }
 
@@ -113,96 +129,115 @@ struct GradLds {
     float dy[GB];
 };
 
-// 64 x 64 x 64 products of the hidden layer on the matrix cores, one wavefront:
-// C[m][n] = sum_k A(m, k) B(k, n), A and B read through the callables (LDS), each
-// element of C handed to out(m, n, c).  v_mfma_f32_16x16x4f32 (FP32 in, FP32
+// 64 x 64 x 64 products of the hidden layer on the matrix cores, rows 16 mt .. 16 mt + 15
+// by one wavefront: C[m][n] = sum_k A(m, k) B(k, n), A and B read through the callables
+// (LDS), each element of C handed to out(m, n, c).  v_mfma_f32_16x16x4f32 (FP32 in, FP32
 // accumulate): lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] of a 16 x 4 and
 // a 4 x 16 block, and holds C[4 (l / 16) + i][l % 16], i = 0..3, of the 16 x 16 block.
 typedef float v4f __attribute__((ext_vector_type(4)));
 template <class FA, class FB, class FO>
-__device__ __forceinline__ void gemm64(FA a, FB b, FO out, int lane) {
+__device__ __forceinline__ void gemm64(FA a, FB b, FO out, int lane, int mt) {
     const int r = lane & 15, q = lane >> 4;
-    for (int mt = 0; mt < 4; mt++) {
-        v4f acc[4];
+    v4f acc[4];
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) acc[nt] = v4f{0.f, 0.f, 0.f, 0.f};
-        for (int kb = 0; kb < NH; kb += 4) {
-            const float av = a(mt * 16 + r, kb + q);
+    for (int nt = 0; nt < 4; nt++) acc[nt] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int kb = 0; kb < NH; kb += 4) {
+        const float av = a(mt * 16 + r, kb + q);
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++)
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b(kb + q, nt * 16 + r), acc[nt],
-                                                               0, 0, 0);
-        }
+        for (int nt = 0; nt < 4; nt++)
+            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b(kb + q, nt * 16 + r), acc[nt], 0,
+                                                           0, 0);
+    }
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
+    for (int nt = 0; nt < 4; nt++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) out(mt * 16 + q * 4 + i, nt * 16 + r, acc[nt][i]);
-        }
+        for (int i = 0; i < 4; i++) out(mt * 16 + q * 4 + i, nt * 16 + r, acc[nt][i]);
     }
 }
 
 // Minibatch of n samples: sample s is row idx[base + s] (idx null: base + s) of the
-// SoA features float[8][fstride] and of the targets.  One wavefront per 64 samples:
-// the 8 -> 64 layer and the gradients of W1, b1, W3, b3 on the VALU, the three 64 x 64
-// products of the hidden layer (forward, dW2, back-propagated delta) on the matrix
-// cores.
-__global__ __launch_bounds__(GB) void rsnet_grad_kernel(int n, const float *__restrict__ feat,
-                                                        const float *__restrict__ tgt,
-                                                        const int *__restrict__ idx, int base,
-                                                        int fstride,
-                                                        const uint16_t *__restrict__ wbf,
-                                                        const float *__restrict__ norm,
-                                                        float *__restrict__ part,
-                                                        float *__restrict__ lpart) {
+// SoA features float[8][fstride] and of the targets.  64 samples per work-group of
+// GW wavefronts: the 8 -> 64 layer and the gradients of W1, b1, W3, b3 on the VALU, the
+// three 64 x 64 products of the hidden layer (forward, dW2, back-propagated delta) on
+// the matrix cores.  Bound by the latency of its chain of short LDS passes (a batch of
+// 8,192 is only 128 work-groups), so each pass is dealt to four wavefronts: wavefront w
+// takes rows 16 w .. of every product and outputs 16 w .. of the layer-1 loop, each sum
+// in the order that one wavefront would take it (same bits).  Batch of 8,192: 49.8 us
+// with one wavefront per work-group, 19.5 us with four, 15.6 us with the weights' loads
+// issued together (load_weights).
+constexpr int GW = 4;
+static_assert(GW * 16 == NH && GW * 16 == GB, "one 16-row tile per wavefront");
+__global__ __launch_bounds__(64 * GW) void rsnet_grad_kernel(
+    int n, const float *__restrict__ feat, const float *__restrict__ tgt,
+    const int *__restrict__ idx, int base, int fstride, const uint16_t *__restrict__ wbf,
+    const float *__restrict__ norm, float *__restrict__ part, float *__restrict__ lpart) {
     __shared__ GradLds L;
-    load_weights(L.w, wbf);
-    const int t = threadIdx.x;
+    const int t = threadIdx.x & 63;      // sample of the block; output of the VALU sums
+    const int w = threadIdx.x >> 6;
     const int s = blockIdx.x * GB + t;
     const bool ok = s < n;
     const int g = ok ? (idx ? idx[base + s] : base + s) : 0;
+    const float tg = ok ? tgt[g] : 0.f;
     float x[NF];
     if (ok) load_features(feat, fstride, g, norm, x);
     else
         for (int f = 0; f < NF; f++) x[f] = 0.f;
+    load_weights<64 * GW>(L.w, wbf);
     __syncthreads();
-    // layer 1 (VALU): h1 of this lane's sample into LDS
+    // layer 1 (VALU): 16 of h1 of this lane's sample into LDS
 #pragma unroll
-    for (int k = 0; k < NH; k++) {
+    for (int q = 0; q < 16; q++) {
+        const int k = w * 16 + q;
         float z = L.w.b1[k];
 #pragma unroll
         for (int f = 0; f < NF; f++) z = fmaf(L.w.w1[k * NF + f], x[f], z);
         L.h1[t][k] = fmaxf(z, 0.f);
     }
+    if (w == 0) {
 #pragma unroll
-    for (int f = 0; f < NF; f++) L.x[t][f] = x[f];
+        for (int f = 0; f < NF; f++) L.x[t][f] = x[f];
+    }
     __syncthreads();
     // layer 2 (matrix cores): h2[s][o] = relu(b2[o] + sum_k h1[s][k] W2[o][k]) into d2
     gemm64([&](int m, int k) { return L.h1[m][k]; },
            [&](int k, int o) { return L.w.w2[o * (NH + 1) + k]; },
-           [&](int m, int o, float z) { L.d2[m][o] = fmaxf(z + L.w.b2[o], 0.f); }, t);
+           [&](int m, int o, float z) { L.d2[m][o] = fmaxf(z + L.w.b2[o], 0.f); }, t, w);
     __syncthreads();
+    // every wavefront forms y of all samples (its copy of the same sum)
     float y = L.w.b3;
+#pragma unroll 16
     for (int o = 0; o < NH; o++) y = fmaf(L.w.w3[o], L.d2[t][o], y);
-    const float r = ok ? y - tgt[g] : 0.f;
+    const float r = ok ? y - tg : 0.f;
     const float dy = 2.0f * r / (float)n;
-    L.dy[t] = dy;
+    if (w == 0) L.dy[t] = dy;
     __syncthreads();
 
     float *P = part + (size_t)blockIdx.x * NPARAM;
-    // w3, b3 from h2 (still in d2)
-    {
+    // w3, b3 from h2 (still in d2); the loss partial: sum of r^2 over the block
+    if (w == 0) {
         float gw = 0.f;
+#pragma unroll 16
         for (int q = 0; q < GB; q++) gw = fmaf(L.dy[q], L.d2[q][t], gw);
         P[OFF_W3 + t] = gw;
+    } else if (w == 1) {
         if (t == 0) {
             float gb = 0.f;
+#pragma unroll 16
             for (int q = 0; q < GB; q++) gb += L.dy[q];
             P[OFF_B3] = gb;
         }
+    } else if (w == 2) {
+        float v = r * r;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if (t == 0) lpart[blockIdx.x] = v;
     }
     __syncthreads();
     // delta2 = dy w3 [h2 > 0], in place of h2
-    for (int o = 0; o < NH; o++) {
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const int o = w * 16 + q;
         const float h2 = L.d2[t][o];
         L.d2[t][o] = h2 > 0.f ? dy * L.w.w3[o] : 0.f;
     }
@@ -210,9 +245,10 @@ __global__ __launch_bounds__(GB) void rsnet_grad_kernel(int n, const float *__re
     // dW2[o][k] = sum_s delta2[s][o] h1[s][k] (matrix cores); b2 = sum_s delta2[s][o]
     gemm64([&](int o, int q) { return L.d2[q][o]; },
            [&](int q, int k) { return L.h1[q][k]; },
-           [&](int o, int k, float v) { P[OFF_W2 + o * NH + k] = v; }, t);
-    {
+           [&](int o, int k, float v) { P[OFF_W2 + o * NH + k] = v; }, t, w);
+    if (w == 0) {
         float gb = 0.f;
+#pragma unroll 16
         for (int q = 0; q < GB; q++) gb += L.d2[q][t];
         P[OFF_B2 + t] = gb;
     }
@@ -221,51 +257,101 @@ __global__ __launch_bounds__(GB) void rsnet_grad_kernel(int n, const float *__re
     // each element is read (for the mask) and written by the same lane only
     gemm64([&](int m, int o) { return L.d2[m][o]; },
            [&](int o, int k) { return L.w.w2[o * (NH + 1) + k]; },
-           [&](int m, int k, float v) { L.h1[m][k] = L.h1[m][k] > 0.f ? v : 0.f; }, t);
+           [&](int m, int k, float v) { L.h1[m][k] = L.h1[m][k] > 0.f ? v : 0.f; }, t, w);
     __syncthreads();
-    // W1 (row k = t), b1
+    // W1 (row k = t; wavefront w: features 2 w, 2 w + 1), b1
     {
         const int k = t;
-        float acc[NF];
-#pragma unroll
-        for (int f = 0; f < NF; f++) acc[f] = 0.f;
-        float gb = 0.f;
+        float a0 = 0.f, a1 = 0.f, gb = 0.f;
+#pragma unroll 16
         for (int q = 0; q < GB; q++) {
             const float d = L.h1[q][k];
             gb += d;
-#pragma unroll
-            for (int f = 0; f < NF; f++) acc[f] = fmaf(d, L.x[q][f], acc[f]);
+            a0 = fmaf(d, L.x[q][2 * w], a0);
+            a1 = fmaf(d, L.x[q][2 * w + 1], a1);
         }
-#pragma unroll
-        for (int f = 0; f < NF; f++) P[OFF_W1 + k * NF + f] = acc[f];
-        P[OFF_B1 + k] = gb;
-    }
-    // loss partial: sum of r^2 over the block
-    {
-        float v = r * r;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (t == 0) lpart[blockIdx.x] = v;
+        P[OFF_W1 + k * NF + 2 * w] = a0;
+        P[OFF_W1 + k * NF + 2 * w + 1] = a1;
+        if (w == 0) P[OFF_B1 + k] = gb;
     }
 }
 
-// fixed-order sum over the block partials (deterministic)
+struct Adam {
+    float *w, *m1, *m2;              // master weights and moments (w null: gradient only)
+    uint16_t *wbf;
+    float lr, c1, c2;
+};
+
+// Fixed-order sum over the block partials (deterministic), SUMP parameters per
+// work-group, and with ad.w the Adam step of those parameters.  Bound by the latency of
+// reading nblk partials per parameter: the wavefronts read SUMB of them at once into LDS
+// and one adds them in block order.  128 partials: 4.8 us; one thread per
+// parameter walking the partials took 33.9 us, and a kernel of its own for Adam 4.8 us.
+// A training epoch of 131,072 samples in batches of 8,192: 1552 -> 510 us.
+constexpr int SUMP = 64, SUMB = 128;
 __global__ __launch_bounds__(256) void rsnet_sum_kernel(const float *__restrict__ part, int nblk,
                                                         float *__restrict__ grad,
                                                         const float *__restrict__ lpart,
                                                         float *__restrict__ loss, int n,
-                                                        double *__restrict__ lacc) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p < NPARAM) {
-        float g = 0.f;
-        for (int b = 0; b < nblk; b++) g += part[(size_t)b * NPARAM + p];
-        grad[p] = g;
-    }
-    if (p == NPARAM) {
+                                                        double *__restrict__ lacc, Adam ad) {
+    __shared__ float sh[SUMB][SUMP];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (blockIdx.x == gridDim.x - 1) {
+        // the last work-group: the loss (one lane adds in block order)
         double l = 0.0;
-        for (int b = 0; b < nblk; b++) l += lpart[b];
-        *loss = (float)(l / n);
-        if (lacc) *lacc += l;   // sum of squared residuals over an epoch
+        float *lb = &sh[0][0];
+        for (int b0 = 0; b0 < nblk; b0 += SUMB * SUMP) {
+            const int c = min(SUMB * SUMP, nblk - b0);
+            __syncthreads();
+            for (int b = threadIdx.x; b < c; b += 256) lb[b] = lpart[b0 + b];
+            __syncthreads();
+            if (threadIdx.x == 0) {
+#pragma unroll 8
+                for (int b = 0; b < c; b++) l += lb[b];
+            }
+        }
+        if (threadIdx.x == 0) {
+            *loss = (float)(l / n);
+            if (lacc) *lacc += l;   // sum of squared residuals over an epoch
+        }
+        return;
+    }
+    const int p = blockIdx.x * SUMP + lane;
+    const bool ok = p < NPARAM;
+    float g = 0.f, wp = 0.f, a1 = 0.f, a2 = 0.f;
+    if (w == 0 && ok && ad.w) {
+        wp = ad.w[p];
+        a1 = ad.m1[p];
+        a2 = ad.m2[p];
+    }
+    for (int b0 = 0; b0 < nblk; b0 += SUMB) {
+        const int c = min(SUMB, nblk - b0);
+        __syncthreads();
+        float v[SUMB / 4];
+#pragma unroll
+        for (int q = 0; q < SUMB / 4; q++) {
+            const int b = q * 4 + w;
+            v[q] = ok && b < c ? part[(size_t)(b0 + b) * NPARAM + p] : 0.f;
+        }
+#pragma unroll
+        for (int q = 0; q < SUMB / 4; q++) sh[q * 4 + w][lane] = v[q];
+        __syncthreads();
+        if (w == 0) {
+#pragma unroll 16
+            for (int b = 0; b < c; b++) g += sh[b][lane];
+        }
+    }
+    if (w != 0 || !ok) return;
+    if (grad) grad[p] = g;
+    if (ad.w) {
+        const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+        const float a = fmaf(b1, a1, (1.f - b1) * g);
+        const float v = fmaf(b2, a2, (1.f - b2) * g * g);
+        ad.m1[p] = a;
+        ad.m2[p] = v;
+        const float wn = wp - ad.lr * (a / ad.c1) / (sqrtf(v / ad.c2) + eps);
+        ad.w[p] = wn;
+        ad.wbf[p] = f32_to_bf16(wn);
     }
 }
 
@@ -285,24 +371,6 @@ __global__ __launch_bounds__(256) void rsnet_keys_kernel(int n, unsigned long lo
 
 __global__ void rsnet_zero_kernel(double *p) { *p = 0.0; }
 
-__global__ __launch_bounds__(256) void rsnet_adam_kernel(float *__restrict__ w, float *__restrict__ m1,
-                                                         float *__restrict__ m2,
-                                                         const float *__restrict__ g,
-                                                         uint16_t *__restrict__ wbf, float lr,
-                                                         float c1, float c2) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= NPARAM) return;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float gp = g[p];
-    const float a = fmaf(b1, m1[p], (1.f - b1) * gp);
-    const float v = fmaf(b2, m2[p], (1.f - b2) * gp * gp);
-    m1[p] = a;
-    m2[p] = v;
-    const float wp = w[p] - lr * (a / c1) / (sqrtf(v / c2) + eps);
-    w[p] = wp;
-    wbf[p] = f32_to_bf16(wp);
-}
-
 __global__ __launch_bounds__(256) void rsnet_round_kernel(const float *__restrict__ w,
                                                           uint16_t *__restrict__ wbf) {
     const int p = blockIdx.x * 256 + threadIdx.x;
@@ -315,7 +383,7 @@ __global__ __launch_bounds__(256) void rsnet_forward_kernel(int n, const float *
                                                             const float *__restrict__ norm,
                                                             float *__restrict__ y) {
     __shared__ SW w;
-    load_weights(w, wbf);
+    load_weights<256>(w, wbf);
     __syncthreads();
     const int s = blockIdx.x * 256 + threadIdx.x;
     if (s >= n) return;
@@ -336,7 +404,7 @@ __global__ __launch_bounds__(256) void rs_predict_kernel(int n, const float *__r
                                                          double *__restrict__ ib, int ib_stride,
                                                          int m_flag, double bodym) {
     __shared__ SW w;
-    load_weights(w, wbf);
+    load_weights<256>(w, wbf);
     __syncthreads();
     const int s = blockIdx.x * 256 + threadIdx.x;
     if (s >= n) return;
@@ -562,7 +630,7 @@ int rsnet_open(unsigned long long seed) {
         s.master.get(NPARAM * sizeof(float));
         s.m1.get(NPARAM * sizeof(float));
         s.m2.get(NPARAM * sizeof(float));
-        s.wbf.get(NPARAM * sizeof(uint16_t));
+        s.wbf.get((NPARAM + 1) * sizeof(uint16_t));
         s.grad.get((NPARAM + 1) * sizeof(float));
         s.loss.get(sizeof(float));
         s.norm.get(2 * NF * sizeof(float));
@@ -641,23 +709,43 @@ int rsnet_forward(int n, const float *d_feat, float *d_y, hipStream_t s) {
     return OK;
 }
 
-// gradient of the mean squared error over n samples into d_grad (NPARAM) and the
-// loss into *d_loss (both device pointers; null: the library's own buffers)
+namespace {
+constexpr int SUM_GRID = (NPARAM + SUMP - 1) / SUMP + 1;   // parameters, and the loss
+
+// gradient of the mean squared error over n samples (rows idx[base ..], see
+// rsnet_grad_kernel) into d_grad (may be null) and the loss into *d_loss; ad.w set: the
+// Adam step with it
+void grad_and_step(int n, const float *feat, const float *tgt, const int *idx, int base,
+                   int fstride, float *d_grad, float *d_loss, double *lacc, const Adam &ad,
+                   hipStream_t s) {
+    NetState &g = g_net;
+    const int nblk = (n + GB - 1) / GB;
+    float *part = static_cast<float *>(g.part.get(((size_t)nblk * NPARAM + nblk) * sizeof(float)));
+    float *lpart = part + (size_t)nblk * NPARAM;
+    hipLaunchKernelGGL(rsnet_grad_kernel, dim3(nblk), dim3(64 * GW), 0, s, n, feat, tgt, idx, base,
+                       fstride, g.wbf.as<uint16_t>(), g.norm.as<float>(), part, lpart);
+    hipLaunchKernelGGL(rsnet_sum_kernel, dim3(SUM_GRID), dim3(256), 0, s, part, nblk, d_grad, lpart,
+                       d_loss, n, lacc, ad);
+    NB6_HIP(hipGetLastError());
+}
+
+// the next Adam step of the network (beta 0.9 / 0.999)
+Adam next_step(float lr) {
+    NetState &g = g_net;
+    g.step++;
+    return Adam{g.master.as<float>(), g.m1.as<float>(), g.m2.as<float>(), g.wbf.as<uint16_t>(), lr,
+                1.f - std::pow(0.9f, (float)g.step), 1.f - std::pow(0.999f, (float)g.step)};
+}
+}  // namespace
+
+// (null d_grad, d_loss: the library's own buffers)
 int rsnet_grad(int n, const float *d_feat, const float *d_t, float *d_grad, float *d_loss,
                hipStream_t s) {
     if (!net_ready()) return E_STATE;
     if (n <= 0) { set_error(E_ARG, "nb6_rsnet_grad: n must be positive"); return E_ARG; }
     NetState &g = g_net;
-    const int nblk = (n + GB - 1) / GB;
-    float *part = static_cast<float *>(g.part.get(((size_t)nblk * NPARAM + nblk) * sizeof(float)));
-    float *lpart = part + (size_t)nblk * NPARAM;
-    hipLaunchKernelGGL(rsnet_grad_kernel, dim3(nblk), dim3(GB), 0, s, n, d_feat, d_t, nullptr, 0,
-                       n, g.wbf.as<uint16_t>(), g.norm.as<float>(), part, lpart);
-    NB6_HIP(hipGetLastError());
-    hipLaunchKernelGGL(rsnet_sum_kernel, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, s, part, nblk,
-                       d_grad ? d_grad : g.grad.as<float>(), lpart, d_loss ? d_loss : g.loss.as<float>(), n,
-                       nullptr);
-    NB6_HIP(hipGetLastError());
+    grad_and_step(n, d_feat, d_t, nullptr, 0, n, d_grad ? d_grad : g.grad.as<float>(),
+                  d_loss ? d_loss : g.loss.as<float>(), nullptr, Adam{}, s);
     return OK;
 }
 
@@ -685,23 +773,10 @@ int rsnet_train_epoch(int n, const float *d_feat, const float *d_t, int batch, f
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, skey, val, perm, n, 0, 32, s));
     double *lacc = static_cast<double *>(g.lacc.get(sizeof(double)));
     hipLaunchKernelGGL(rsnet_zero_kernel, dim3(1), dim3(1), 0, s, lacc);
-    const int nblk = (batch + GB - 1) / GB;
-    float *part = static_cast<float *>(g.part.get(((size_t)nblk * NPARAM + nblk) * sizeof(float)));
-    float *lpart = part + (size_t)nblk * NPARAM;
     const int nb = n / batch;
-    for (int b = 0; b < nb; b++) {
-        hipLaunchKernelGGL(rsnet_grad_kernel, dim3(nblk), dim3(GB), 0, s, batch, d_feat, d_t, perm,
-                           b * batch, n, g.wbf.as<uint16_t>(), g.norm.as<float>(), part, lpart);
-        hipLaunchKernelGGL(rsnet_sum_kernel, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, s, part,
-                           nblk, g.grad.as<float>(), lpart, g.loss.as<float>(), batch, lacc);
-        g.step++;
-        const float c1 = 1.f - std::pow(0.9f, (float)g.step);
-        const float c2 = 1.f - std::pow(0.999f, (float)g.step);
-        hipLaunchKernelGGL(rsnet_adam_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, s,
-                           g.master.as<float>(), g.m1.as<float>(), g.m2.as<float>(),
-                           g.grad.as<float>(), g.wbf.as<uint16_t>(), lr, c1, c2);
-    }
-    NB6_HIP(hipGetLastError());
+    for (int b = 0; b < nb; b++)
+        grad_and_step(batch, d_feat, d_t, perm, b * batch, n, nullptr, g.loss.as<float>(), lacc,
+                      next_step(lr), s);
     if (h_loss) {
         double l = 0.0;
         NB6_HIP(hipMemcpyAsync(&l, lacc, sizeof(double), hipMemcpyDeviceToHost, s));
@@ -713,16 +788,11 @@ int rsnet_train_epoch(int n, const float *d_feat, const float *d_t, int batch, f
 
 int rsnet_train_step(int n, const float *d_feat, const float *d_t, float lr, float *h_loss,
                      hipStream_t s) {
-    int rc = rsnet_grad(n, d_feat, d_t, nullptr, nullptr, s);
-    if (rc != OK) return rc;
+    if (!net_ready()) return E_STATE;
+    if (n <= 0) { set_error(E_ARG, "nb6_rsnet_grad: n must be positive"); return E_ARG; }
     NetState &g = g_net;
-    g.step++;
-    const float c1 = 1.f - std::pow(0.9f, (float)g.step);
-    const float c2 = 1.f - std::pow(0.999f, (float)g.step);
-    hipLaunchKernelGGL(rsnet_adam_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, s,
-                       g.master.as<float>(), g.m1.as<float>(), g.m2.as<float>(), g.grad.as<float>(),
-                       g.wbf.as<uint16_t>(), lr, c1, c2);
-    NB6_HIP(hipGetLastError());
+    grad_and_step(n, d_feat, d_t, nullptr, 0, n, nullptr, g.loss.as<float>(), nullptr,
+                  next_step(lr), s);
     if (h_loss) {
         NB6_HIP(hipMemcpyAsync(h_loss, g.loss.p, sizeof(float), hipMemcpyDeviceToHost, s));
         NB6_HIP(hipStreamSynchronize(s));
