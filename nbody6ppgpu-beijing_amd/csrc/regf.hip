@@ -34,8 +34,8 @@
 //    the reference computes them; if even the soft slots run out the row's
 //    forces are NaN.
 //
-//  * regf_finalize_kernel: one wavefront per i (regf_finalize_wide_kernel: eight for at
-//    most 16384 i in 16 chunks or more, four for 32 chunks or more).  Sums the FP64 chunk partials,
+//  * regf_finalize_kernel: one wavefront per i (regf_finalize_wide_kernel: four for at most
+//    16384 i, eight for at most 2048 in 16 chunks or more).  Sums the FP64 chunk partials,
 //    re-tests every hard candidate in FP64 with the reference formula (no FMA
 //    contraction), adds the FP64 force of every non-neighbour candidate, maps
 //    neighbours back to the caller's indices and writes each row in ascending
@@ -43,6 +43,7 @@
 #include "nb6_internal.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 namespace nb6 {
@@ -58,7 +59,8 @@ constexpr int NPART = 7 + NERR;
 constexpr int CAP_SOFT = 1024;        // soft (near-field) slots per (i, chunk)
 constexpr int BAND_SLOTS = 16;        // of which kept for band pairs of overflowing rows
 constexpr int NB_SORT_MAX = 2048;     // largest neighbour row the finalize sorts
-constexpr int FIN_WIDE_NI = 16384;    // i-set size below which 16 chunks take the wide finalize
+constexpr int FIN_WIDE_NI = 16384;    // largest i-set for four wavefronts per i in the finalize
+constexpr int FIN_WIDEST_NI = 2048;   // and for eight (regf_launch_impl)
 
 // rounding-error margins (u = 2^-24)
 constexpr double U24 = 5.9604644775390625e-08;
@@ -793,21 +795,42 @@ __device__ __forceinline__ bool needs_fp64(const double *s, const double *e, boo
     return !(ea <= q.ta) || !(ej <= q.tj);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Sums over a wavefront, the same in every lane: within rows of 16 lanes by row shifts,
+// then across the rows (DPP moves: no LDS traffic), the total read from lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int v) {   // 0 where the source lane does not exist
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp0(double v) {
+    return __hiloint2double(dpp0<CTRL, ROWS>(__double2hiint(v)), dpp0<CTRL, ROWS>(__double2loint(v)));
+}
+template <class T>
+__device__ __forceinline__ T wave_last(T v) {   // (row_shr 1, 2, 4, 8; row_bcast 15, 31)
+    v += dpp0<0x111, 0xf>(v);
+    v += dpp0<0x112, 0xf>(v);
+    v += dpp0<0x114, 0xf>(v);
+    v += dpp0<0x118, 0xf>(v);
+    v += dpp0<0x142, 0xa>(v);
+    v += dpp0<0x143, 0xc>(v);
     return v;
 }
+__device__ __forceinline__ double wave_sum(double v) {
+    v = wave_last(v);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
 __device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return __builtin_amdgcn_readlane(wave_last(v), 63);
 }
 
 __device__ __forceinline__ int lane_prefix(unsigned long long b) {
     return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32),
                                           __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u));
 }
+
+// room for a row's neighbours in LDS: a longer row overflows and lists none
+__host__ __device__ __forceinline__ int row_cap(int nnbmax) { return (max(nnbmax, 1) + 3) & ~3; }
 
 struct IF64 {
     double x, y, z, u, v, w, h2, dtr;
@@ -915,15 +938,64 @@ __device__ __forceinline__ bool classify(const double *__restrict__ rec, const I
     return pair64<MFLAG>(r0, r1, I, test, s);
 }
 
+// Work memory in LDS of one wavefront of the finalize: the records of 64 candidates
+// (64 bytes each, their 16-byte pieces swizzled) and the candidates' place by chunk.
+struct FinStage {
+    double2 rec[256];
+    int2 pre[64];            // candidates before a chunk's first; its hard ones
+};
+
+// FP64 records of the sorted particles sj (one per lane) into st.rec: four lanes fetch one
+// record's line, so 64 records cost 64 line accesses instead of the 256 that a lane
+// reading its own four pieces would make.  Piece p of record r lies at 4 r + (p ^ (r / 4 mod
+// 4)), which spreads the lanes' reads of one piece over all LDS banks.
+__device__ __forceinline__ void stage_records(const double *__restrict__ rec64, int sj, int lane,
+                                              double2 *rec) {
+    const double2 *src = reinterpret_cast<const double2 *>(rec64);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r = q * 16 + (lane >> 2);
+        const int j = __shfl(sj, r, 64);
+        const int pc = (lane & 3) ^ ((r >> 2) & 3);
+        __builtin_amdgcn_global_load_lds((glb_void *)(src + 4 * (size_t)j + pc),
+                                         (lds_void *)&rec[q * 64], 16, 0, 0);
+    }
+}
+__device__ __forceinline__ void staged_record(const double2 *rec, int r, double4 &r0, double4 &r1) {
+    const int x = (r >> 2) & 3;
+    const double2 a = rec[4 * r + x], b = rec[4 * r + (1 ^ x)];
+    const double2 c = rec[4 * r + (2 ^ x)], d = rec[4 * r + (3 ^ x)];
+    r0 = make_double4(a.x, a.y, b.x, b.y);
+    r1 = make_double4(c.x, c.y, d.x, d.y);
+}
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The FP64 pass over one i's candidates, in the chunks c = c0 + cstep (64 p + lane),
-// p = 0, 1, ...: every hard candidate is re-tested (neighbours into buf), every
+// p = 0, 1, ...: every hard candidate is re-tested (neighbours into buf, at most cap), every
 // non-neighbour candidate's force is added to s.  SHARED: several wavefronts fill one
 // row, taking buffer positions from *nshared; otherwise this wavefront's nnb counts them.
+// The candidates of 64 chunks form one list (per chunk the hard slots, then the soft
+// ones), taken 64 at a time, one per lane: the slot entries of the next 64 are read while
+// the records of the current ones are fetched, and chunks with a few candidates each (or
+// a massive star each, with m_flag) cost no pass of their own.  Bound by FP64 issue
+// (about 55 % of the time) and by the latency of the gathers, which the number of resident
+// wavefronts hides: fetching 64 records ahead in a second LDS set left 16 wavefronts per CU
+// in place of 24 and took 2.41 ms where this takes 1.87 (64 clusters, 381,067 rows; 2.39
+// with a pass per chunk and every lane reading its own record).  N = 65,536, ni = N:
+// 1.28 -> 0.70 ms; N = 100,003, ni = 6007 with m_flag, whose massive stars lie in every
+// chunk: 0.56 -> 0.23 ms; N = 2^20, ni = 2^17: 2.06 -> 1.57 ms.  Listing all hard candidates
+// before all soft ones, so that most passes need no neighbour test, gained 1 % there and
+// lost 3 % on many chunks.
 template <bool MFLAG, bool SHARED>
 __device__ __forceinline__ void fin_candidates(const FinParams &f, const IF64 &I, int i, int jb,
                                                int c0, int cstep, int lane, double *s, int *buf,
-                                               int *nshared, int &nnb, int &dropped, int &unres,
-                                               bool &dropped_any) {
+                                               int cap, FinStage &st, int *nshared, int &nnb,
+                                               int &dropped, int &unres, bool &dropped_any) {
+    enum { HARD, SOFT, BAND, NONE };
     for (int cg = 0; c0 + cstep * cg < f.nchunk; cg += 64) {
         const int c = c0 + cstep * (cg + lane);
         const int nh = c < f.nchunk ? f.cnt[((size_t)c * 2 + 0) * f.ni + i] : 0;
@@ -931,57 +1003,92 @@ __device__ __forceinline__ void fin_candidates(const FinParams &f, const IF64 &I
         const int over = wave_sum_i(nh > f.caph ? nh - f.caph : 0);
         dropped += over;
         dropped_any = dropped_any || over > 0;
-        unsigned long long mask = __ballot(nh > 0 || ns > 0);
-        while (mask) {
-            const int cl = __builtin_ctzll(mask);
-            mask &= mask - 1;
-            const size_t rowc = (size_t)(c0 + cstep * (cg + cl)) * f.ni + i;
-            const int nhc = min(__shfl(nh, cl, 64), f.caph);
-            const int nsc = __shfl(ns, cl, 64);
-            const int *hs = f.hslot + rowc * f.caph;
-            for (int kb = 0; kb < nhc; kb += 64) {
-                const int k = kb + lane;
-                bool isnb = false;
-                int jo = 0;
-                if (k < nhc) {
-                    const int sj = hs[k];
-                    if ((unsigned)sj < (unsigned)f.nj) {
-                        isnb = classify<MFLAG>(f.rec64 + (size_t)sj * 8, I, true, s);
-                        jo = f.perm[sj] - jb;
-                    }
-                }
-                const unsigned long long b = __ballot(isnb);
+        const int nhc = min(nh, f.caph), nsr = min(ns, f.caps);
+        if (__ballot(ns > nsr)) unres += wave_sum_i(ns - nsr);
+        const int end = wave_last(nhc + nsr);   // (an inclusive scan)
+        const int total = __builtin_amdgcn_readlane(end, 63);
+        if (total == 0) continue;
+        wave_lds_sync();                 // the last group's reads of pre are done
+        st.pre[lane] = make_int2(end - nhc - nsr, nhc);
+        wave_lds_sync();
+        // candidate e of the list: its slot entry and kind
+        auto entry = [&](int e, int &kind) {
+            kind = NONE;
+            if (e >= total) return 0;
+            int m = 0;
+            if (f.nchunk > 1) {
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1)
+                    if (st.pre[m + o].x <= e) m += o;
+            }
+            const int2 pr = st.pre[m];
+            const int k = e - pr.x;
+            const size_t rowc = (size_t)(c0 + cstep * (cg + m)) * f.ni + i;
+            kind = k < pr.y ? HARD : SOFT;
+            return k < pr.y ? f.hslot[rowc * f.caph + k] : f.sslot[rowc * f.caps + (k - pr.y)];
+        };
+        int kn, en = entry(lane, kn);
+        for (int e0 = 0; e0 < total; e0 += 64) {
+            int kind = kn;
+            int sj = en;
+            // soft slots hold near-field pairs (force only) and, marked ~j, band pairs
+            // beyond the hard slots of an overflowing row; those were counted in
+            // dropped and are re-counted by the FP64 test here
+            const bool band = kind == SOFT && sj < 0;
+            if (band) {
+                sj = ~sj;
+                kind = BAND;
+            }
+            const bool ok = kind != NONE && (unsigned)sj < (unsigned)f.nj;
+            if (!ok) sj = 0;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last records are read
+            stage_records(f.rec64, sj, lane, st.rec);
+            const int jo = ok && kind == HARD ? f.perm[sj] - jb : 0;
+            kn = NONE;
+            if (e0 + 64 < total) en = entry(e0 + 64 + lane, kn);
+            lds_dma_wait();
+            bool isnb = false;
+            if (ok) {
+                double4 r0, r1;
+                staged_record(st.rec, lane, r0, r1);
+                isnb = pair64<MFLAG>(r0, r1, I, kind != SOFT, s);
+            }
+            const unsigned long long b = __ballot(isnb && kind == HARD);
+            if (b) {
                 int base = nnb;
                 if (SHARED) {
                     int t = 0;
-                    if (lane == 0 && b) t = atomicAdd(nshared, __popcll(b));
+                    if (lane == 0) t = atomicAdd(nshared, __popcll(b));
                     base = __shfl(t, 0, 64);
                 }
                 const int pos = base + lane_prefix(b);
-                if (isnb && pos < NB_SORT_MAX) buf[pos] = jo;
+                if (isnb && kind == HARD && pos < cap) buf[pos] = jo;
                 nnb += __popcll(b);
             }
-            // soft slots: near-field pairs (force only) and, marked ~j, band pairs
-            // beyond the hard slots of an overflowing row; those were counted in
-            // dropped and are re-counted by the FP64 test here
-            const int *ss = f.sslot + rowc * f.caps;
-            const int nsr = min(nsc, f.caps);
-            unres += nsc - nsr;
-            for (int kb = 0; kb < nsr; kb += 64) {
-                const int k = kb + lane;
-                bool band = false, isnb = false;
-                if (k < nsr) {
-                    const int e = ss[k];
-                    band = e < 0;
-                    const int sj = band ? ~e : e;
-                    if ((unsigned)sj < (unsigned)f.nj)
-                        isnb = classify<MFLAG>(f.rec64 + (size_t)sj * 8, I, band, s);
-                }
-                dropped += __popcll(__ballot(isnb)) - __popcll(__ballot(band));
-            }
+            dropped += __popcll(__ballot(isnb && band)) - __popcll(__ballot(band));
         }
     }
+}
 
+// ascending row from the nnb (distinct) indices in buf (16-byte aligned, room up to the
+// next multiple of four), by nt threads t of one wavefront or work-group: the rank of
+// each index among the row, four indices per LDS read
+__device__ __forceinline__ void rank_pad(int *buf, int nnb, int t) {
+    if (t < 3 && nnb + t < ((nnb + 3) & ~3)) buf[nnb + t] = INT_MAX;
+}
+__device__ __forceinline__ void rank_row(const int *buf, int nnb, int t, int nt, int *row) {
+    const int4 *b4 = reinterpret_cast<const int4 *>(buf);
+    const int n4 = (nnb + 3) >> 2;
+    for (int k = t; k < nnb; k += nt) {
+        const int e = buf[k];
+        int rank = 0;
+#pragma unroll 4
+        for (int m = 0; m < n4; m++) {
+            const int4 v = b4[m];
+            rank += (v.x < e) + (v.y < e) + (v.z < e) + (v.w < e);
+        }
+        row[1 + rank] = e;
+    }
 }
 
 // A flagged row whose sums are finite: the chunks to recompute in FP64, chosen so that
@@ -992,6 +1099,7 @@ __device__ __forceinline__ void fin_candidates(const FinParams &f, const IF64 &I
 // contiguous and in chunk order; a row whose items do not fit the item buffer takes the
 // whole-row pass instead.
 constexpr int SHARE_LDS = 2048;   // segments whose shares the wide finalize keeps in LDS
+static_assert(SHARE_LDS * sizeof(float2) <= 4 * sizeof(FinStage), "shares take the place of the stages");
 
 __device__ void emit_chunks(const FinParams &f, int i, int r, const double *s, int lane,
                             float2 *lds_share = nullptr) {
@@ -1142,16 +1250,19 @@ __device__ void emit_chunks(const FinParams &f, int i, int r, const double *s, i
     if (lane == 0) f.rowsel[atomicAdd(f.nrows, 1)] = make_int4(r, start, cnt, 0);
 }
 
+// (six wavefronts per SIMD: 80 VGPRs, a few spilled in the choice of FP64-pass segments)
 template <bool MFLAG>
-__global__ __launch_bounds__(256) void regf_finalize_kernel(FinParams f) {
-    __shared__ int nbuf[4][NB_SORT_MAX];
+__global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
+    extern __shared__ __align__(16) int nbuf[];   // [4][row_cap]
+    __shared__ FinStage stage[4];
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
-    const int i = blockIdx.x * 4 + wid;   // slot
+    const int i = xcd_order(blockIdx.x, gridDim.x) * 4 + wid;   // slot
     if (i >= f.ni) return;   // whole wavefront leaves together
     const int r = f.imap ? f.imap[i] : i;   // caller row
     if (r < 0) return;
-    int *buf = nbuf[wid];
+    const int cap = row_cap(f.nnbmax);
+    int *buf = nbuf + wid * cap;
 
     // 1. FP64 sum of the chunk partials (and of the error scales)
     double s[7], e[NERR] = {0.0, 0.0, 0.0, 0.0};
@@ -1179,8 +1290,8 @@ __global__ __launch_bounds__(256) void regf_finalize_kernel(FinParams f) {
     int dropped = 0;      // hard candidates beyond the slot capacity
     int unres = 0;        // band pairs of an overflowing row left without a slot
     bool dropped_any = false;
-    fin_candidates<MFLAG, false>(f, I, i, jb, 0, 1, lane, s, buf, nullptr, nnb, dropped, unres,
-                                 dropped_any);
+    fin_candidates<MFLAG, false>(f, I, i, jb, 0, 1, lane, s, buf, cap, stage[wid], nullptr, nnb,
+                                 dropped, unres, dropped_any);
 
 #pragma unroll
     for (int q = 0; q < 7; q++) s[q] = wave_sum(s[q]);
@@ -1225,36 +1336,31 @@ __global__ __launch_bounds__(256) void regf_finalize_kernel(FinParams f) {
         }
     }
     if (!ovf && nnb > 0) {
-        // ascending row: the rank of each (distinct) index among the row
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (int k = lane; k < nnb; k += 64) {
-            const int e = buf[k];
-            int rank = 0;
-            for (int m = 0; m < nnb; m++) rank += buf[m] < e;
-            row[1 + rank] = e;
-        }
+        rank_pad(buf, nnb, lane);
+        wave_lds_sync();
+        rank_row(buf, nnb, lane, 64, row);
     }
 }
 
 // One work-group of W wavefronts per i, for small i-sets, where one wavefront per i
 // leaves most of the GPU idle while it waits on its gathers: wavefront w takes the
 // chunks c = w (mod W), so the few chunks that hold an i's candidates (they lie close
-// together in the Morton order) are spread over the W.  Forces are combined in a fixed
+// together in the Morton order) are spread over the W.  The rows of neighbouring i go to
+// one XCD (xcd_order; also in regf_finalize_kernel), whose L2 then serves the records and
+// the partial sums' lines they share.  Forces are combined in a fixed
 // order; the row is rank-sorted as in regf_finalize_kernel.
 template <bool MFLAG, int W>
 __global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f) {
-    __shared__ int buf[NB_SORT_MAX];
+    extern __shared__ __align__(16) int buf[];   // [row_cap]
+    __shared__ FinStage stage[W];
     __shared__ double red[W][NPART];
     __shared__ int cnts[W][3];
     __shared__ int nshared;
     __shared__ int flag;             // 1: chunk items, 2: whole-row pass
     __shared__ double vtot[NPART];
-    __shared__ float2 shr[SHARE_LDS];
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
-    const int i = blockIdx.x;   // slot
+    const int i = xcd_order(blockIdx.x, gridDim.x);   // slot
     const int r = f.imap ? f.imap[i] : i;
     if (r < 0) return;   // the whole work-group leaves together
     if (threadIdx.x == 0) {
@@ -1283,8 +1389,8 @@ __global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f)
     const int jb = f.jbase ? f.jbase[r] : 0;
     int nnb = 0, dropped = 0, unres = 0;
     bool dropped_any = false;
-    fin_candidates<MFLAG, true>(f, I, i, jb, w, W, lane, s, buf, &nshared, nnb, dropped, unres,
-                                dropped_any);
+    fin_candidates<MFLAG, true>(f, I, i, jb, w, W, lane, s, buf, row_cap(f.nnbmax), stage[w],
+                                &nshared, nnb, dropped, unres, dropped_any);
 #pragma unroll
     for (int q = 0; q < NPART; q++) s[q] = wave_sum(s[q]);
     if (lane == 0) {
@@ -1308,6 +1414,7 @@ __global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f)
     // band pairs left without a slot make the row's forces NaN
     const bool ovf = tot > f.nnbmax || dany;
     int *row = f.list + (size_t)r * f.lmax;
+    if (!ovf) rank_pad(buf, nall, threadIdx.x);
     if (threadIdx.x == 0) {
         double *o = f.out + r;
         const int os = f.out_stride;
@@ -1335,15 +1442,10 @@ __global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f)
         double se[NPART];
 #pragma unroll
         for (int q = 0; q < NPART; q++) se[q] = vtot[q];
-        emit_chunks(f, i, r, se, lane, shr);
+        emit_chunks(f, i, r, se, lane, reinterpret_cast<float2 *>(stage));
     }
     if (!ovf && nall > 0) {
-        for (int k = threadIdx.x; k < nall; k += 64 * W) {
-            const int e = buf[k];
-            int rank = 0;
-            for (int m = 0; m < nall; m++) rank += buf[m] < e;
-            row[1 + rank] = e;
-        }
+        rank_row(buf, nall, threadIdx.x, 64 * W, row);
     }
 }
 
@@ -1958,7 +2060,14 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     const int caps = std::min(CAP_SOFT, clen);
     // the finalize form depends on the whole call, never on the batching below, so a
     // batched call gives the same bits as an unbatched one
-    const int fin_form = (ni <= FIN_WIDE_NI && nchunk >= 16) ? 8 : (nchunk >= 32 ? 4 : 1);
+    // one wavefront per i where there are enough i to fill the GPU (N = 65,536: 703 us with
+    // one and 1034 us with four at ni = 65,536, 448 and 601 at 40,000; N = 100,003,
+    // ni = 20,011: 247 and 292); below that each i's chunks are dealt to four wavefronts
+    // (N = 65,536: 225 us against 257 at ni = 16,000, 117 against 225 at 6,000), and to
+    // eight in the smallest calls, where even those leave wavefront slots free (53 us
+    // against 59 with four at ni = 1024, 105 against 93 at 3,000)
+    const int fin_form = ni > FIN_WIDE_NI || nchunk < 2 ? 1
+                                                        : (ni <= FIN_WIDEST_NI && nchunk >= 16 ? 8 : 4);
 
     // Work arrays hold one row per (i, chunk): FP64 partials, counts and the hard and
     // soft candidate slots.  Calls whose rows would exceed the slot budget run in
@@ -2146,24 +2255,23 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         if (refine && b0 > 0)   // item counters per batch (the rows' total is kept in [3])
             hipLaunchKernelGGL(next_batch_kernel, dim3(1), dim3(256), 0, s, ctr, nseg);
         if (timed && b0 == 0) t2.start(s);
+        const size_t rl = (size_t)row_cap(nnbeff) * sizeof(int);   // one row in LDS
         if (fin_form == 8) {
-            // few i: eight wavefronts per i
             if (m_flag)
-                hipLaunchKernelGGL((regf_finalize_wide_kernel<true, 8>), dim3(nb), dim3(512), 0, s, fp);
+                hipLaunchKernelGGL((regf_finalize_wide_kernel<true, 8>), dim3(nb), dim3(512), rl, s, fp);
             else
-                hipLaunchKernelGGL((regf_finalize_wide_kernel<false, 8>), dim3(nb), dim3(512), 0, s, fp);
+                hipLaunchKernelGGL((regf_finalize_wide_kernel<false, 8>), dim3(nb), dim3(512), rl, s, fp);
         } else if (fin_form == 4) {
-            // many chunks per i: four wavefronts per i
             if (m_flag)
-                hipLaunchKernelGGL((regf_finalize_wide_kernel<true, 4>), dim3(nb), dim3(256), 0, s, fp);
+                hipLaunchKernelGGL((regf_finalize_wide_kernel<true, 4>), dim3(nb), dim3(256), rl, s, fp);
             else
-                hipLaunchKernelGGL((regf_finalize_wide_kernel<false, 4>), dim3(nb), dim3(256), 0, s, fp);
+                hipLaunchKernelGGL((regf_finalize_wide_kernel<false, 4>), dim3(nb), dim3(256), rl, s, fp);
         } else {
             const dim3 fgrid((nb + 3) / 4);
             if (m_flag)
-                hipLaunchKernelGGL(regf_finalize_kernel<true>, fgrid, dim3(256), 0, s, fp);
+                hipLaunchKernelGGL(regf_finalize_kernel<true>, fgrid, dim3(256), 4 * rl, s, fp);
             else
-                hipLaunchKernelGGL(regf_finalize_kernel<false>, fgrid, dim3(256), 0, s, fp);
+                hipLaunchKernelGGL(regf_finalize_kernel<false>, fgrid, dim3(256), 4 * rl, s, fp);
         }
         NB6_HIP(hipGetLastError());
         if (timed && b0 + nb >= ni) t2.stop(s);
@@ -2387,10 +2495,11 @@ int regf_items_launch(const JSet &js, int nslots, const int *imap, int stride, c
     for (int q = 0; q < NERR; q++) fp.kf[q] = cfg.kref_ens[q];
     fp.fix_rows = fix_slots; fp.nfix = nfix;
     const dim3 fgrid((nslots + 3) / 4);
+    const size_t rl = (size_t)row_cap(nnbeff) * sizeof(int);   // one row in LDS
     if (m_flag)
-        hipLaunchKernelGGL(regf_finalize_kernel<true>, fgrid, dim3(256), 0, s, fp);
+        hipLaunchKernelGGL(regf_finalize_kernel<true>, fgrid, dim3(256), 4 * rl, s, fp);
     else
-        hipLaunchKernelGGL(regf_finalize_kernel<false>, fgrid, dim3(256), 0, s, fp);
+        hipLaunchKernelGGL(regf_finalize_kernel<false>, fgrid, dim3(256), 4 * rl, s, fp);
     NB6_HIP(hipGetLastError());
     if (refine) {
         // FP64 pass of the flagged rows: items bucketed by cluster, each cluster's records
