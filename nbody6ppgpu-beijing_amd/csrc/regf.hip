@@ -244,6 +244,49 @@ __device__ __forceinline__ PairBase pair_base(const IC &c, const float4 &a, cons
     return q;
 }
 
+// min(r2, |dx + dtr dv|^2) less its rounding band, for the neighbour test
+__device__ __forceinline__ float pair_min(const IC &ck, const PairBase &q) {
+    // keep the full test inside the rare branch: the empty asm makes dtr opaque here, so
+    // the compiler cannot hoist it
+    float dtl = ck.dt1;
+    asm volatile("" : "+v"(dtl));
+    const float ex = fmaf(dtl, q.du, q.dx);
+    const float ey = fmaf(dtl, q.dv, q.dy);
+    const float ez = fmaf(dtl, q.dw, q.dz);
+    const float r2p = fmaf(ez, ez, fmaf(ey, ey, ex * ex));
+    return fminf(q.r2, fmaf(-KAPPA_P, q.r2, r2p));
+}
+
+// v_rsq_f32 plus one Newton-Raphson step
+__device__ __forceinline__ float rinv_nr(float r2) {
+    const float rinv = __builtin_amdgcn_rsqf(r2);
+    const float h = rinv * rinv;
+    const float e = fmaf(-r2, h, 1.0f);
+    return fmaf(rinv, 0.5f * e, rinv);
+}
+
+// acc, pot and jerk terms of one pair (none with rinv = 0).  The jerk term
+// m/r^3 (dv - 3 (dx.dv / r^2) dx) is summed whole: its two parts partly cancel within a
+// pair, so the FP32 partial sum stays smaller than the sums of m dv / r^3 and of
+// 3 m (dx.dv) dx / r^5 would be apart.
+__device__ __forceinline__ void pair_add(const PairBase &q, float rinv, float m,
+                                         float *__restrict__ acc, float &s3) {
+    const float rinv2 = rinv * rinv;
+    const float mr1 = m * rinv;
+    const float mr3 = mr1 * rinv2;
+    const float al = q.rv * (-3.0f * rinv2);
+    acc[0] = fmaf(mr3, q.dx, acc[0]);
+    acc[1] = fmaf(mr3, q.dy, acc[1]);
+    acc[2] = fmaf(mr3, q.dz, acc[2]);
+    acc[3] += mr1;
+    acc[4] = fmaf(mr3, fmaf(al, q.dx, q.du), acc[4]);
+    acc[5] = fmaf(mr3, fmaf(al, q.dy, q.dv), acc[5]);
+    acc[6] = fmaf(mr3, fmaf(al, q.dz, q.dw), acc[6]);
+    // sum of m/r^3: times the tile's bounds of the FP32 rounding of positions
+    // and velocities it bounds the rounding error of the pair terms
+    s3 += mr3;
+}
+
 // One j against the IPL i-particles of this lane.  TEST=false leaves out the
 // candidate test: only used where lane_far holds for every lane of the wavefront,
 // where the test could not have recorded anything, so both forms give the same sums.
@@ -254,28 +297,14 @@ __device__ __forceinline__ void pair_step(const TileParams &p, const IC &ck, con
                                           float *__restrict__ acc, float &s3) {
     {
         const PairBase q = pair_base(ck, a, b);
-        // v_rsq_f32 plus one Newton-Raphson step
-        float rinv = __builtin_amdgcn_rsqf(q.r2);
-        {
-            const float h = rinv * rinv;
-            const float e = fmaf(-q.r2, h, 1.0f);
-            rinv = fmaf(rinv, 0.5f * e, rinv);
-        }
+        float rinv = rinv_nr(q.r2);
         if (TEST) {
             // cheap conservative bound on the soft test:
             // r2p >= r2 + 2 dtr min(rv, 0)  (dt2 carries the 1/(1-kappa) slack)
             const float t1 = fmaf(ck.dt2, fminf(q.rv, 0.f), q.r2);
             const float thq = MFLAG ? fmaf(a.w, ck.hQ, ck.dQ) : ck.hQ;
             if (t1 < thq) {
-                // keep the full test inside the rare branch: the empty asm
-                // makes dtr opaque here, so the compiler cannot hoist it
-                float dtl = ck.dt1;
-                asm volatile("" : "+v"(dtl));
-                const float ex = fmaf(dtl, q.du, q.dx);
-                const float ey = fmaf(dtl, q.dv, q.dy);
-                const float ez = fmaf(dtl, q.dw, q.dz);
-                const float r2p = fmaf(ez, ez, fmaf(ey, ey, ex * ex));
-                const float mn = fminf(q.r2, fmaf(-KAPPA_P, q.r2, r2p));
+                const float mn = pair_min(ck, q);
                 const float thh = MFLAG ? fmaf(a.w, ck.hH, ck.dH) : ck.hH;
                 const float ths = MFLAG ? fmaf(a.w, ck.hS, ck.dS) : ck.hS;
                 if (mn < thh && jg < j1) {
@@ -302,23 +331,7 @@ __device__ __forceinline__ void pair_step(const TileParams &p, const IC &ck, con
                 }
             }
         }
-        // jerk term m/r^3 (dv - 3 (dx.dv / r^2) dx) summed whole: its two parts partly
-        // cancel within a pair, so the FP32 partial sum stays smaller than the sums of
-        // m dv / r^3 and of 3 m (dx.dv) dx / r^5 would be apart
-        const float rinv2 = rinv * rinv;
-        const float mr1 = a.w * rinv;
-        const float mr3 = mr1 * rinv2;
-        const float al = q.rv * (-3.0f * rinv2);
-        acc[0] = fmaf(mr3, q.dx, acc[0]);
-        acc[1] = fmaf(mr3, q.dy, acc[1]);
-        acc[2] = fmaf(mr3, q.dz, acc[2]);
-        acc[3] += mr1;
-        acc[4] = fmaf(mr3, fmaf(al, q.dx, q.du), acc[4]);
-        acc[5] = fmaf(mr3, fmaf(al, q.dy, q.dv), acc[5]);
-        acc[6] = fmaf(mr3, fmaf(al, q.dz, q.dw), acc[6]);
-        // sum of m/r^3: times the tile's bounds of the FP32 rounding of positions
-        // and velocities it bounds the rounding error of the pair terms
-        s3 += mr3;
+        pair_add(q, rinv, a.w, acc, s3);
     }
 }
 
@@ -1526,14 +1539,6 @@ __global__ __launch_bounds__(256) void regf_fix_kernel(FixParams f) {
     fix_body<MFLAG>(f, blockIdx.x, gridDim.x, sA, sB);
 }
 
-// element q of v[7] without indexing by a lane-varying value
-__device__ __forceinline__ double pick7(const double *v, int q) {
-    double r = v[0];
-#pragma unroll
-    for (int k = 1; k < 7; k++) r = q == k ? v[k] : r;
-    return r;
-}
-
 // one wavefront per whole row: lane l sums chunks l, l + 64, ... in order, then a
 // fixed tree over the lanes
 __device__ __forceinline__ void fix_reduce_body(const FixParams &f, int bid) {
@@ -1551,7 +1556,10 @@ __device__ __forceinline__ void fix_reduce_body(const FixParams &f, int bid) {
 #pragma unroll
     for (int q = 0; q < 7; q++) sum[q] = wave_sum(sum[q]);
     const int r = f.rows[k];
-    if (lane < 7) f.out[(size_t)lane * f.out_stride + r] = pick7(sum, lane);
+    if (lane == 0) {
+#pragma unroll
+        for (int q = 0; q < 7; q++) f.out[(size_t)q * f.out_stride + r] = sum[q];
+    }
 }
 
 __global__ __launch_bounds__(256) void regf_fix_reduce_kernel(FixParams f) {
@@ -1615,32 +1623,63 @@ __device__ __forceinline__ IF64 load_if64(const double *__restrict__ ib, int is,
     return I;
 }
 
-// one wavefront per item of the row entries (rows whose items were all stored)
+// Prefix sums over the buckets in LDS (spre[nchunk + 1], wtot[4]): spre[c] = sum over the
+// buckets before c of their items in groups of `grp`.  All 256 threads; nchunk <= SEGCNT_LDS.
+__device__ __forceinline__ void bucket_prefix(const ChunkFixParams &f, int grp, int *spre,
+                                              int *wtot) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int per = (f.nchunk + 255) / 256;
+    int n = 0;
+    for (int q = 0; q < per; q++) {
+        const int c = t * per + q;
+        n += c < f.nchunk ? (f.seg_cnt[c] + grp - 1) / grp : 0;
+    }
+    const int incl = wave_last(n);
+    if (lane == 63) wtot[w] = incl;
+    __syncthreads();
+    int base = incl - n;
+    for (int q = 0; q < w; q++) base += wtot[q];
+    for (int q = 0; q < per; q++) {
+        const int c = t * per + q;
+        if (c >= f.nchunk) break;
+        spre[c] = base;
+        base += (f.seg_cnt[c] + grp - 1) / grp;
+    }
+    if (t == 0) spre[f.nchunk] = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+    __syncthreads();
+}
+// the last bucket c with spre[c] <= g
+__device__ __forceinline__ int find_bucket(const int *spre, int n, int g) {
+    int c = 0, hi = n;
+    while (hi - c > 1) {
+        const int mid = (c + hi) >> 1;
+        if (spre[mid] <= g) c = mid; else hi = mid;
+    }
+    return c;
+}
+// bucket c's item list: one of ni entries, or (batched form: (cluster, segment) c) of its
+// cluster's slots
+__device__ __forceinline__ const int *bucket_of(const ChunkFixParams &f, int c) {
+    if (!f.padoff) return f.seg_items + (size_t)c * f.ni;
+    const int cl = c / f.nseg_c, sg = c - cl * f.nseg_c;
+    const int p0 = f.padoff[cl];
+    return f.seg_items + (size_t)p0 * f.nseg_c + (size_t)sg * (f.padoff[cl + 1] - p0);
+}
+
+// one wavefront per item, the items of all buckets dealt evenly (spre: LDS[SEGCNT_LDS + 1],
+// wtot: LDS[4]); more buckets than that: every bucket in turn
 template <bool MFLAG>
-__device__ __forceinline__ void cand_body(const ChunkFixParams &f, int bid, int nblk) {
+__device__ __forceinline__ void cand_body(const ChunkFixParams &f, int bid, int nblk, int *spre,
+                                          int *wtot) {
     const int lane = threadIdx.x & 63;
-    const int nr = *f.nrows;
-    const int ri = max(f.row_items, 1);
-    // (entry, item) pairs in contiguous runs per wavefront, a row's items one after
-    // another; past a row's last item the run goes on at the next row
-    const long long nw = (long long)nr * ri;
-    const long long nwave = (long long)nblk * 4;
-    const long long per = (nw + nwave - 1) / nwave;
-    const long long w0 = (long long)(bid * 4 + (threadIdx.x >> 6)) * per;
-    const long long w1 = min(nw, w0 + per);
-    int ecur = -1;
-    int4 rs = make_int4(0, 0, 0, 0);
-    for (long long w = w0; w < w1; w++) {
-        const int e = (int)(w / ri), m = (int)(w - (long long)e * ri);
-        if (e != ecur) {
-            rs = f.rowsel[e];
-            ecur = e;
-        }
-        if (m >= rs.z) {
-            w = (long long)(e + 1) * ri - 1;   // the next row
-            continue;
-        }
-        const int k = rs.y + m;
+    const int w0 = __builtin_amdgcn_readfirstlane(bid * 4 + (threadIdx.x >> 6)), nw = nblk * 4;
+    const bool cached = f.nchunk <= SEGCNT_LDS;
+    if (cached) bucket_prefix(f, 1, spre, wtot);
+    for (int cb = 0; cb < (cached ? 1 : f.nchunk); cb++) {
+    const int total = cached ? spre[f.nchunk] : f.seg_cnt[cb];
+    for (int w = w0; w < total; w += nw) {
+        const int cw = cached ? find_bucket(spre, f.nchunk, w) : cb;
+        const int k = bucket_of(f, cw)[cached ? w - spre[cw] : w];
         const int2 it = f.items[k];
         const int i = it.x, c = f.padoff ? 0 : it.y / f.nseg_c;   // work-array chunk
         // the segment's j range (the batched form: segment it.y % nseg_c of cluster
@@ -1671,95 +1710,111 @@ __device__ __forceinline__ void cand_body(const ChunkFixParams &f, int bid, int 
         }
 #pragma unroll
         for (int q = 0; q < 7; q++) cd[q] = wave_sum(cd[q]);
-        if (lane < 7) f.cand[(size_t)k * 7 + lane] = pick7(cd, lane);
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < 7; q++) f.cand[(size_t)k * 7 + q] = cd[q];
+        }
+    }
     }
 }
 
 template <bool MFLAG>
 __global__ __launch_bounds__(256) void regf_cand_kernel(ChunkFixParams f) {
-    cand_body<MFLAG>(f, blockIdx.x, gridDim.x);
+    __shared__ int spre[SEGCNT_LDS + 1], wtot[4];
+    cand_body<MFLAG>(f, blockIdx.x, gridDim.x, spre, wtot);
 }
 
+// Work units (bucket c, up to 64 of its items, sub-range): lane = item, and each of the four
+// wavefronts takes a quarter of the sub-range, 64 records at a time through LDS of its own;
+// the four sums are added in j order.  Bound by FP64 issue
+// (60 instructions per pair; 2.36 ms for 1.14e9 pairs at N = 2^20, 82 % of the issue limit).
+// With 256 items per work-group, a thread each, the last group of a bucket was mostly empty
+// and few units spread over the GPU: 4.22 ms there, 490 us against 148 for the 28,916 items
+// of 2048 j at N = ni = 65,536.
 template <bool MFLAG>
 __device__ __forceinline__ void segfix_body(const ChunkFixParams &f, int bid, int nblk,
-                                            double4 *sA, double4 *sB, int *scnt) {
-    const int t = threadIdx.x;
-    int gmax = ((f.padoff ? f.maxseg : f.ni) + 255) / 256;
-    // bucket sizes into LDS (scnt[SEGCNT_LDS]: their maximum): the unit loop then reads
-    // them there and ends after the last group that any bucket fills
+                                            double2 (*st)[256], int *spre, int *wtot) {
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const bool cached = f.nchunk <= SEGCNT_LDS;
-    if (cached) {
-        if (t == 0) scnt[SEGCNT_LDS] = 0;
-        __syncthreads();
-        int mx = 0;
-        for (int c = t; c < f.nchunk; c += 256) {
-            const int v = f.seg_cnt[c];
-            scnt[c] = v;
-            mx = max(mx, v);
-        }
-        atomicMax(&scnt[SEGCNT_LDS], mx);
-        __syncthreads();
-        gmax = min(gmax, (scnt[SEGCNT_LDS] + 255) / 256);
-    }
-    const long long units = (long long)f.nchunk * gmax * f.nsub;
-    // units ordered (item group, chunk, sub-range): the few busy groups of every chunk
-    // come first and spread over the whole grid
-    const int per_g = f.nchunk * f.nsub;
-    for (long long u = bid; u < units; u += nblk) {   // uniform per work-group
-        const int g = (int)(u / per_g);
-        const int rem = (int)(u - (long long)g * per_g);
-        const int c = rem / f.nsub, sub = rem - c * f.nsub;
-        const int nc = cached ? scnt[c] : f.seg_cnt[c];
-        if (g * 256 >= nc) continue;
+    if (cached) bucket_prefix(f, 64, spre, wtot);
+    // (more buckets than LDS has room for: every group that a bucket could have in turn)
+    const int gmax = ((f.padoff ? f.maxseg : f.ni) + 63) / 64;
+    const long long groups = cached ? spre[f.nchunk] : (long long)f.nchunk * gmax;
+    for (long long u = bid; u < groups * f.nsub; u += nblk) {   // uniform per work-group
+        const long long gi = u / f.nsub;
+        const int sub = (int)(u - gi * f.nsub);
+        const int c = cached ? find_bucket(spre, f.nchunk, (int)gi) : (int)(gi / gmax);
+        const int i0 = 64 * (cached ? (int)gi - spre[c] : (int)(gi - (long long)c * gmax));
+        const int nc = f.seg_cnt[c];
+        if (i0 >= nc) continue;
         // (the last chunk or a short cluster: trailing sub-ranges are empty and write 0)
         int sb, se;
-        size_t bucket;
         if (f.padoff) {
             // segment sg of cluster cl
             const int cl = c / f.nseg_c, sg = c - cl * f.nseg_c;
-            const int p0 = f.padoff[cl], p1 = f.padoff[cl + 1];
-            sb = p0 + sg * f.clen;
-            se = min(p1, sb + f.clen);
-            bucket = (size_t)p0 * f.nseg_c + (size_t)sg * (p1 - p0);
+            sb = f.padoff[cl] + sg * f.clen;
+            se = min(f.padoff[cl + 1], sb + f.clen);
         } else {
             sb = c * f.clen;
-            se = min(f.nj, (c + 1) * f.clen);
-            bucket = (size_t)c * f.ni;
+            se = min(f.nj, sb + f.clen);
         }
-        const int j0 = sb + sub * FIX_SUB;
-        const int j1 = min(se, j0 + FIX_SUB);
-        const bool ok = g * 256 + t < nc;
-        const int k = ok ? f.seg_items[bucket + g * 256 + t] : 0;
-        IF64 I;
-        if (ok) {
-            const int i = f.items[k].x;
-            I = load_if64(f.ib, f.ib_stride, f.imap ? f.imap[i] : i);
-        }
+        const int j0 = sb + sub * FIX_SUB, j1 = min(se, j0 + FIX_SUB);
+        const int qt = ((max(j1 - j0, 0) + 3) / 4 + 15) & ~15;
+        const int jb = min(j1, j0 + (w + 1) * qt);
+        const int *bucket = bucket_of(f, c);
+        const bool ok = i0 + lane < nc;
+        const int k = bucket[i0 + (ok ? lane : 0)];
+        const int i = f.items[k].x;
+        const IF64 I = load_if64(f.ib, f.ib_stride, f.imap ? f.imap[i] : i);
         double sum[7] = {0, 0, 0, 0, 0, 0, 0};
-        for (int jt = j0; jt < j1; jt += JTILE) {
-            __syncthreads();
-            const int j = jt + t;
-            if (j < j1) {
-                sA[t] = reinterpret_cast<const double4 *>(f.rec64)[2 * (size_t)j];
-                sB[t] = reinterpret_cast<const double4 *>(f.rec64)[2 * (size_t)j + 1];
+        for (int jp = j0 + w * qt; jp < jb; jp += 64) {
+            const int n = min(64, jb - jp);
+            const double2 *src = reinterpret_cast<const double2 *>(f.rec64) + 4 * (size_t)jp;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last records are read
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                __builtin_amdgcn_global_load_lds(
+                    (glb_void *)(src + min(q * 64 + lane, 4 * n - 1)), (lds_void *)&st[w][q * 64], 16,
+                    0, 0);
+            lds_dma_wait();
+            int jj = 0;
+            for (; jj + 4 <= n; jj += 4) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const double4 *r = reinterpret_cast<const double4 *>(&st[w][4 * (jj + v)]);
+                    pair64_sum<MFLAG>(r[0], r[1], I, sum);
+                }
             }
-            __syncthreads();
-            const int jn = min(JTILE, j1 - jt);
-            if (ok) tile_sum64<MFLAG>(sA, sB, jn, I, sum);
+            for (; jj < n; jj++) {
+                const double4 *r = reinterpret_cast<const double4 *>(&st[w][4 * jj]);
+                pair64_sum<MFLAG>(r[0], r[1], I, sum);
+            }
         }
-        if (ok) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        double *mine = reinterpret_cast<double *>(st[w]);
+#pragma unroll
+        for (int q = 0; q < 7; q++) mine[q * 64 + lane] = sum[q];
+        __syncthreads();
+        if (w == 0 && ok) {
             double *o = f.part64 + ((size_t)k * f.nsub + sub) * 7;
 #pragma unroll
-            for (int q = 0; q < 7; q++) o[q] = sum[q];
+            for (int q = 0; q < 7; q++) {
+                double v = sum[q];
+#pragma unroll
+                for (int x = 1; x < 4; x++) v += reinterpret_cast<const double *>(st[x])[q * 64 + lane];
+                o[q] = v;
+            }
         }
+        __syncthreads();
     }
 }
 
 template <bool MFLAG>
 __global__ __launch_bounds__(256) void regf_segfix_kernel(ChunkFixParams f) {
-    __shared__ double4 sA[JTILE], sB[JTILE];
-    __shared__ int scnt[SEGCNT_LDS + 1];
-    segfix_body<MFLAG>(f, blockIdx.x, gridDim.x, sA, sB, scnt);
+    __shared__ double2 st[4][256];
+    __shared__ int spre[SEGCNT_LDS + 1], wtot[4];
+    segfix_body<MFLAG>(f, blockIdx.x, gridDim.x, st, spre, wtot);
 }
 
 // each flagged row, one wavefront: lane l sums the corrections of items l, l + 64, ...
@@ -1786,12 +1841,68 @@ __device__ __forceinline__ void segapply_body(const ChunkFixParams &f, int bid, 
         }
 #pragma unroll
         for (int q = 0; q < 7; q++) d[q] = wave_sum(d[q]);
-        if (lane < 7) f.out[(size_t)lane * f.out_stride + e.x] += pick7(d, lane);
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < 7; q++) f.out[(size_t)q * f.out_stride + e.x] += d[q];
+        }
     }
 }
 
 __global__ __launch_bounds__(256) void regf_segapply_kernel(ChunkFixParams f) {
     segapply_body(f, blockIdx.x, gridDim.x);
+}
+
+// segfix_body for small calls, whose buckets hold few items: a thread per item would walk a
+// whole sub-range alone.  Work units (segment, up to four of its items, sub-range): each
+// row of 16 lanes of every wavefront takes one item, a lane every 16th j of its
+// wavefront's quarter of the sub-range; sums by lanes, then by wavefronts, in a fixed order.
+// Bound by latency.  regf_pass1_kernel with it and with the candidates' items dealt evenly
+// (cand_body): N = 1024, ni = 40 47 -> 6 us; N = 65,536, ni = 1024 53 -> 14 us; N = 100,003,
+// ni = 6007 125 -> 43 us.
+template <bool MFLAG>
+__device__ __forceinline__ void segfix_small_body(const ChunkFixParams &f, int bid, int nblk,
+                                                  double (*red)[4][7], int *wtot, int *spre) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    bucket_prefix(f, 4, spre, wtot);
+    const long long units = (long long)spre[f.nchunk] * f.nsub;
+    for (long long u = bid; u < units; u += nblk) {   // uniform per work-group
+        const int gi = (int)(u / f.nsub), sub = (int)(u - (long long)gi * f.nsub);
+        const int c = find_bucket(spre, f.nchunk, gi);
+        const int i0 = (gi - spre[c]) * 4, nc = f.seg_cnt[c];
+        const int *bucket = f.seg_items + (size_t)c * f.ni;
+        const int im = i0 + (lane >> 4);
+        const bool ok = im < nc;
+        const int i = f.items[bucket[ok ? im : i0]].x;
+        const IF64 I = load_if64(f.ib, f.ib_stride, f.imap ? f.imap[i] : i);
+        const int sb = c * f.clen + sub * FIX_SUB;
+        const int se = min(min(f.nj, (c + 1) * f.clen), sb + FIX_SUB);
+        const int qt = ((se - sb + 3) / 4 + 15) & ~15;
+        const int je = min(se, sb + (w + 1) * qt);
+        double sum[7] = {0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+        for (int j = sb + w * qt + (lane & 15); j < je; j += 16) {
+            const double4 r0 = reinterpret_cast<const double4 *>(f.rec64)[2 * (size_t)j];
+            const double4 r1 = reinterpret_cast<const double4 *>(f.rec64)[2 * (size_t)j + 1];
+            pair64_sum<MFLAG>(r0, r1, I, sum);
+        }
+#pragma unroll
+        for (int q = 0; q < 7; q++) {                 // (row_shr 1, 2, 4, 8: lane 15 of a row)
+            double v = sum[q];
+            v += dpp0<0x111, 0xf>(v);
+            v += dpp0<0x112, 0xf>(v);
+            v += dpp0<0x114, 0xf>(v);
+            v += dpp0<0x118, 0xf>(v);
+            if ((lane & 15) == 15) red[w][lane >> 4][q] = v;
+        }
+        __syncthreads();
+        if (t < 28) {
+            const int g = t / 7, q = t - g * 7;
+            if (i0 + g < nc)
+                f.part64[((size_t)bucket[i0 + g] * f.nsub + sub) * 7 + q] =
+                    ((red[0][g][q] + red[1][g][q]) + red[2][g][q]) + red[3][g][q];
+        }
+        __syncthreads();
+    }
 }
 
 // A batch's FP64 pass in two launches (small calls feel every launch): the segment
@@ -1801,16 +1912,20 @@ __global__ __launch_bounds__(256) void regf_segapply_kernel(ChunkFixParams f) {
 // (disjoint rows).
 template <bool MFLAG>
 __global__ __launch_bounds__(256) void regf_pass1_kernel(ChunkFixParams f, FixParams x, int gs,
-                                                         int gc) {
-    __shared__ double4 sA[JTILE], sB[JTILE];
+                                                         int gc, bool small) {
+    __shared__ double4 sA[2 * JTILE];
+    __shared__ int wtot[4];
     __shared__ int scnt[SEGCNT_LDS + 1];
     const int b = blockIdx.x;   // uniform per work-group
-    if (b < gs)
-        segfix_body<MFLAG>(f, b, gs, sA, sB, scnt);
-    else if (b < gs + gc)
-        cand_body<MFLAG>(f, b - gs, gc);
+    if (b < gs) {
+        if (small)
+            segfix_small_body<MFLAG>(f, b, gs, reinterpret_cast<double(*)[4][7]>(sA), wtot, scnt);
+        else
+            segfix_body<MFLAG>(f, b, gs, reinterpret_cast<double2(*)[256]>(sA), scnt, wtot);
+    } else if (b < gs + gc)
+        cand_body<MFLAG>(f, b - gs, gc, scnt, wtot);
     else
-        fix_body<MFLAG>(x, b - gs - gc, (int)gridDim.x - gs - gc, sA, sB);
+        fix_body<MFLAG>(x, b - gs - gc, (int)gridDim.x - gs - gc, sA, sA + JTILE);
 }
 __global__ __launch_bounds__(256) void regf_pass2_kernel(ChunkFixParams f, FixParams x, int ga) {
     const int b = blockIdx.x;
@@ -2223,9 +2338,8 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         tp.fnear = cfg.near;
         tp.nseg_c = P;
         tp.seg_tiles = P > 1 ? seglen / T : 0;
-        dim3 grid(bnib * nchunk);
         if (timed && b0 == 0) t1.start(s);
-        launch_tile(cfg, m_flag != 0, grid, tp, s);
+        launch_tile(cfg, m_flag != 0, dim3(bnib * nchunk), tp, s);
         NB6_HIP(hipGetLastError());
         if (timed && b0 + nb >= ni) t1.stop(s);
 
@@ -2307,8 +2421,11 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
             // grids); whole rows: at most (ni / 256 row groups) x (j tiles) items
             const int gc = (int)std::min<size_t>(CHUNKFIX_GROUPS,
                                                  ((size_t)nb * cp.row_items + 3) / 4);
+            // (by the whole call's size: a batched call gives the same bits)
+            const bool few = ni <= PASS_MERGE_NI && nseg <= SEGCNT_LDS;
+            const size_t ig = few ? 4 : 64;           // items per work unit
             const int gs = (int)std::min<size_t>(
-                CHUNKFIX_GROUPS, (size_t)nseg * (((size_t)nb + 255) / 256) * (size_t)nsub);
+                CHUNKFIX_GROUPS, (size_t)nseg * (((size_t)nb + ig - 1) / ig) * (size_t)nsub);
             const int gf = last ? (int)std::min<size_t>(fix_items, (((size_t)ni + 255) / 256) *
                                                       (((size_t)nj + JTILE - 1) / JTILE))
                                 : 0;
@@ -2318,10 +2435,10 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
                 // small batches: two launches
                 if (m_flag)
                     hipLaunchKernelGGL(regf_pass1_kernel<true>, dim3(gs + gc + gf), dim3(256), 0,
-                                       s, cp, xp, gs, gc);
+                                       s, cp, xp, gs, gc, few);
                 else
                     hipLaunchKernelGGL(regf_pass1_kernel<false>, dim3(gs + gc + gf), dim3(256), 0,
-                                       s, cp, xp, gs, gc);
+                                       s, cp, xp, gs, gc, few);
                 NB6_HIP(hipGetLastError());
                 hipLaunchKernelGGL(regf_pass2_kernel, dim3(ga + gr), dim3(256), 0, s, cp, xp, ga);
             } else {
