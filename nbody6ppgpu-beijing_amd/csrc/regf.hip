@@ -423,7 +423,10 @@ __device__ __forceinline__ void tile_work(const TileParams &p, int ibase, int ie
             if (js0 == 0 || (T > JTILE && js0 % JTILE == 0)) {
                 // i relative to the origin of the 256-j tile this segment lies in,
                 // and whether the whole wavefront is outside its near field
-                const size_t tt = (size_t)((jt + js0) / JTILE);
+                // (a 512-wide tile can end past the last 256-j tile: only massless dummy
+                // records lie there, and the last tile's origin and box serve them)
+                const int jl = jt + js0;
+                const size_t tt = (size_t)((T > JTILE && jl >= p.nj ? p.nj - 1 : jl) / JTILE);
                 bool far = p.far_test != 0;
 #pragma unroll
                 for (int k = 0; k < IPL; k++) {
