@@ -520,6 +520,175 @@ __global__ __launch_bounds__(T, (regf_waves<T, IPL>())) void regf_tile_kernel(Ti
                              sB);
 }
 
+// Form of regf_tile_kernel for calls whose 256-wide work-groups would not fill the GPU once
+// (regf_launch_impl): 64 i per work-group of four wavefronts, which take the four 64-j
+// pieces of each 256-j tile side by side.  Bound by latency: one wavefront walks 64 j in place
+// of 256.  Partial sums, error scales and candidate slots come out as the 256-wide form
+// leaves them, bit for bit: a piece is one FP32 partial sum there too, and wavefront 0 adds
+// the four in j order; which soft pairs still find a slot depends on the pieces before, so
+// the neighbour test runs first and leaves bit masks, from which every wavefront knows the
+// slots taken before its own, and the force loop leaves out the pairs that got one.
+// N = 50,021, ni = 257: 74 -> 42 us; N = 1024, ni = 40: 69 -> 32 us.
+struct PieceMask {
+    unsigned long long hard, soft, band;   // band: hard pairs that the FP64 test has to decide
+};
+
+// slot counts of one i past the 64 pairs of a piece; soft pairs that get a slot into kept
+__device__ __forceinline__ void piece_slots(const TileParams &p, const PieceMask &m, int &nh, int &ns,
+                                            unsigned long long &kept) {
+    const int lim = p.caps - BAND_SLOTS;
+    const int c = __popcll(m.hard), d = __popcll(m.soft);
+    if (nh + c <= p.caph && ns + d <= lim) {
+        kept = m.soft;
+        nh += c;
+        ns += d;
+        return;
+    }
+    kept = 0ull;
+    for (unsigned long long b = m.hard | m.soft; b; b &= b - 1) {
+        const unsigned long long bit = b & (0ull - b);
+        if (m.hard & bit) {
+            if (nh >= p.caph && (m.band & bit)) ns++;
+            nh++;
+        } else if (ns < lim) {
+            kept |= bit;
+            ns++;
+        }
+    }
+}
+
+template <bool MFLAG>
+__global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
+    __shared__ float4 sA[JTILE], sB[JTILE];
+    __shared__ PieceMask sM[4][64];
+    __shared__ float sP[4][8][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int b = xcd_order(blockIdx.x, gridDim.x);
+    const int chunk = b / p.nib;
+    const int i = (b - chunk * p.nib) * 64 + lane;   // slot
+    const int j0 = chunk * p.chunk_len, j1 = min(j0 + p.chunk_len, p.nj);
+    const bool in = i < p.ni;
+    int r = i;
+    if (in && p.imap) r = p.imap[i];
+    const bool ok = in && r >= 0;
+    const ILane L = make_lane<MFLAG>(p.ib, p.ib_stride, r, ok, p.mmax, p.fnear);
+    const size_t row = (size_t)chunk * p.ni + (in ? i : 0);
+    int *hp = p.hslot + row * p.caph, *sp = p.sslot + row * p.caps;
+    int nh = 0, ns = 0;                      // slots used, the same in every wavefront
+    double a64[7] = {0, 0, 0, 0, 0, 0, 0};   // (wavefront 0)
+    float err[NERR] = {0.f, 0.f, 0.f, 0.f};
+
+    for (int jt = j0; jt < j1; jt += JTILE) {
+        {
+            const int j = jt + (int)threadIdx.x;
+            const float4 *src = j < j1 ? p.rec32 + 2 * (size_t)j : g_far_rec;
+            __builtin_amdgcn_global_load_lds((glb_void *)src, (lds_void *)&sA[w * 64], 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((glb_void *)(src + 1), (lds_void *)&sB[w * 64], 16, 0, 0);
+        }
+        const size_t tt = (size_t)(jt / JTILE);
+        const IC c = tile_ic<MFLAG>(L, p.torg + tt * 8, p.tbox + tt * TBOX);
+        const bool near = !(p.far_test && lane_far<MFLAG>(c, ok, p.tbox + tt * TBOX));
+        lds_dma_wait();                      // a wavefront reads only the records it staged
+        PieceMask m = {0ull, 0ull, 0ull};
+        if (__ballot(near)) {
+#pragma unroll 4
+            for (int jj = 0; jj < 64; jj++) {
+                const float4 ra = sA[w * 64 + jj], rb = sB[w * 64 + jj];
+                const PairBase q = pair_base(c, ra, rb);
+                const float t1 = fmaf(c.dt2, fminf(q.rv, 0.f), q.r2);
+                const float thq = MFLAG ? fmaf(ra.w, c.hQ, c.dQ) : c.hQ;
+                if (t1 < thq && jt + w * 64 + jj < j1) {
+                    const float mn = pair_min(c, q);
+                    const float thh = MFLAG ? fmaf(ra.w, c.hH, c.dH) : c.hH;
+                    const float ths = MFLAG ? fmaf(ra.w, c.hS, c.dS) : c.hS;
+                    const float thl = MFLAG ? fmaf(ra.w, c.hL, -2.0f * c.dH) : c.hL;
+                    const unsigned long long bit = 1ull << jj;
+                    if (mn < thh) {
+                        m.hard |= bit;
+                        if (!(fmaf(KAPPA_P, q.r2, mn) < thl)) m.band |= bit;
+                    } else if (mn < ths) {
+                        m.soft |= bit;
+                    }
+                }
+            }
+        }
+        sM[w][lane] = m;
+        __syncthreads();
+        // slots before this piece, then this piece's own, then the tile's
+        unsigned long long kept = 0ull, left = 0ull;
+        for (int q = 0; q < 4; q++) {
+            int h = nh, s = ns;
+            piece_slots(p, sM[q][lane], nh, ns, kept);
+            if (q != w) continue;
+            left = m.hard | kept;
+            const int jp = jt + w * 64;
+            for (unsigned long long x = m.hard | kept; x; x &= x - 1) {
+                const int k = __builtin_ctzll(x);
+                const unsigned long long bit = x & (0ull - x);
+                if (!(m.hard & bit)) {
+                    sp[s++] = jp + k;
+                } else {
+                    if (h < p.caph) hp[h] = jp + k;
+                    else if (m.band & bit) {
+                        if (s < p.caps) sp[s] = ~(jp + k);
+                        s++;
+                    }
+                    h++;
+                }
+            }
+        }
+        float acc[NACC] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, s3 = 0.f;
+        if (__ballot(left != 0ull)) {
+#pragma unroll 4
+            for (int jj = 0; jj < 64; jj++) {
+                const float4 ra = sA[w * 64 + jj], rb = sB[w * 64 + jj];
+                const PairBase q = pair_base(c, ra, rb);
+                const float rinv = (left >> jj) & 1ull ? 0.f : rinv_nr(q.r2);
+                pair_add(q, rinv, ra.w, acc, s3);
+            }
+        } else {
+#pragma unroll 4
+            for (int jj = 0; jj < 64; jj++) {
+                const float4 ra = sA[w * 64 + jj], rb = sB[w * 64 + jj];
+                const PairBase q = pair_base(c, ra, rb);
+                pair_add(q, rinv_nr(q.r2), ra.w, acc, s3);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NACC; q++) sP[w][q][lane] = acc[q];
+        sP[w][7][lane] = s3;
+        __syncthreads();
+        if (w == 0) {
+            // as the 256-wide form flushes its FP32 partials every 64 j
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float v[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) v[q] = sP[u][q][lane];
+                a64[0] += (double)v[0];
+                a64[1] += (double)v[1];
+                a64[2] += (double)v[2];
+                a64[3] += (double)v[4];
+                a64[4] += (double)v[5];
+                a64[5] += (double)v[6];
+                a64[6] += (double)v[3];
+                err[0] += fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]);
+                err[1] += fabsf(v[4]) + fabsf(v[5]) + fabsf(v[6]);
+                err[2] = fmaf(v[7], c.eP, err[2]);
+                err[3] = fmaf(v[7], c.eV, err[3]);
+            }
+        }
+    }
+    if (w != 0 || !in) return;
+    double *pp = p.part + (size_t)chunk * NPART * p.ni + i;
+#pragma unroll
+    for (int f = 0; f < 7; f++) pp[(size_t)f * p.ni] = a64[f];
+#pragma unroll
+    for (int f = 0; f < NERR; f++) pp[(size_t)(7 + f) * p.ni] = (double)err[f];
+    p.cnt[((size_t)chunk * 2 + 0) * p.ni + i] = nh;
+    p.cnt[((size_t)chunk * 2 + 1) * p.ni + i] = ns;
+}
+
 // Persistent form for a batch of independent clusters: each work-group takes the
 // next work item from a queue (items are ordered longest first) until none is left.
 template <int T, int IPL, bool MFLAG>
@@ -2216,6 +2385,12 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         nbatch_i = (int)std::max<size_t>((size_t)nbi, rows_max / (size_t)nchunk / nbi * nbi);
         nbatch_i = std::min(nbatch_i, ni);
     }
+    // 64 i per work-group and the tile's four pieces side by side (the same bits) up to 1792
+    // such work-groups, seven per CU; with more the 256-wide form fills the GPU by itself and
+    // runs the neighbour test and the force in one loop.  Whole call: N = 65,536, ni = 256
+    // (1024 of them) 244 -> 216 us, ni = 512 (2048) 248 and 250, ni = 700 (2816) 262 and 279
+    const bool small = cfg.prec == 0 && cfg.threads == 256 && cfg.ipl == 1 && P == 1 &&
+                       (long long)((ni + 63) / 64) * nchunk <= 1792;
     const size_t rows = (size_t)nchunk * nbatch_i;
     // rows the finalize flags for the FP64 pass (FP32 production kernel only)
     const int fix_items = na ? na->fix_items : FIX_ITEMS;
@@ -2342,7 +2517,16 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         tp.nseg_c = P;
         tp.seg_tiles = P > 1 ? seglen / T : 0;
         if (timed && b0 == 0) t1.start(s);
-        launch_tile(cfg, m_flag != 0, dim3(bnib * nchunk), tp, s);
+        if (small) {
+            tp.nib = (nb + 63) / 64;
+            const dim3 grid(tp.nib * nchunk);
+            if (m_flag)
+                hipLaunchKernelGGL(regf_tile_small_kernel<true>, grid, dim3(256), 0, s, tp);
+            else
+                hipLaunchKernelGGL(regf_tile_small_kernel<false>, grid, dim3(256), 0, s, tp);
+        } else {
+            launch_tile(cfg, m_flag != 0, dim3(bnib * nchunk), tp, s);
+        }
         NB6_HIP(hipGetLastError());
         if (timed && b0 + nb >= ni) t1.stop(s);
 
