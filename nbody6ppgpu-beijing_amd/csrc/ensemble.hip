@@ -37,14 +37,18 @@ __device__ __forceinline__ unsigned spread10e(unsigned a) {
     return a;
 }
 
-// per-cluster bounding box and maximum mass: one work-group per cluster
-__global__ __launch_bounds__(256) void ens_bbox_kernel(const double *__restrict__ aos,
-                                                       const int *__restrict__ off,
-                                                       double *__restrict__ box) {
-    __shared__ double sh[7][256];
-    const int c = blockIdx.x;
+// per-cluster bounding box and maximum mass: one work-group per cluster; the maximum mass of
+// all of them (positive, so its bits order as it does) into *mmax
+constexpr int EB = 1024;
+__global__ __launch_bounds__(EB) void ens_bbox_kernel(const double *__restrict__ aos,
+                                                      const int *__restrict__ off,
+                                                      double *__restrict__ box,
+                                                      unsigned long long *__restrict__ mmax) {
+    __shared__ double sh[EB / 64][7];
+    const int c = blockIdx.x, t = threadIdx.x;
     double v[7] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX, 0.0};
-    for (int j = off[c] + threadIdx.x; j < off[c + 1]; j += 256) {
+#pragma unroll 4
+    for (int j = off[c] + t; j < off[c + 1]; j += EB) {
         const double *r = aos + (size_t)j * 8;
         for (int d = 0; d < 3; d++) {
             v[d] = fmin(v[d], r[d]);
@@ -52,16 +56,22 @@ __global__ __launch_bounds__(256) void ens_bbox_kernel(const double *__restrict_
         }
         v[6] = fmax(v[6], r[3]);
     }
-    for (int q = 0; q < 7; q++) sh[q][threadIdx.x] = v[q];
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            for (int d = 0; d < 3; d++) sh[d][threadIdx.x] = fmin(sh[d][threadIdx.x], sh[d][threadIdx.x + o]);
-            for (int d = 3; d < 7; d++) sh[d][threadIdx.x] = fmax(sh[d][threadIdx.x], sh[d][threadIdx.x + o]);
+#pragma unroll
+    for (int q = 0; q < 7; q++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const double u = __shfl_xor(v[q], o, 64);
+            v[q] = q < 3 ? fmin(v[q], u) : fmax(v[q], u);
         }
-        __syncthreads();
+        if ((t & 63) == 0) sh[t >> 6][q] = v[q];
     }
-    if (threadIdx.x < 7) box[c * 7 + threadIdx.x] = sh[threadIdx.x][0];
+    __syncthreads();
+    if (t < 7) {
+        double u = sh[0][t];
+        for (int w = 1; w < EB / 64; w++) u = t < 3 ? fmin(u, sh[w][t]) : fmax(u, sh[w][t]);
+        box[c * 7 + t] = u;
+        if (t == 6) atomicMax(mmax, (unsigned long long)__double_as_longlong(u));
+    }
 }
 
 __global__ __launch_bounds__(256) void ens_key_kernel(const double *__restrict__ aos, int n,
@@ -85,40 +95,11 @@ __global__ __launch_bounds__(256) void ens_key_kernel(const double *__restrict__
     val[j] = j;
 }
 
-// fill every padded slot with a far massless dummy (overwritten for real particles)
-__global__ __launch_bounds__(256) void ens_dummy_kernel(double *__restrict__ rec64,
-                                                        int *__restrict__ perm, int npad) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= npad) return;
-    double *o = rec64 + (size_t)s * 8;
-    o[0] = 1.0e17; o[1] = 0.0; o[2] = 0.0; o[3] = 0.0;
-    o[4] = 0.0; o[5] = 0.0; o[6] = 0.0; o[7] = 0.0;
-    perm[s] = -1;
-}
-
-// compact sorted position s -> padded position (cluster start + rank in cluster)
-__global__ __launch_bounds__(256) void ens_scatter_kernel(const double *__restrict__ in, int n,
-                                                          const int *__restrict__ sorted,
-                                                          const int *__restrict__ cid,
-                                                          const int *__restrict__ off,
-                                                          const int *__restrict__ padoff,
-                                                          double *__restrict__ rec64,
-                                                          int *__restrict__ perm) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= n) return;
-    const int j = sorted[s];
-    const int c = cid[j];
-    const int ps = padoff[c] + (s - off[c]);   // clusters keep their order in the sort
-    const double *r = in + (size_t)j * 8;
-    double *o = rec64 + (size_t)ps * 8;
-#pragma unroll
-    for (int f = 0; f < 8; f++) o[f] = r[f];
-    perm[ps] = j;
-}
-
 __global__ __launch_bounds__(256) void ens_soa_to_aos(const double *__restrict__ soa, int n,
-                                                      int stride, double *__restrict__ aos) {
+                                                      int stride, double *__restrict__ aos,
+                                                      double *__restrict__ mmax) {
     const int j = blockIdx.x * 256 + threadIdx.x;
+    if (j == 0) *mmax = 0.0;             // (ens_bbox_kernel's maximum)
     if (j >= n) return;
     double *o = aos + (size_t)j * 8;
     o[0] = soa[0 * (size_t)stride + j];
@@ -296,9 +277,12 @@ int ens_send_device(int nc, const int *offsets, const double *d_soa, int stride,
     }
     const int n = e.ntot;
     double *in64 = e.js.in64.as<double>();
-    hipLaunchKernelGGL(ens_soa_to_aos, dim3((n + 255) / 256), dim3(256), 0, s, d_soa, n, stride, in64);
-    hipLaunchKernelGGL(ens_bbox_kernel, dim3(nc), dim3(256), 0, s, in64, e.d_off.as<int>(),
-                       e.d_box.as<double>());
+    double *mmax = e.js.stat.as<double>() + 6;
+    hipLaunchKernelGGL(ens_soa_to_aos, dim3((n + 255) / 256), dim3(256), 0, s, d_soa, n, stride, in64,
+                       mmax);
+    jset_input_queued(e.js, s);
+    hipLaunchKernelGGL(ens_bbox_kernel, dim3(nc), dim3(EB), 0, s, in64, e.d_off.as<int>(),
+                       e.d_box.as<double>(), reinterpret_cast<unsigned long long *>(mmax));
     hipLaunchKernelGGL(ens_key_kernel, dim3((n + 255) / 256), dim3(256), 0, s, in64, n,
                        e.d_cid.as<int>(), e.d_box.as<double>(),
                        e.d_keys.as<unsigned long long>(), e.d_vals.as<int>());
@@ -313,25 +297,11 @@ int ens_send_device(int nc, const int *offsets, const double *d_soa, int stride,
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, e.d_keys.as<unsigned long long>(),
                                                e.d_skeys.as<unsigned long long>(), e.d_vals.as<int>(),
                                                e.d_svals.as<int>(), n, 0, hi, s));
-    const int np = e.npad;
-    hipLaunchKernelGGL(ens_dummy_kernel, dim3((np + 255) / 256), dim3(256), 0, s,
-                       e.js.rec64.as<double>(), e.js.perm.as<int>(), np);
-    hipLaunchKernelGGL(ens_scatter_kernel, dim3((n + 255) / 256), dim3(256), 0, s, in64, n,
-                       e.d_svals.as<int>(), e.d_cid.as<int>(), e.d_off.as<int>(),
-                       e.d_padoff.as<int>(), e.js.rec64.as<double>(), e.js.perm.as<int>());
-    NB6_HIP(hipGetLastError());
     // tile origins and FP32 records on the padded layout: P from a tile's first record
     // (padding sits at the end of a cluster's last tile)
-    jset_tiles(e.js, np, 0, s);
-    e.js.n = np;
-    e.js.ntile = np / JTILE;
-    // maximum mass, for the m_flag error band
-    std::vector<double> box((size_t)nc * 7);
-    NB6_HIP(hipMemcpyAsync(box.data(), e.d_box.p, box.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-    NB6_HIP(hipStreamSynchronize(s));
-    double mmax = 0.0;
-    for (int c = 0; c < nc; c++) mmax = std::max(mmax, box[(size_t)c * 7 + 6]);
-    e.js.mmax = mmax;
+    jset_build_clusters(e.js, e.npad, in64, e.d_svals.as<int>(), e.d_off.as<int>(),
+                        e.d_padoff.as<int>(), nc, s);
+    jset_input_wait(e.js);
     const RegfConfig cfg = regf_effective(0);
     if (same_layout && e.items_bi == cfg.threads * cfg.ipl) return OK;
     const int rc = build_items(e, s);
@@ -361,17 +331,15 @@ int ens_regf_device(const double *d_i, int stride, int lmax, int nnbmax, int m_f
                                  nnbmax, m_flag, d_out, d_list, grid, e.work, st);
     };
     if (!use_graph) return step(s);
-    // The graph holds kernel arguments by value: pointers, sizes, the launch shape and
-    // (for m_flag) the maximum mass of the j-set.  Any change there needs a new capture.
+    // The graph holds kernel arguments by value: pointers, sizes and the launch shape.  Any
+    // change there needs a new capture.
     GraphKey key;
     key.ptr[0] = d_i; key.ptr[1] = d_out; key.ptr[2] = d_list; key.ptr[3] = e.d_items.p;
-    long long mbits = 0;
-    if (m_flag) std::memcpy(&mbits, &e.js.mmax, sizeof(mbits));
     int nbits = 0, kb[4] = {0, 0, 0, 0};
     std::memcpy(&nbits, &cfg.near, sizeof(nbits));
     std::memcpy(kb, cfg.kref_ens, sizeof(kb));
     const long long v[18] = {stride, lmax, nnbmax, m_flag, cfg.threads, cfg.ipl, e.nitems, grid,
-                             e.ntot, e.npad, mbits, cfg.far_test, cfg.refine, nbits,
+                             e.ntot, e.npad, 0, cfg.far_test, cfg.refine, nbits,
                              kb[0], kb[1], kb[2], kb[3]};
     std::copy(v, v + 18, key.val);
     const bool same = e.exec && key == e.gkey;

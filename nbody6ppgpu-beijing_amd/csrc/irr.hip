@@ -315,14 +315,18 @@ __global__ __launch_bounds__(256) void irr_force_kernel(
 
 // Morton key of each active i's record position (for the processing order)
 __global__ __launch_bounds__(256) void irr_key_kernel(int ni, const int *__restrict__ addr,
-                                                      const IrrRec *__restrict__ rec, double lx,
-                                                      double ly, double lz, double sx, double sy,
-                                                      double sz, unsigned *__restrict__ key,
+                                                      const IrrRec *__restrict__ rec,
+                                                      const double *__restrict__ box,
+                                                      unsigned *__restrict__ key,
                                                       int *__restrict__ val) {
     const int w = blockIdx.x * 256 + threadIdx.x;
     if (w >= ni) return;
     const IrrRec &r = rec[addr[w] - 1];
-    const double f[3] = {(r.x - lx) * sx, (r.y - ly) * sy, (r.z - lz) * sz};
+    double f[3] = {r.x, r.y, r.z};
+    for (int d = 0; d < 3; d++) {
+        const double wd = box[3 + d] - box[d];
+        f[d] = (f[d] - box[d]) * (wd > 0.0 ? 1024.0 / (wd * (1.0 + 1e-12)) : 0.0);
+    }
     unsigned q[3];
     for (int d = 0; d < 3; d++) q[d] = f[d] > 0.0 ? (f[d] < 1023.0 ? (unsigned)f[d] : 1023u) : 0u;
     unsigned kk = 0;
@@ -430,18 +434,12 @@ const int *irr_order(int ni, const int *d_addr, const int **oaddr, hipStream_t s
     const JSet *js = gpunb_jset();
     *oaddr = d_addr;
     if (!g_irrcfg.sort_i || ni < 2048 || !js || js->n <= 0) return nullptr;
-    double sc[3];
-    for (int d = 0; d < 3; d++) {
-        const double w = js->box[3 + d] - js->box[d];
-        sc[d] = w > 0.0 ? 1024.0 / (w * (1.0 + 1e-12)) : 0.0;
-    }
     unsigned *k0 = static_cast<unsigned *>(g.d_okey.get((size_t)ni * 2 * sizeof(unsigned)));
     unsigned *k1 = k0 + ni;
     int *v0 = static_cast<int *>(g.d_oval.get((size_t)ni * 2 * sizeof(int)));
     int *v1 = v0 + ni;
     hipLaunchKernelGGL(irr_key_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, ni, d_addr,
-                       g.rec.as<IrrRec>(), js->box[0], js->box[1], js->box[2], sc[0], sc[1], sc[2],
-                       k0, v0);
+                       g.rec.as<IrrRec>(), js->stat.as<double>(), k0, v0);
     NB6_HIP(hipGetLastError());
     size_t tb = 0;
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, ni, 0, 30, s));

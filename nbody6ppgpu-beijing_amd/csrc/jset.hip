@@ -48,196 +48,243 @@ __device__ __forceinline__ unsigned long long morton63(double x, double y, doubl
     return spread21(qx) | (spread21(qy) << 1) | (spread21(qz) << 2);
 }
 
+constexpr int STATS_GROUPS = 512;
+
+__device__ __forceinline__ void stat_identity(double *v) {
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        v[d] = DBL_MAX;
+        v[3 + d] = -DBL_MAX;
+    }
+    v[6] = 0.0;
+}
+__device__ __forceinline__ void stat_add(double *v, double x, double y, double z, double m) {
+    const double r[3] = {x, y, z};
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        v[d] = fmin(v[d], r[d]);
+        v[3 + d] = fmax(v[3 + d], r[d]);
+    }
+    v[6] = fmax(v[6], m);
+}
+// bounds (lo[3], hi[3]) and maximum mass over the 256 threads, in every thread
+__device__ __forceinline__ void stat_group(double *v, double (*sh)[8]) {
+#pragma unroll
+    for (int q = 0; q < 7; q++)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const double u = __shfl_xor(v[q], o, 64);
+            v[q] = q < 3 ? fmin(v[q], u) : fmax(v[q], u);
+        }
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int q = 0; q < 7; q++) sh[threadIdx.x >> 6][q] = v[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 7; q++)
+#pragma unroll
+        for (int w = 0; w < 4; w++) v[q] = q < 3 ? fmin(v[q], sh[w][q]) : fmax(v[q], sh[w][q]);
+}
+
+// SoA [7][stride] (x y z vx vy vz m; null: aos is there already) -> AoS [n][8] (x y z m vx vy
+// vz 0), and each work-group's bounds and maximum mass: part[group][7]
+__global__ __launch_bounds__(256) void aos_stats_kernel(const double *__restrict__ soa, int n,
+                                                        int stride, double *__restrict__ aos,
+                                                        double *__restrict__ part) {
+    __shared__ double sh[4][8];
+    double v[7];
+    stat_identity(v);
+    for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
+        double *o = aos + (size_t)j * 8;
+        if (soa) {
+            const size_t st = stride;
+            const double x = soa[j], y = soa[st + j], z = soa[2 * st + j], m = soa[6 * st + j];
+            o[0] = x; o[1] = y; o[2] = z; o[3] = m;
+            o[4] = soa[3 * st + j]; o[5] = soa[4 * st + j]; o[6] = soa[5 * st + j];
+            o[7] = 0.0;
+            stat_add(v, x, y, z, m);
+        } else {
+            stat_add(v, o[0], o[1], o[2], o[3]);
+        }
+    }
+    stat_group(v, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q < 7; q++) part[blockIdx.x * 7 + q] = v[q];
+}
+
+struct JStat {
+    double v[7];             // lo[3], hi[3], maximum mass
+};
+__device__ __forceinline__ double morton_scale(const double *box, int d) {
+    const double w = box[3 + d] - box[d];
+    return w > 0.0 ? MORTON_CELLS / (w * (1.0 + 1e-12)) : 0.0;
+}
+
+// Morton keys of the AoS positions in their box, from the groups' bounds (every work-group
+// reduces them: cheaper than a launch) or, with groups = 0, from `host`; the first
+// work-group leaves the bounds and the maximum mass in stat[7]
 __global__ __launch_bounds__(256) void morton_kernel(const double *__restrict__ in, int n,
-                                                     double lx, double ly, double lz, double sx,
-                                                     double sy, double sz,
+                                                     const double *__restrict__ part, int groups,
+                                                     JStat host, double *__restrict__ stat,
                                                      unsigned long long *__restrict__ key,
                                                      int *__restrict__ val) {
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= n) return;
-    const double *r = in + (size_t)j * 8;
-    key[j] = morton63(r[0], r[1], r[2], lx, ly, lz, sx, sy, sz);
-    val[j] = j;
-}
-
-// sorted position s <- original j = perm[s]
-__global__ __launch_bounds__(256) void build_kernel(const double *__restrict__ in, int n,
-                                                    const int *__restrict__ perm,
-                                                    double *__restrict__ rec64) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= n) return;
-    const double *r = in + (size_t)perm[s] * 8;
-    double *o = rec64 + (size_t)s * 8;
+    __shared__ double sh[4][8];
+    double v[7];
+    if (groups > 0) {
+        stat_identity(v);
+        for (int g = threadIdx.x; g < groups; g += 256)
 #pragma unroll
-    for (int f = 0; f < 8; f++) o[f] = r[f];
+            for (int q = 0; q < 7; q++) {
+                const double u = part[g * 7 + q];
+                v[q] = q < 3 ? fmin(v[q], u) : fmax(v[q], u);
+            }
+        stat_group(v, sh);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 7; q++) v[q] = host.v[q];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q < 7; q++) stat[q] = v[q];
+    const double sx = morton_scale(v, 0), sy = morton_scale(v, 1), sz = morton_scale(v, 2);
+    for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
+        const double *r = in + (size_t)j * 8;
+        key[j] = morton63(r[0], r[1], r[2], v[0], v[1], v[2], sx, sy, sz);
+        val[j] = j;
+    }
 }
 
-// One work-group per tile: P = position of record `pos` of the tile (its middle one,
-// or its first), V = mean velocity of the tile's records with m > 0 (that record's
-// velocity if there are none).
-__global__ __launch_bounds__(256) void origin_kernel(const double *__restrict__ rec64, int n,
-                                                     int middle, double *__restrict__ torg) {
-    __shared__ double sh[4][4];
-    const int t = blockIdx.x;
+// Morton key of i-particle positions (SoA rows 0-2) in the j-set's box (clamped)
+__global__ __launch_bounds__(256) void imorton_kernel(const double *__restrict__ ib, int stride,
+                                                      int ni, const double *__restrict__ box,
+                                                      unsigned long long *__restrict__ key,
+                                                      int *__restrict__ val) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= ni) return;
+    key[i] = morton63(ib[i], ib[(size_t)stride + i], ib[2 * (size_t)stride + i], box[0], box[1],
+                      box[2], morton_scale(box, 0), morton_scale(box, 1), morton_scale(box, 2));
+    val[i] = i;
+}
+
+// v and the lane that the DPP pattern names (the lane's own value where there is none)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_bound(float v, bool lo) {
+    const int i = __float_as_int(v);
+    const float u = __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false));
+    return lo ? fminf(v, u) : fmaxf(v, u);
+}
+
+// One work-group per tile: the records in sorted order (rec64), the tile's origin, its FP32
+// records relative to the origin and their bounds (JSet::tbox), in one pass over the
+// records.  P = position of the tile's middle record (its first in the padded layout), V =
+// mean velocity of the tile's records with m > 0 (that record's velocity if there are none).
+// Plain j-set (padoff null): position s holds the caller's record perm[s].  Padded layout of
+// independent clusters: slot s of cluster c (padoff) holds record sorted[off[c] + s -
+// padoff[c]] of the compact order, or past the cluster's last one a far massless record, and
+// perm is written.  Four launches of separate kernels took 17 us at N = 50,021 where this
+// takes 8.7.
+__global__ __launch_bounds__(256) void tile_build_kernel(
+    const double *__restrict__ in, int n, int *__restrict__ perm, const int *__restrict__ sorted,
+    const int *__restrict__ off, const int *__restrict__ padoff, int nc,
+    double *__restrict__ rec64, double *__restrict__ torg, float4 *__restrict__ rec32,
+    float *__restrict__ tbox) {
+    __shared__ double sh[4][4], rep[6], org[6];
+    __shared__ float sb[4][16];
+    const int t = blockIdx.x, k = threadIdx.x, lane = k & 63, w = k >> 6;
+    const int s = t * JTILE + k;
     const int c = min(JTILE, n - t * JTILE);
-    const int k = threadIdx.x;
-    const double *r = rec64 + ((size_t)t * JTILE + k) * 8;
+    const int mid = padoff ? 0 : c / 2;
+    int j = -1;
+    if (padoff) {
+        int cl = 0, hi = nc;             // the cluster with padoff[cl] <= tile start (uniform)
+        while (hi - cl > 1) {
+            const int m = (cl + hi) >> 1;
+            if (padoff[m] <= t * JTILE) cl = m; else hi = m;
+        }
+        const int q = off[cl] + (s - padoff[cl]);
+        if (q < off[cl + 1]) j = sorted[q];
+        perm[s] = j;
+    } else if (k < c) {
+        j = perm[s];
+    }
+    double r[8] = {1.0e17, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (j >= 0) {
+        const double2 *p = reinterpret_cast<const double2 *>(in + (size_t)j * 8);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const double2 u = p[q];
+            r[2 * q] = u.x;
+            r[2 * q + 1] = u.y;
+        }
+    }
+    if (k < c) {
+        double2 *o = reinterpret_cast<double2 *>(rec64 + (size_t)s * 8);
+#pragma unroll
+        for (int q = 0; q < 4; q++) o[q] = make_double2(r[2 * q], r[2 * q + 1]);
+    }
     const bool use = k < c && r[3] > 0.0;
     double q[4] = {use ? r[4] : 0.0, use ? r[5] : 0.0, use ? r[6] : 0.0, use ? 1.0 : 0.0};
 #pragma unroll
     for (int f = 0; f < 4; f++)
         for (int o = 32; o > 0; o >>= 1) q[f] += __shfl_xor(q[f], o, 64);
-    if ((k & 63) == 0)
-        for (int f = 0; f < 4; f++) sh[k >> 6][f] = q[f];
+    if (lane == 0)
+        for (int f = 0; f < 4; f++) sh[w][f] = q[f];
+    if (k == mid) {
+        rep[0] = r[0]; rep[1] = r[1]; rep[2] = r[2];
+        rep[3] = r[4]; rep[4] = r[5]; rep[5] = r[6];
+    }
     __syncthreads();
     if (k == 0) {
         double v[4];
         for (int f = 0; f < 4; f++) v[f] = (sh[0][f] + sh[1][f]) + (sh[2][f] + sh[3][f]);
-        const double *p = rec64 + ((size_t)t * JTILE + (middle ? c / 2 : 0)) * 8;
         double *o = torg + (size_t)t * 8;
-        o[0] = p[0]; o[1] = p[1]; o[2] = p[2];
-        if (v[3] > 0.0) {
-            o[3] = v[0] / v[3]; o[4] = v[1] / v[3]; o[5] = v[2] / v[3];
-        } else {
-            o[3] = p[4]; o[4] = p[5]; o[5] = p[6];
+        for (int f = 0; f < 3; f++) {
+            org[f] = rep[f];
+            org[3 + f] = v[3] > 0.0 ? v[f] / v[3] : rep[3 + f];
+            o[f] = org[f];
+            o[3 + f] = org[3 + f];
         }
         o[6] = 0.0; o[7] = 0.0;
     }
-}
-
-// FP32 records relative to their tile's origin
-__global__ __launch_bounds__(256) void rec32_kernel(const double *__restrict__ rec64, int n,
-                                                    const double *__restrict__ torg,
-                                                    float4 *__restrict__ rec32) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= n) return;
-    const double *p = torg + (size_t)(s / JTILE) * 8;
-    const double *r = rec64 + (size_t)s * 8;
-    rec32[2 * (size_t)s] = make_float4((float)(r[0] - p[0]), (float)(r[1] - p[1]),
-                                       (float)(r[2] - p[2]), (float)r[3]);
-    rec32[2 * (size_t)s + 1] = make_float4((float)(r[4] - p[3]), (float)(r[5] - p[4]),
-                                           (float)(r[6] - p[5]), 0.f);
-}
-
-// SoA [7][stride] (x y z vx vy vz m) -> AoS [n][8] (x y z m vx vy vz 0)
-__global__ __launch_bounds__(256) void soa_to_aos_kernel(const double *__restrict__ soa,
-                                                         int n, int stride,
-                                                         double *__restrict__ aos) {
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= n) return;
-    double *o = aos + (size_t)j * 8;
-    o[0] = soa[0 * (size_t)stride + j];
-    o[1] = soa[1 * (size_t)stride + j];
-    o[2] = soa[2 * (size_t)stride + j];
-    o[3] = soa[6 * (size_t)stride + j];
-    o[4] = soa[3 * (size_t)stride + j];
-    o[5] = soa[4 * (size_t)stride + j];
-    o[6] = soa[5 * (size_t)stride + j];
-    o[7] = 0.0;
-}
-
-// bounding box of positions and maximum mass, pass 1: each work-group reduces a
-// strided share of the records into one partial row of 7
-constexpr int STATS_GROUPS = 256;
-
-__global__ __launch_bounds__(256) void stats_kernel(const double *__restrict__ aos, int n,
-                                                    double *__restrict__ part /* [groups][7] */) {
-    __shared__ double sh[7][256];
-    double v[7] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX, 0.0};
-    for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
-        const double *r = aos + (size_t)j * 8;
-        for (int d = 0; d < 3; d++) {
-            v[d] = fmin(v[d], r[d]);
-            v[3 + d] = fmax(v[3 + d], r[d]);
-        }
-        v[6] = fmax(v[6], r[3]);
-    }
-    for (int q = 0; q < 7; q++) sh[q][threadIdx.x] = v[q];
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            for (int d = 0; d < 3; d++) sh[d][threadIdx.x] = fmin(sh[d][threadIdx.x], sh[d][threadIdx.x + o]);
-            for (int d = 3; d < 7; d++) sh[d][threadIdx.x] = fmax(sh[d][threadIdx.x], sh[d][threadIdx.x + o]);
-        }
-        __syncthreads();
+    const float4 a = make_float4((float)(r[0] - org[0]), (float)(r[1] - org[1]),
+                                 (float)(r[2] - org[2]), (float)r[3]);
+    const float4 b = make_float4((float)(r[4] - org[3]), (float)(r[5] - org[4]),
+                                 (float)(r[6] - org[5]), 0.f);
+    if (k < c) {
+        rec32[2 * (size_t)s] = a;
+        rec32[2 * (size_t)s + 1] = b;
     }
-    if (threadIdx.x < 7) part[blockIdx.x * 7 + threadIdx.x] = sh[threadIdx.x][0];
-}
-
-// pass 2: one work-group reduces the partial rows
-__global__ __launch_bounds__(256) void stats_final_kernel(const double *__restrict__ part, int groups,
-                                                          double *__restrict__ out /* 7 */) {
-    __shared__ double sh[7][256];
-    const int t = threadIdx.x;
-    for (int q = 0; q < 7; q++) {
-        const double id = q < 3 ? DBL_MAX : (q < 6 ? -DBL_MAX : 0.0);
-        sh[q][t] = t < groups ? part[t * 7 + q] : id;
-    }
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (t < o) {
-            for (int d = 0; d < 3; d++) sh[d][t] = fmin(sh[d][t], sh[d][t + o]);
-            for (int d = 3; d < 7; d++) sh[d][t] = fmax(sh[d][t], sh[d][t + o]);
-        }
-        __syncthreads();
-    }
-    if (t < 7) out[t] = sh[t][0];
-}
-
-// Morton key of i-particle positions (SoA rows 0-2) in a given box (clamped)
-__global__ __launch_bounds__(256) void imorton_kernel(const double *__restrict__ ib, int stride,
-                                                      int ni, double lx, double ly, double lz,
-                                                      double sx, double sy, double sz,
-                                                      unsigned long long *__restrict__ key,
-                                                      int *__restrict__ val) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= ni) return;
-    key[i] = morton63(ib[i], ib[(size_t)stride + i], ib[2 * (size_t)stride + i], lx, ly, lz, sx,
-                      sy, sz);
-    val[i] = i;
-}
-
-// FP32 bounds of one tile's tile-relative records (see JSet::tbox)
-__global__ __launch_bounds__(256) void tile_box_kernel(const float4 *__restrict__ rec32, int n,
-                                                       float *__restrict__ tbox) {
-    __shared__ float sh[14][256];
-    const int t = blockIdx.x;
-    const int s = t * JTILE + threadIdx.x;
-    float v[14];
+    // bounds: position lo[3], hi[3], velocity lo[3], hi[3], maximum mass, record count
+    const bool in_box = k < c && fabsf(a.x) < 1.0e16f;
+    float v[13] = {a.x, a.y, a.z, a.x, a.y, a.z, b.x, b.y, b.z, b.x, b.y, b.z, a.w};
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-        v[q] = FLT_MAX; v[3 + q] = -FLT_MAX; v[6 + q] = FLT_MAX; v[9 + q] = -FLT_MAX;
+    for (int f = 0; f < 13; f++) {
+        const bool lo = f < 3 || (f >= 6 && f < 9);
+        if (!in_box) v[f] = lo ? FLT_MAX : (f == 12 ? 0.f : -FLT_MAX);
+        // (row_shr 1, 2, 4, 8, row_bcast 15, 31: lane 63 has seen every lane)
+        v[f] = dpp_bound<0x111, 0xf>(v[f], lo);
+        v[f] = dpp_bound<0x112, 0xf>(v[f], lo);
+        v[f] = dpp_bound<0x114, 0xf>(v[f], lo);
+        v[f] = dpp_bound<0x118, 0xf>(v[f], lo);
+        v[f] = dpp_bound<0x142, 0xa>(v[f], lo);
+        v[f] = dpp_bound<0x143, 0xc>(v[f], lo);
+        if (lane == 63) sb[w][f] = v[f];
     }
-    v[12] = 0.f;
-    v[13] = 0.f;
-    if (threadIdx.x < JTILE && s < n) {
-        const float4 a = rec32[2 * (size_t)s];
-        const float4 b = rec32[2 * (size_t)s + 1];
-        if (fabsf(a.x) < 1.0e16f) {
-            v[0] = v[3] = a.x; v[1] = v[4] = a.y; v[2] = v[5] = a.z;
-            v[6] = v[9] = b.x; v[7] = v[10] = b.y; v[8] = v[11] = b.z;
-            v[12] = a.w;
-            v[13] = 1.f;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 14; q++) sh[q][threadIdx.x] = v[q];
+    const unsigned long long held = __ballot(in_box);
+    if (lane == 63) sb[w][13] = (float)__popcll(held);
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            const int u = threadIdx.x, w = threadIdx.x + o;
-            for (int q = 0; q < 3; q++) {
-                sh[q][u] = fminf(sh[q][u], sh[q][w]);
-                sh[3 + q][u] = fmaxf(sh[3 + q][u], sh[3 + q][w]);
-                sh[6 + q][u] = fminf(sh[6 + q][u], sh[6 + q][w]);
-                sh[9 + q][u] = fmaxf(sh[9 + q][u], sh[9 + q][w]);
-            }
-            sh[12][u] = fmaxf(sh[12][u], sh[12][w]);
-            sh[13][u] += sh[13][w];
+    if (k < TBOX) {
+        float u = 0.f;
+        if (k < 14) {
+            const bool lo = k < 3 || (k >= 6 && k < 9);
+            u = sb[0][k];
+            for (int x = 1; x < 4; x++)
+                u = k == 13 ? u + sb[x][k] : (lo ? fminf(u, sb[x][k]) : fmaxf(u, sb[x][k]));
         }
-        __syncthreads();
+        tbox[(size_t)t * TBOX + k] = u;
     }
-    if (threadIdx.x < TBOX) tbox[(size_t)t * TBOX + threadIdx.x] = threadIdx.x < 14 ? sh[threadIdx.x][0] : 0.f;
 }
 
 // plain streaming copy (used to calibrate HBM byte counters against a known size)
@@ -269,16 +316,8 @@ void jset_reserve(JSet &js, int cap) {
     js.perm.get((size_t)cap * sizeof(int));
     js.keys.get((size_t)cap * 2 * sizeof(unsigned long long));
     js.vals.get((size_t)cap * sizeof(int));
-    js.stat.get((8 + 7 * STATS_GROUPS) * sizeof(double));
+    js.stat.get((8 + 7 * STATS_GROUPS) * sizeof(double));   // stat[7], groups' parts
     js.tbox.get((size_t)ntile * TBOX * sizeof(float));
-}
-
-void jset_tile_boxes(JSet &js, int n, hipStream_t s) {
-    const int nt = (n + JTILE - 1) / JTILE;
-    if (nt <= 0) return;
-    hipLaunchKernelGGL(tile_box_kernel, dim3(nt), dim3(256), 0, s, js.rec32.as<float4>(), n,
-                       js.tbox.as<float>());
-    NB6_HIP(hipGetLastError());
 }
 
 void jset_release(JSet &js) {
@@ -286,74 +325,80 @@ void jset_release(JSet &js) {
     js.perm.release(); js.keys.release(); js.vals.release(); js.stat.release();
     js.sort_tmp.release(); js.tbox.release();
     js.cap = 0; js.n = 0; js.ntile = 0;
+    if (js.read) (void)hipEventDestroy(js.read);
+    js.read = nullptr;
 }
 
-// in64 holds n AoS records in the caller's order; box = {lo[3], hi[3]} or nullptr
-void jset_build(JSet &js, int n, const double *box, double mmax, hipStream_t s) {
+// The caller's input has been read once the work queued so far is done; a send returns after
+// that (its caller may then reuse the memory, on any stream), not after the whole build.
+void jset_input_queued(JSet &js, hipStream_t s) {
+    if (!js.read) NB6_HIP(hipEventCreateWithFlags(&js.read, hipEventDisableTiming));
+    NB6_HIP(hipEventRecord(js.read, s));
+}
+void jset_input_wait(JSet &js) { NB6_HIP(hipEventSynchronize(js.read)); }
+
+namespace {
+int stat_groups(int n) { return std::min(STATS_GROUPS, (n + 255) / 256); }
+
+// from in64 and, with groups > 0, its groups' parts in js.stat (else host.v)
+void build(JSet &js, int n, int groups, const JStat &host, hipStream_t s) {
     js.n = n;
     js.ntile = (n + JTILE - 1) / JTILE;
     if (n <= 0) return;
-    double st[7];
-    if (!box) {
-        const int groups = std::min(STATS_GROUPS, (n + 255) / 256);
-        double *part = js.stat.as<double>() + 8;
-        hipLaunchKernelGGL(stats_kernel, dim3(groups), dim3(256), 0, s, js.in64.as<double>(), n, part);
-        hipLaunchKernelGGL(stats_final_kernel, dim3(1), dim3(256), 0, s, part, groups,
-                           js.stat.as<double>());
-        NB6_HIP(hipGetLastError());
-        NB6_HIP(hipMemcpyAsync(st, js.stat.p, 7 * sizeof(double), hipMemcpyDeviceToHost, s));
-        NB6_HIP(hipStreamSynchronize(s));
-        box = st;
-        mmax = st[6];
-    }
-    js.mmax = mmax;
-    for (int d = 0; d < 6; d++) js.box[d] = box[d];
-    double sc[3];
-    for (int d = 0; d < 3; d++) {
-        const double w = box[3 + d] - box[d];
-        sc[d] = w > 0.0 ? MORTON_CELLS / (w * (1.0 + 1e-12)) : 0.0;
-    }
     unsigned long long *k0 = js.keys.as<unsigned long long>();
     unsigned long long *k1 = k0 + js.cap;
     int *v0 = js.vals.as<int>();
     int *v1 = js.perm.as<int>();
-    hipLaunchKernelGGL(morton_kernel, dim3((n + 255) / 256), dim3(256), 0, s, js.in64.as<double>(),
-                       n, box[0], box[1], box[2], sc[0], sc[1], sc[2], k0, v0);
+    double *stat = js.stat.as<double>();
+    hipLaunchKernelGGL(morton_kernel, dim3(std::min(1024, (n + 255) / 256)), dim3(256), 0, s,
+                       js.in64.as<double>(), n, stat + 8, groups, host, stat, k0, v0);
     NB6_HIP(hipGetLastError());
     size_t tb = 0;
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, n, 0, 63, s));
     void *tmp = js.sort_tmp.get(tb);
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, v0, v1, n, 0, 63, s));
-    hipLaunchKernelGGL(build_kernel, dim3((n + 255) / 256), dim3(256), 0, s, js.in64.as<double>(), n,
-                       js.perm.as<int>(), js.rec64.as<double>());
+    hipLaunchKernelGGL(tile_build_kernel, dim3(js.ntile), dim3(256), 0, s, js.in64.as<double>(), n,
+                       v1, nullptr, nullptr, nullptr, 0, js.rec64.as<double>(), js.torg.as<double>(),
+                       js.rec32.as<float4>(), js.tbox.as<float>());
     NB6_HIP(hipGetLastError());
-    jset_tiles(js, n, 1, s);
+}
+}  // namespace
+
+// in64 holds n AoS records in the caller's order; box = {lo[3], hi[3]} or nullptr
+void jset_build(JSet &js, int n, const double *box, double mmax, hipStream_t s) {
+    JStat host{};
+    int groups = 0;
+    if (n > 0 && box) {
+        for (int q = 0; q < 6; q++) host.v[q] = box[q];
+        host.v[6] = mmax;
+    } else if (n > 0) {
+        groups = stat_groups(n);
+        hipLaunchKernelGGL(aos_stats_kernel, dim3(groups), dim3(256), 0, s, nullptr, n, 0,
+                           js.in64.as<double>(), js.stat.as<double>() + 8);
+        NB6_HIP(hipGetLastError());
+    }
+    build(js, n, groups, host, s);
 }
 
-void jset_tiles(JSet &js, int n, int middle, hipStream_t s) {
-    const int nt = (n + JTILE - 1) / JTILE;
-    hipLaunchKernelGGL(origin_kernel, dim3(nt), dim3(256), 0, s, js.rec64.as<double>(), n, middle,
-                       js.torg.as<double>());
-    hipLaunchKernelGGL(rec32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, js.rec64.as<double>(),
-                       n, js.torg.as<double>(), js.rec32.as<float4>());
+void jset_build_clusters(JSet &js, int npad, const double *in, const int *sorted, const int *off,
+                         const int *padoff, int nc, hipStream_t s) {
+    js.n = npad;
+    js.ntile = npad / JTILE;
+    hipLaunchKernelGGL(tile_build_kernel, dim3(js.ntile), dim3(256), 0, s, in, npad,
+                       js.perm.as<int>(), sorted, off, padoff, nc, js.rec64.as<double>(),
+                       js.torg.as<double>(), js.rec32.as<float4>(), js.tbox.as<float>());
     NB6_HIP(hipGetLastError());
-    jset_tile_boxes(js, n, s);
 }
 
 const int *jset_sort_i(const JSet &js, int ni, int stride, const double *d_i, RegfWork &w,
                        hipStream_t s) {
-    double sc[3];
-    for (int d = 0; d < 3; d++) {
-        const double wd = js.box[3 + d] - js.box[d];
-        sc[d] = wd > 0.0 ? MORTON_CELLS / (wd * (1.0 + 1e-12)) : 0.0;
-    }
     unsigned long long *k0 =
         static_cast<unsigned long long *>(w.ikey.get((size_t)ni * 2 * sizeof(unsigned long long)));
     unsigned long long *k1 = k0 + ni;
     int *v0 = static_cast<int *>(w.ival.get((size_t)ni * 2 * sizeof(int)));
     int *v1 = v0 + ni;
     hipLaunchKernelGGL(imorton_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, d_i, stride, ni,
-                       js.box[0], js.box[1], js.box[2], sc[0], sc[1], sc[2], k0, v0);
+                       js.stat.as<double>(), k0, v0);
     NB6_HIP(hipGetLastError());
     size_t tb = 0;
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, ni, 0, 63, s));
@@ -404,12 +449,17 @@ void pack_rows(const int *list, int n, int lmax, int maxc, int *len, int *off, i
 }
 
 void jset_from_soa(JSet &js, int n, int stride, const double *d_soa, hipStream_t s) {
-    if (n > 0) {
-        hipLaunchKernelGGL(soa_to_aos_kernel, dim3((n + 255) / 256), dim3(256), 0, s, d_soa, n,
-                           stride, js.in64.as<double>());
-        NB6_HIP(hipGetLastError());
+    if (n <= 0) {
+        build(js, n, 0, JStat{}, s);
+        return;
     }
-    jset_build(js, n, nullptr, 0.0, s);
+    const int groups = stat_groups(n);
+    hipLaunchKernelGGL(aos_stats_kernel, dim3(groups), dim3(256), 0, s, d_soa, n, stride,
+                       js.in64.as<double>(), js.stat.as<double>() + 8);
+    NB6_HIP(hipGetLastError());
+    jset_input_queued(js, s);
+    build(js, n, groups, JStat{}, s);
+    jset_input_wait(js);
 }
 
 }  // namespace nb6

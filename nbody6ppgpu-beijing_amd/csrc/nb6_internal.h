@@ -77,6 +77,7 @@ constexpr int JTILE = 256;   // j-particles per tile (one tile origin each)
 //   rec32 [cap][2] float4 sorted       (x-P, y-P, z-P, m), (vx-V, vy-V, vz-V, 0)
 //   torg  [ntile][8] FP64 tile origins (Px Py Pz Vx Vy Vz 0 0)
 //   perm  [cap] int: sorted position -> caller's 0-based index
+//   stat  FP64 [7]: bounds of the positions lo[3], hi[3], maximum mass (then scratch)
 //   tbox  [ntile][16] FP32 bounds of each tile's records relative to its origin:
 //         pos lo[3], pos hi[3], vel lo[3], vel hi[3], max mass, record count, 0, 0
 //         (far massless padding records, |x| >= 1e16, are left out)
@@ -85,11 +86,9 @@ struct JSet {
     int n = 0;
     int cap = 0;
     int ntile = 0;
-    double mmax = 0.0;
-    double box[6] = {0, 0, 0, 0, 0, 0};   // lo[3], hi[3] of the positions (host copy)
+    hipEvent_t read = nullptr;   // the caller's input has been read (jset_input_queued)
     DBuf in64, rec64, rec32, torg, perm, keys, vals, stat, sort_tmp, tbox;
 };
-// per-tile bounds of rec32 (after rec32 is built): one work-group per tile
 // Work-group b of G -> position in the work order such that XCD x (work-groups are
 // dealt to the 8 XCDs round robin, b mod 8) receives a contiguous range of the work,
 // and its L2 sees one region of it at a time.
@@ -99,15 +98,18 @@ __device__ __forceinline__ int xcd_order(int b, int G) {
     return xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
 }
 
-void jset_tile_boxes(JSet &js, int n, hipStream_t s);
-// tile origins (P from the middle record, or the first: middle = 0), FP32 records,
-// tile boxes, from the sorted rec64 of n records
-void jset_tiles(JSet &js, int n, int middle, hipStream_t s);
 void jset_reserve(JSet &js, int cap);
 void jset_release(JSet &js);
 // in64 already holds n records; box = {lo x,y,z, hi x,y,z} or nullptr (computed)
 void jset_build(JSet &js, int n, const double *box, double mmax, hipStream_t s);
 void jset_from_soa(JSet &js, int n, int stride, const double *d_soa, hipStream_t s);
+// the padded layout of nc clusters (npad slots, a multiple of JTILE) from AoS records in[]:
+// sorted = compact order, off / padoff = the clusters' starts there and in the slots
+void jset_build_clusters(JSet &js, int npad, const double *in, const int *sorted, const int *off,
+                         const int *padoff, int nc, hipStream_t s);
+// a send's input is read by the work queued on s up to here / wait for that
+void jset_input_queued(JSet &js, hipStream_t s);
+void jset_input_wait(JSet &js);
 // Rows [count, entries...] of a [n][lmax] list array packed end to end on the device:
 // off[i] (n + 1 entries, off[n] = total) and pack[off[i] .. off[i + 1]) = the row's
 // 1 + count leading ints (only the count if it is negative or above maxc); len is

@@ -84,7 +84,7 @@ struct TileParams {
     int nj;
     int chunk_len;                   // multiple of the block size T and of JTILE
     int nib;                         // i-blocks of the grid (regf_tile_kernel)
-    double mmax;
+    const double *__restrict__ mmax; // maximum mass of the j-set
     double *__restrict__ part;       // [nchunk][NPART][ni]
     int *__restrict__ cnt;           // [nchunk][2][ni]: hard, soft
     int *__restrict__ hslot;         // [(chunk*ni + i) * caph + k]
@@ -119,7 +119,7 @@ struct IC {
 
 template <bool MFLAG>
 __device__ __forceinline__ ILane make_lane(const double *__restrict__ ib, int is, int i, bool ok,
-                                           double mmax, float fnear) {
+                                           const double *__restrict__ mmax, float fnear) {
     ILane L;
     const int ii = ok ? i : 0;
     L.x = ib[0 * is + ii]; L.y = ib[1 * is + ii]; L.z = ib[2 * is + ii];
@@ -134,7 +134,7 @@ __device__ __forceinline__ ILane make_lane(const double *__restrict__ ib, int is
     L.h2H = (float)hk;
     L.h2S = (float)(hk * (double)(fnear * fnear));
     L.h2L = (float)(hh * (1.0 - H_REL) * (1.0 - 12.0 * U24));
-    const double rs = MFLAG ? sqrt(hh * mmax) : sqrt(hh);
+    const double rs = MFLAG ? sqrt(hh * *mmax) : sqrt(hh);
     L.rsH = (float)(rs * (1.0 + 4.0 * U24));
     L.rsS = fnear * L.rsH;
     L.ok = ok;
@@ -2510,7 +2510,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         tp.rec64 = js.rec64.as<double>();
         tp.chunk_len = clen;
         tp.nib = bnib;
-        tp.mmax = js.mmax;
+        tp.mmax = js.stat.as<double>() + 6;
         tp.part = part; tp.cnt = cnt;
         tp.hslot = hslot; tp.caph = caph; tp.sslot = sslot; tp.caps = caps;
         tp.fnear = cfg.near;
@@ -2768,7 +2768,7 @@ int regf_items_launch(const JSet &js, int nslots, const int *imap, int stride, c
     tp.far_test = cfg.far_test;
     tp.rec64 = js.rec64.as<double>();
     tp.chunk_len = js.n;
-    tp.mmax = js.mmax;
+    tp.mmax = js.stat.as<double>() + 6;
     tp.part = part; tp.cnt = cnt;
     tp.hslot = hslot; tp.caph = caph; tp.sslot = sslot; tp.caps = caps;
     tp.fnear = cfg.near;
