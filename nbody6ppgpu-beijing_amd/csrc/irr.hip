@@ -19,6 +19,8 @@
 // (r^2 bits, index) minimum.
 #include "nb6_internal.h"
 
+#include "block_sort.h"
+
 #include <hipcub/hipcub.hpp>
 
 #include <chrono>
@@ -313,26 +315,39 @@ __global__ __launch_bounds__(256) void irr_force_kernel(
     }
 }
 
-// Morton key of each active i's record position (for the processing order)
-__global__ __launch_bounds__(256) void irr_key_kernel(int ni, const int *__restrict__ addr,
-                                                      const IrrRec *__restrict__ rec,
-                                                      const double *__restrict__ box,
-                                                      unsigned *__restrict__ key,
+// Morton keys of the active i's record positions in the j-set's box (10 bits per axis)
+struct IrrKeys {
+    const int *addr;
+    const IrrRec *rec;
+    const double *box;
+    __device__ void begin() {}
+    __device__ unsigned long long key(int w) const {
+        const IrrRec &r = rec[addr[w] - 1];
+        const double f[3] = {r.x, r.y, r.z};
+        unsigned q[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const double wd = box[3 + d] - box[d];
+            const double p = (f[d] - box[d]) * (wd > 0.0 ? 1024.0 / (wd * (1.0 + 1e-12)) : 0.0);
+            q[d] = p > 0.0 ? (p < 1023.0 ? (unsigned)p : 1023u) : 0u;
+        }
+        return spread21(q[0]) | (spread21(q[1]) << 1) | (spread21(q[2]) << 2);
+    }
+};
+// the order and the addresses in it
+struct PutIrr {
+    int *order, *oaddr;
+    const int *addr;
+    __device__ void put(int place, int w, unsigned long long) const {
+        order[place] = w;
+        oaddr[place] = addr[w];
+    }
+};
+__global__ __launch_bounds__(256) void irr_key_kernel(IrrKeys kf, int ni, unsigned *__restrict__ key,
                                                       int *__restrict__ val) {
     const int w = blockIdx.x * 256 + threadIdx.x;
     if (w >= ni) return;
-    const IrrRec &r = rec[addr[w] - 1];
-    double f[3] = {r.x, r.y, r.z};
-    for (int d = 0; d < 3; d++) {
-        const double wd = box[3 + d] - box[d];
-        f[d] = (f[d] - box[d]) * (wd > 0.0 ? 1024.0 / (wd * (1.0 + 1e-12)) : 0.0);
-    }
-    unsigned q[3];
-    for (int d = 0; d < 3; d++) q[d] = f[d] > 0.0 ? (f[d] < 1023.0 ? (unsigned)f[d] : 1023u) : 0u;
-    unsigned kk = 0;
-    for (int bit = 9; bit >= 0; bit--)
-        for (int d = 2; d >= 0; d--) kk = (kk << 1) | ((q[d] >> bit) & 1u);
-    key[w] = kk;
+    key[w] = (unsigned)kf.key(w);
     val[w] = w;
 }
 
@@ -434,12 +449,19 @@ const int *irr_order(int ni, const int *d_addr, const int **oaddr, hipStream_t s
     const JSet *js = gpunb_jset();
     *oaddr = d_addr;
     if (!g_irrcfg.sort_i || ni < 2048 || !js || js->n <= 0) return nullptr;
-    unsigned *k0 = static_cast<unsigned *>(g.d_okey.get((size_t)ni * 2 * sizeof(unsigned)));
-    unsigned *k1 = k0 + ni;
-    int *v0 = static_cast<int *>(g.d_oval.get((size_t)ni * 2 * sizeof(int)));
-    int *v1 = v0 + ni;
-    hipLaunchKernelGGL(irr_key_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, ni, d_addr,
-                       g.rec.as<IrrRec>(), js->stat.as<double>(), k0, v0);
+    unsigned long long *kb =
+        static_cast<unsigned long long *>(g.d_okey.get((size_t)ni * 2 * sizeof(unsigned long long)));
+    int *v0 = static_cast<int *>(g.d_oval.get((size_t)ni * 4 * sizeof(int)));
+    int *v1 = v0 + 2 * (size_t)ni;
+    const IrrKeys kf{d_addr, g.rec.as<IrrRec>(), js->stat.as<double>()};
+    if (ni <= BSORT_MAX) {
+        int *oa = v1 + ni;
+        bsort(kf, PutIrr{v1, oa, d_addr}, ni, kb, v0, s);
+        *oaddr = oa;
+        return v1;
+    }
+    unsigned *k0 = reinterpret_cast<unsigned *>(kb), *k1 = k0 + ni;
+    hipLaunchKernelGGL(irr_key_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, kf, ni, k0, v0);
     NB6_HIP(hipGetLastError());
     size_t tb = 0;
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, ni, 0, 30, s));

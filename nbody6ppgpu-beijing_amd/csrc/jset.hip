@@ -15,6 +15,8 @@
 // perm[s] maps a sorted position back to the caller's 0-based j index.
 #include "nb6_internal.h"
 
+#include "block_sort.h"
+
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -25,16 +27,6 @@ namespace nb6 {
 namespace {
 
 // 21 bits per axis: a cluster with escapers far out still gets a fine order in its core
-__device__ __forceinline__ unsigned long long spread21(unsigned long long a) {
-    a &= 0x1fffffull;
-    a = (a | (a << 32)) & 0x1f00000000ffffull;
-    a = (a | (a << 16)) & 0x1f0000ff0000ffull;
-    a = (a | (a << 8)) & 0x100f00f00f00f00full;
-    a = (a | (a << 4)) & 0x10c30c30c30c30c3ull;
-    a = (a | (a << 2)) & 0x1249249249249249ull;
-    return a;
-}
-
 constexpr double MORTON_CELLS = 2097152.0;   // 2^21 per axis
 
 __device__ __forceinline__ unsigned long long morton63(double x, double y, double z, double lx,
@@ -67,7 +59,7 @@ __device__ __forceinline__ void stat_add(double *v, double x, double y, double z
     }
     v[6] = fmax(v[6], m);
 }
-// bounds (lo[3], hi[3]) and maximum mass over the 256 threads, in every thread
+// bounds (lo[3], hi[3]) and maximum mass over the work-group's wavefronts, in every thread
 __device__ __forceinline__ void stat_group(double *v, double (*sh)[8]) {
 #pragma unroll
     for (int q = 0; q < 7; q++)
@@ -83,7 +75,8 @@ __device__ __forceinline__ void stat_group(double *v, double (*sh)[8]) {
 #pragma unroll
     for (int q = 0; q < 7; q++)
 #pragma unroll
-        for (int w = 0; w < 4; w++) v[q] = q < 3 ? fmin(v[q], sh[w][q]) : fmax(v[q], sh[w][q]);
+        for (int w = 0; w < (int)(blockDim.x >> 6); w++)
+            v[q] = q < 3 ? fmin(v[q], sh[w][q]) : fmax(v[q], sh[w][q]);
 }
 
 // SoA [7][stride] (x y z vx vy vz m; null: aos is there already) -> AoS [n][8] (x y z m vx vy
@@ -124,46 +117,70 @@ __device__ __forceinline__ double morton_scale(const double *box, int d) {
 // Morton keys of the AoS positions in their box, from the groups' bounds (every work-group
 // reduces them: cheaper than a launch) or, with groups = 0, from `host`; the first
 // work-group leaves the bounds and the maximum mass in stat[7]
-__global__ __launch_bounds__(256) void morton_kernel(const double *__restrict__ in, int n,
-                                                     const double *__restrict__ part, int groups,
-                                                     JStat host, double *__restrict__ stat,
+struct JKeys {
+    const double *in, *part;
+    int groups;
+    JStat host;
+    double *stat;
+    double v[7], sc[3];      // (device, from begin)
+    __device__ void begin() {
+        __shared__ double sh[16][8];
+        stat_identity(v);
+        if (groups > 0) {
+            for (int g = threadIdx.x; g < groups; g += blockDim.x)
+#pragma unroll
+                for (int q = 0; q < 7; q++) {
+                    const double u = part[g * 7 + q];
+                    v[q] = q < 3 ? fmin(v[q], u) : fmax(v[q], u);
+                }
+            stat_group(v, sh);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 7; q++) v[q] = host.v[q];
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0)
+#pragma unroll
+            for (int q = 0; q < 7; q++) stat[q] = v[q];
+#pragma unroll
+        for (int d = 0; d < 3; d++) sc[d] = morton_scale(v, d);
+    }
+    __device__ unsigned long long key(int j) const {
+        const double *r = in + (size_t)j * 8;
+        return morton63(r[0], r[1], r[2], v[0], v[1], v[2], sc[0], sc[1], sc[2]);
+    }
+};
+__global__ __launch_bounds__(256) void morton_kernel(JKeys kf, int n,
                                                      unsigned long long *__restrict__ key,
                                                      int *__restrict__ val) {
-    __shared__ double sh[4][8];
-    double v[7];
-    if (groups > 0) {
-        stat_identity(v);
-        for (int g = threadIdx.x; g < groups; g += 256)
-#pragma unroll
-            for (int q = 0; q < 7; q++) {
-                const double u = part[g * 7 + q];
-                v[q] = q < 3 ? fmin(v[q], u) : fmax(v[q], u);
-            }
-        stat_group(v, sh);
-    } else {
-#pragma unroll
-        for (int q = 0; q < 7; q++) v[q] = host.v[q];
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-#pragma unroll
-        for (int q = 0; q < 7; q++) stat[q] = v[q];
-    const double sx = morton_scale(v, 0), sy = morton_scale(v, 1), sz = morton_scale(v, 2);
+    kf.begin();
     for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
-        const double *r = in + (size_t)j * 8;
-        key[j] = morton63(r[0], r[1], r[2], v[0], v[1], v[2], sx, sy, sz);
+        key[j] = kf.key(j);
         val[j] = j;
     }
 }
 
-// Morton key of i-particle positions (SoA rows 0-2) in the j-set's box (clamped)
-__global__ __launch_bounds__(256) void imorton_kernel(const double *__restrict__ ib, int stride,
-                                                      int ni, const double *__restrict__ box,
+// Morton keys of i-particle positions (SoA rows 0-2) in the j-set's box (clamped)
+struct IKeys {
+    const double *ib;
+    int stride;
+    const double *box;
+    __device__ void begin() {}
+    __device__ unsigned long long key(int i) const {
+        return morton63(ib[i], ib[(size_t)stride + i], ib[2 * (size_t)stride + i], box[0], box[1],
+                        box[2], morton_scale(box, 0), morton_scale(box, 1), morton_scale(box, 2));
+    }
+};
+struct PutOrder {
+    int *order;
+    __device__ void put(int place, int e, unsigned long long) const { order[place] = e; }
+};
+
+__global__ __launch_bounds__(256) void imorton_kernel(IKeys kf, int ni,
                                                       unsigned long long *__restrict__ key,
                                                       int *__restrict__ val) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= ni) return;
-    key[i] = morton63(ib[i], ib[(size_t)stride + i], ib[2 * (size_t)stride + i], box[0], box[1],
-                      box[2], morton_scale(box, 0), morton_scale(box, 1), morton_scale(box, 2));
+    key[i] = kf.key(i);
     val[i] = i;
 }
 
@@ -315,7 +332,7 @@ void jset_reserve(JSet &js, int cap) {
     js.torg.get((size_t)ntile * 8 * sizeof(double));
     js.perm.get((size_t)cap * sizeof(int));
     js.keys.get((size_t)cap * 2 * sizeof(unsigned long long));
-    js.vals.get((size_t)cap * sizeof(int));
+    js.vals.get((size_t)cap * 2 * sizeof(int));
     js.stat.get((8 + 7 * STATS_GROUPS) * sizeof(double));   // stat[7], groups' parts
     js.tbox.get((size_t)ntile * TBOX * sizeof(float));
 }
@@ -350,13 +367,17 @@ void build(JSet &js, int n, int groups, const JStat &host, hipStream_t s) {
     int *v0 = js.vals.as<int>();
     int *v1 = js.perm.as<int>();
     double *stat = js.stat.as<double>();
-    hipLaunchKernelGGL(morton_kernel, dim3(std::min(1024, (n + 255) / 256)), dim3(256), 0, s,
-                       js.in64.as<double>(), n, stat + 8, groups, host, stat, k0, v0);
-    NB6_HIP(hipGetLastError());
-    size_t tb = 0;
-    NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, n, 0, 63, s));
-    void *tmp = js.sort_tmp.get(tb);
-    NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, v0, v1, n, 0, 63, s));
+    const JKeys kf{js.in64.as<double>(), stat + 8, groups, host, stat, {}, {}};
+    if (n <= BSORT_MAX) {
+        bsort(kf, PutOrder{v1}, n, k0, v0, s);
+    } else {
+        hipLaunchKernelGGL(morton_kernel, dim3(1024), dim3(256), 0, s, kf, n, k0, v0);
+        NB6_HIP(hipGetLastError());
+        size_t tb = 0;
+        NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, n, 0, 63, s));
+        void *tmp = js.sort_tmp.get(tb);
+        NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, v0, v1, n, 0, 63, s));
+    }
     hipLaunchKernelGGL(tile_build_kernel, dim3(js.ntile), dim3(256), 0, s, js.in64.as<double>(), n,
                        v1, nullptr, nullptr, nullptr, 0, js.rec64.as<double>(), js.torg.as<double>(),
                        js.rec32.as<float4>(), js.tbox.as<float>());
@@ -395,10 +416,14 @@ const int *jset_sort_i(const JSet &js, int ni, int stride, const double *d_i, Re
     unsigned long long *k0 =
         static_cast<unsigned long long *>(w.ikey.get((size_t)ni * 2 * sizeof(unsigned long long)));
     unsigned long long *k1 = k0 + ni;
-    int *v0 = static_cast<int *>(w.ival.get((size_t)ni * 2 * sizeof(int)));
-    int *v1 = v0 + ni;
-    hipLaunchKernelGGL(imorton_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, d_i, stride, ni,
-                       js.stat.as<double>(), k0, v0);
+    int *v0 = static_cast<int *>(w.ival.get((size_t)ni * 3 * sizeof(int)));
+    int *v1 = v0 + 2 * (size_t)ni;
+    const IKeys kf{d_i, stride, js.stat.as<double>()};
+    if (ni <= BSORT_MAX) {
+        bsort(kf, PutOrder{v1}, ni, k0, v0, s);
+        return v1;
+    }
+    hipLaunchKernelGGL(imorton_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, kf, ni, k0, v0);
     NB6_HIP(hipGetLastError());
     size_t tb = 0;
     NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, v0, v1, ni, 0, 63, s));
