@@ -335,6 +335,101 @@ __device__ __forceinline__ void pair_step(const TileParams &p, const IC &ck, con
     }
 }
 
+// The far loop (pair_step without the test) of one i per lane over RF_FLUSH j, written out so
+// that registers and wave priorities can be chosen.  Bound by VALU issue, at the clock that
+// the power limit leaves (2.1 GHz where the loop that the compiler made ran at 2.27).
+//
+//  * The vector register file has an even and an odd bank.  An FP32 instruction takes two
+//    cycles of its SIMD, but four if it has three register sources and all lie in one
+//    bank, or reads an SGPR (measured 0.94 against 1.79 instructions per cycle and CU).  The
+//    compiler does not look at banks: its loop had 23 such instructions among the 131 of
+//    four pairs, this one has none.
+//  * Two wavefronts of a SIMD issue side by side, each one instruction in four cycles.
+//    After a slow instruction (v_rsq_f32: eight cycles) both fall into the same half of
+//    the four cycles and take turns from then on, which leaves the SIMD half idle until
+//    something else moves them apart.  Raised priority around v_rsq_f32 does: the loop
+//    alone takes 20.9 cycles per pair, wavefront and CU in place of 24.2 (18 with every
+//    instruction at its own rate).
+//  * ds_read_b128 takes half the time of ds_read_b96 (4 cycles against 8).
+//
+// Each pair's operations, their roundings and the order of the sums are pair_step's, so the
+// sums are the same bits.  N = 2^20, ni = 2^17: 51.6e9 -> 45.0e9 CU cycles, 92.3 -> 87.8 ms.
+//
+// a: LDS byte address of the first record's position (then 16 bytes each), b: of its
+// velocity.  The next pair's two reads are in flight while a pair is evaluated; the
+// register sets A and B take the pairs in turn.  A result of v_rsq_f32 must not be read by
+// the next vector instruction; six others stand between.
+#define FAR_READ(ra, rb, o)                                                                \
+    "ds_read_b128 " ra ", %[a] offset:" o "\n"                                             \
+    "ds_read_b128 " rb ", %[b] offset:" o "\n"
+// dx dy in place of x y (even, odd), dz in Z (odd), du in v19 (odd), dv dw in place (odd,
+// even), r2 in v16, rv in v22, 1/r in v18, 1/r^2 in v20, m/r in v21, m/r^3 in v16
+#define FAR_PAIR(X, Y, Z0, M, U, V, W, Z, NEXT)                                             \
+    "s_waitcnt lgkmcnt(0)\n" NEXT                                                          \
+    "v_sub_f32 " X ", " X ", v24\n"                                                        \
+    "v_sub_f32 " Y ", " Y ", v25\n"                                                        \
+    "v_sub_f32 " Z ", " Z0 ", v26\n"                                                       \
+    "v_mul_f32 v16, " X ", " X "\n"                                                        \
+    "v_fmac_f32 v16, " Y ", " Y "\n"                                                       \
+    "v_fmac_f32 v16, " Z ", " Z "\n"                                                       \
+    "s_setprio 1\n"                                                                        \
+    "v_rsq_f32 v18, v16\n"                                                                 \
+    "v_sub_f32 v19, " U ", v27\n"                                                          \
+    "v_sub_f32 " V ", " V ", v28\n"                                                        \
+    "v_sub_f32 " W ", " W ", v29\n"                                                        \
+    "s_setprio 0\n"                                                                        \
+    "v_mul_f32 v22, " X ", v19\n"                                                          \
+    "v_fmac_f32 v22, " Y ", " V "\n"                                                       \
+    "v_fmac_f32 v22, " Z ", " W "\n"                                                       \
+    "v_mul_f32 v20, v18, v18\n"                                                            \
+    "v_fma_f32 v17, -v16, v20, 1.0\n"                                                      \
+    "v_mul_f32 v17, 0.5, v17\n"                                                            \
+    "v_fmac_f32 v18, v18, v17\n"                                                           \
+    "v_mul_f32 v20, v18, v18\n"                                                            \
+    "v_mul_f32 v21, " M ", v18\n"                                                          \
+    "v_fmac_f32 v34, " M ", v18\n"                                                         \
+    "v_mul_f32 v17, 0xc0400000, v20\n"                                                     \
+    "v_mul_f32 v16, v20, v21\n"                                                            \
+    "v_mul_f32 v22, v22, v17\n"                                                            \
+    "v_fmac_f32 v31, v16, " X "\n"                                                         \
+    "v_fmac_f32 v30, v16, " Y "\n"                                                         \
+    "v_fmac_f32 v32, v16, " Z "\n"                                                         \
+    "v_fmac_f32 v19, v22, " X "\n"                                                         \
+    "v_fmac_f32 " V ", v22, " Y "\n"                                                       \
+    "v_fmac_f32 " W ", v22, " Z "\n"                                                       \
+    "v_fmac_f32 v35, v16, v19\n"                                                           \
+    "v_fmac_f32 v36, v16, " V "\n"                                                         \
+    "v_fmac_f32 v33, v16, " W "\n"                                                         \
+    "v_fmac_f32 v37, v20, v21\n"
+#define FAR_A(NEXT) FAR_PAIR("v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", NEXT)
+#define FAR_B(NEXT) FAR_PAIR("v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", NEXT)
+#define FAR_LA(o) FAR_READ("v[0:3]", "v[4:7]", o)
+#define FAR_LB(o) FAR_READ("v[8:11]", "v[12:15]", o)
+__device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, const IC &c,
+                                         float *__restrict__ acc, float &s3) {
+    static_assert(RF_FLUSH == 64, "four rounds of 16 pairs");
+    unsigned a = (unsigned)(uintptr_t)(lds_void *)sA, b = (unsigned)(uintptr_t)(lds_void *)sB;
+    int k;
+    asm volatile(
+        "s_movk_i32 %[k], 4\n"
+        ".Lfar%=:\n" FAR_LA("0")
+        FAR_A(FAR_LB("16")) FAR_B(FAR_LA("32")) FAR_A(FAR_LB("48")) FAR_B(FAR_LA("64"))
+        FAR_A(FAR_LB("80")) FAR_B(FAR_LA("96")) FAR_A(FAR_LB("112")) FAR_B(FAR_LA("128"))
+        FAR_A(FAR_LB("144")) FAR_B(FAR_LA("160")) FAR_A(FAR_LB("176")) FAR_B(FAR_LA("192"))
+        FAR_A(FAR_LB("208")) FAR_B(FAR_LA("224")) FAR_A(FAR_LB("240")) FAR_B("")
+        "v_add_u32 %[a], 0x100, %[a]\n"
+        "v_add_u32 %[b], 0x100, %[b]\n"
+        "s_sub_i32 %[k], %[k], 1\n"
+        "s_cmp_lg_u32 %[k], 0\n"
+        "s_cbranch_scc1 .Lfar%=\n"
+        : [a] "+v"(a), [b] "+v"(b), [k] "=&s"(k), "+{v31}"(acc[0]), "+{v30}"(acc[1]),
+          "+{v32}"(acc[2]), "+{v34}"(acc[3]), "+{v35}"(acc[4]), "+{v36}"(acc[5]),
+          "+{v33}"(acc[6]), "+{v37}"(s3)
+        : "{v24}"(c.x), "{v25}"(c.y), "{v26}"(c.z), "{v27}"(c.u), "{v28}"(c.v), "{v29}"(c.w)
+        : "v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13",
+          "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "scc", "memory");
+}
+
 // FP64 partial sums and error scales of this lane's i-particles to part row `row`
 // (of the chunk's partial-sum segments), then zeroed for the next segment
 template <int T, int IPL>
@@ -435,7 +530,9 @@ __device__ __forceinline__ void tile_work(const TileParams &p, int ibase, int ie
                 }
                 allfar = __ballot(!far) == 0ull;
             }
-            if (allfar) {
+            if (allfar && IPL == 1) {
+                far_loop(&sA[buf][js0], &sB[buf][js0], c[0], a32[0], s3[0]);
+            } else if (allfar) {
 #pragma unroll 4
                 for (int jj = js0; jj < js0 + RF_FLUSH; jj++) {
                     const float4 a = sA[buf][jj], b = sB[buf][jj];
@@ -647,12 +744,7 @@ __global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
                 pair_add(q, rinv, ra.w, acc, s3);
             }
         } else {
-#pragma unroll 4
-            for (int jj = 0; jj < 64; jj++) {
-                const float4 ra = sA[w * 64 + jj], rb = sB[w * 64 + jj];
-                const PairBase q = pair_base(c, ra, rb);
-                pair_add(q, rinv_nr(q.r2), ra.w, acc, s3);
-            }
+            far_loop(&sA[w * 64], &sB[w * 64], c, acc, s3);
         }
 #pragma unroll
         for (int q = 0; q < NACC; q++) sP[w][q][lane] = acc[q];
