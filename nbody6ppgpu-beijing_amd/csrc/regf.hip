@@ -422,12 +422,171 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
         "s_sub_i32 %[k], %[k], 1\n"
         "s_cmp_lg_u32 %[k], 0\n"
         "s_cbranch_scc1 .Lfar%=\n"
-        : [a] "+v"(a), [b] "+v"(b), [k] "=&s"(k), "+{v31}"(acc[0]), "+{v30}"(acc[1]),
+        : [a] "+&v"(a), [b] "+&v"(b), [k] "=&s"(k), "+{v31}"(acc[0]), "+{v30}"(acc[1]),
           "+{v32}"(acc[2]), "+{v34}"(acc[3]), "+{v35}"(acc[4]), "+{v36}"(acc[5]),
           "+{v33}"(acc[6]), "+{v37}"(s3)
         : "{v24}"(c.x), "{v25}"(c.y), "{v26}"(c.z), "{v27}"(c.u), "{v28}"(c.v), "{v29}"(c.w)
         : "v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13",
           "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "scc", "memory");
+}
+
+// The loop with the neighbour test (pair_step) of one i per lane over the RF_FLUSH j from sorted
+// index j0 on, written out as far_loop is.  Per pair three instructions more: the cheap test
+// takes r2 - |2 dtr rv|, which is no larger than r2 + 2 dtr min(rv, 0) and needs no minimum (an
+// instruction of half the rate), and a branch to the full test where a lane passes it.  The
+// full test decides, so candidates, their order and the sums are pair_step's, bit for bit.
+// Returns the first j not done: that of a pair for which a lane has no slot left (the caller
+// goes on with pair_step, which knows overflowing rows), or j0 + RF_FLUSH.
+// Tile kernel (the loop that the compiler made, then this one): N = 100,003, ni = 6007 with
+// m_flag, where 99 % of the tiles are tested, 640 -> 564 us; N = 65,536, ni = 1024
+// (all) 100 -> 86 us; send and force of N = 2^20, ni = 2^17 (9 %) 92.8 -> 89.5 ms.
+#define NEAR_PAIR(X, Y, Z0, M, U, V, W, Z, K, NEXT, THQ, TQ, THR)                           \
+    "s_waitcnt lgkmcnt(0)\n" NEXT                                                           \
+    "v_sub_f32 " X ", " X ", v24\n"                                                         \
+    "v_sub_f32 " Y ", " Y ", v25\n"                                                         \
+    "v_sub_f32 " Z ", " Z0 ", v26\n"                                                        \
+    "v_mul_f32 v16, " X ", " X "\n"                                                         \
+    "v_fmac_f32 v16, " Y ", " Y "\n"                                                        \
+    "v_fmac_f32 v16, " Z ", " Z "\n"                                                        \
+    "v_sub_f32 v19, " U ", v27\n"                                                           \
+    "v_sub_f32 " V ", " V ", v28\n"                                                         \
+    "v_sub_f32 " W ", " W ", v29\n"                                                         \
+    "v_mul_f32 v22, " X ", v19\n"                                                           \
+    "v_fmac_f32 v22, " Y ", " V "\n"                                                        \
+    "v_fmac_f32 v22, " Z ", " W "\n"                                                        \
+    "v_fma_f32 v23, -|v39|, |v22|, v16\n"                                                   \
+    THQ                                                                                     \
+    "s_setprio 1\n"                                                                         \
+    "v_rsq_f32 v18, v16\n"                                                                  \
+    "v_cmp_lt_f32 vcc, v23, " TQ "\n"                                                       \
+    "s_setprio 0\n"                                                                         \
+    "v_mul_f32 v20, v18, v18\n"                                                             \
+    "v_fma_f32 v17, -v16, v20, 1.0\n"                                                       \
+    "v_mul_f32 v17, 0.5, v17\n"                                                             \
+    "v_fmac_f32 v18, v18, v17\n"                                                            \
+    "s_cbranch_vccz .Ls" K "_%=\n"                                                          \
+    "s_and_b64 exec, exec, vcc\n"                                                           \
+    "v_fma_f32 v54, v38, v19, " X "\n"                                                      \
+    "v_fma_f32 v55, v38, " V ", " Y "\n"                                                    \
+    "v_fma_f32 v23, v38, " W ", " Z "\n"                                                    \
+    "v_mul_f32 v54, v54, v54\n"                                                             \
+    "v_fmac_f32 v54, v55, v55\n"                                                            \
+    "v_fmac_f32 v54, v23, v23\n"                                                            \
+    "v_fmac_f32 v54, 0xb6000000, v16\n"                                                     \
+    "v_min_f32 v54, v16, v54\n"                                                             \
+    THR                                                                                     \
+    "s_or_b64 %[x], %[h], vcc\n"                                                            \
+    "s_cbranch_scc0 .Lr" K "_%=\n"                                                          \
+    "s_andn2_b64 %[f], vcc, %[h]\n"                                                         \
+    "s_add_i32 %[j], %[jb], " K "\n"                                                        \
+    "v_cmp_le_i32 vcc, %[caph], v46\n"                                                      \
+    "s_and_b64 vcc, vcc, %[h]\n"                                                            \
+    "s_cbranch_scc1 .Lx_%=\n"                                                               \
+    "v_cmp_le_i32 vcc, %[lim], v47\n"                                                       \
+    "s_and_b64 vcc, vcc, %[f]\n"                                                            \
+    "s_cbranch_scc1 .Lx_%=\n"                                                               \
+    "v_mov_b32 v23, %[j]\n"                                                                 \
+    "s_mov_b64 exec, %[h]\n"                                                                \
+    "s_cbranch_execz .Lf" K "_%=\n"                                                         \
+    "v_mad_u64_u32 v[54:55], vcc, v46, 4, v[48:49]\n"                                       \
+    "global_store_dword v[54:55], v23, off\n"                                               \
+    "v_add_u32 v46, 1, v46\n"                                                               \
+    ".Lf" K "_%=:\n"                                                                        \
+    "s_mov_b64 exec, %[f]\n"                                                                \
+    "s_cbranch_execz .Lh" K "_%=\n"                                                         \
+    "v_mad_u64_u32 v[54:55], vcc, v47, 4, v[50:51]\n"                                       \
+    "global_store_dword v[54:55], v23, off\n"                                               \
+    "v_add_u32 v47, 1, v47\n"                                                               \
+    ".Lh" K "_%=:\n"                                                                        \
+    "s_mov_b64 exec, %[x]\n"                                                                \
+    "v_mov_b32 v18, 0\n"                                                                    \
+    ".Lr" K "_%=:\n"                                                                        \
+    "s_mov_b64 exec, -1\n"                                                                  \
+    ".Ls" K "_%=:\n"                                                                        \
+    "v_mul_f32 v20, v18, v18\n"                                                             \
+    "v_mul_f32 v21, " M ", v18\n"                                                           \
+    "v_fmac_f32 v34, " M ", v18\n"                                                          \
+    "v_mul_f32 v17, 0xc0400000, v20\n"                                                      \
+    "v_mul_f32 v16, v20, v21\n"                                                             \
+    "v_mul_f32 v22, v22, v17\n"                                                             \
+    "v_fmac_f32 v31, v16, " X "\n"                                                          \
+    "v_fmac_f32 v30, v16, " Y "\n"                                                          \
+    "v_fmac_f32 v32, v16, " Z "\n"                                                          \
+    "v_fmac_f32 v19, v22, " X "\n"                                                          \
+    "v_fmac_f32 " V ", v22, " Y "\n"                                                        \
+    "v_fmac_f32 " W ", v22, " Z "\n"                                                        \
+    "v_fmac_f32 v35, v16, v19\n"                                                            \
+    "v_fmac_f32 v36, v16, " V "\n"                                                          \
+    "v_fmac_f32 v33, v16, " W "\n"                                                          \
+    "v_fmac_f32 v37, v20, v21\n"
+#define NEAR_A(K, NEXT, THQ, TQ, THR)                                                       \
+    NEAR_PAIR("v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", K, NEXT, THQ("v3"), TQ, THR("v3"))
+#define NEAR_B(K, NEXT, THQ, TQ, THR)                                                       \
+    NEAR_PAIR("v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", K, NEXT, THQ("v11"), TQ, \
+              THR("v11"))
+#define NEAR_LOOP(THQ, TQ, THR)                                                             \
+    ".Ln%=:\n" FAR_LA("0")                                                                  \
+    NEAR_A("0", FAR_LB("16"), THQ, TQ, THR)                                                 \
+    NEAR_B("1", FAR_LA("32"), THQ, TQ, THR)                                                 \
+    NEAR_A("2", FAR_LB("48"), THQ, TQ, THR)                                                 \
+    NEAR_B("3", FAR_LA("64"), THQ, TQ, THR)                                                 \
+    NEAR_A("4", FAR_LB("80"), THQ, TQ, THR)                                                 \
+    NEAR_B("5", FAR_LA("96"), THQ, TQ, THR)                                                 \
+    NEAR_A("6", FAR_LB("112"), THQ, TQ, THR)                                                \
+    NEAR_B("7", "", THQ, TQ, THR)                                                           \
+    "v_add_u32 %[a], 0x80, %[a]\n"                                                          \
+    "v_add_u32 %[b], 0x80, %[b]\n"                                                          \
+    "s_add_i32 %[jb], %[jb], 8\n"                                                           \
+    "s_cmp_lg_u32 %[jb], %[je]\n"                                                           \
+    "s_cbranch_scc1 .Ln%=\n"                                                                \
+    "s_mov_b32 %[j], %[jb]\n"                                                               \
+    ".Lx_%=:\n"                                                                             \
+    "s_waitcnt lgkmcnt(0)\n"                                                                \
+    "s_mov_b64 exec, -1\n"
+// thresholds of the cheap test, and the full test's (hard ones to %[h], soft or hard to vcc)
+#define NEAR_TQ0(M) ""
+#define NEAR_TQ1(M) "v_fma_f32 v54, " M ", v40, v43\n"
+#define NEAR_TH0(M) "v_cmp_lt_f32 %[h], v54, v41\nv_cmp_lt_f32 vcc, v54, v42\n"
+#define NEAR_TH1(M)                                                                        \
+    "v_fma_f32 v55, " M ", v41, v44\n"                                                     \
+    "v_cmp_lt_f32 %[h], v54, v55\n"                                                        \
+    "v_fma_f32 v55, " M ", v42, v45\n"                                                     \
+    "v_cmp_lt_f32 vcc, v54, v55\n"
+#define NEAR_CLOBBERS                                                                      \
+    "v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13", \
+        "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "v23", "v54", "v55", \
+        "vcc", "scc", "memory"
+template <bool MFLAG>
+__device__ __forceinline__ int near_loop(const float4 *sA, const float4 *sB, const IC &c, int j0,
+                                         int caph, int lim, int &nhk, int &nsk, int *hpk, int *spk,
+                                         float *__restrict__ acc, float &s3) {
+    unsigned a = (unsigned)(uintptr_t)(lds_void *)sA, b = (unsigned)(uintptr_t)(lds_void *)sB;
+    unsigned long long mh, mf, mx;
+    int j, jb = j0;
+    if (MFLAG)
+        asm volatile(NEAR_LOOP(NEAR_TQ1, "v54", NEAR_TH1)
+                     : [a] "+&v"(a), [b] "+&v"(b), [jb] "+&s"(jb), [j] "=&s"(j), [h] "=&s"(mh),
+                       [f] "=&s"(mf), [x] "=&s"(mx), "+{v46}"(nhk), "+{v47}"(nsk),
+                       "+{v31}"(acc[0]), "+{v30}"(acc[1]), "+{v32}"(acc[2]), "+{v34}"(acc[3]),
+                       "+{v35}"(acc[4]), "+{v36}"(acc[5]), "+{v33}"(acc[6]), "+{v37}"(s3)
+                     : "{v24}"(c.x), "{v25}"(c.y), "{v26}"(c.z), "{v27}"(c.u), "{v28}"(c.v),
+                       "{v29}"(c.w), "{v38}"(c.dt1), "{v39}"(c.dt2), "{v40}"(c.hQ), "{v41}"(c.hH),
+                       "{v42}"(c.hS), "{v43}"(c.dQ), "{v44}"(c.dH), "{v45}"(c.dS),
+                       "{v[48:49]}"(hpk), "{v[50:51]}"(spk),
+                       [caph] "s"(caph), [lim] "s"(lim), [je] "s"(j0 + RF_FLUSH)
+                     : NEAR_CLOBBERS);
+    else
+        asm volatile(NEAR_LOOP(NEAR_TQ0, "v40", NEAR_TH0)
+                     : [a] "+&v"(a), [b] "+&v"(b), [jb] "+&s"(jb), [j] "=&s"(j), [h] "=&s"(mh),
+                       [f] "=&s"(mf), [x] "=&s"(mx), "+{v46}"(nhk), "+{v47}"(nsk),
+                       "+{v31}"(acc[0]), "+{v30}"(acc[1]), "+{v32}"(acc[2]), "+{v34}"(acc[3]),
+                       "+{v35}"(acc[4]), "+{v36}"(acc[5]), "+{v33}"(acc[6]), "+{v37}"(s3)
+                     : "{v24}"(c.x), "{v25}"(c.y), "{v26}"(c.z), "{v27}"(c.u), "{v28}"(c.v),
+                       "{v29}"(c.w), "{v38}"(c.dt1), "{v39}"(c.dt2), "{v40}"(c.hQ), "{v41}"(c.hH),
+                       "{v42}"(c.hS), "{v[48:49]}"(hpk), "{v[50:51]}"(spk),
+                       [caph] "s"(caph), [lim] "s"(lim), [je] "s"(j0 + RF_FLUSH)
+                     : NEAR_CLOBBERS);
+    return j;
 }
 
 // FP64 partial sums and error scales of this lane's i-particles to part row `row`
@@ -541,6 +700,16 @@ __device__ __forceinline__ void tile_work(const TileParams &p, int ibase, int ie
                         pair_step<MFLAG, false>(p, c[k], a, b, jt + jj, j1, nh[k], ns[k], hp[k],
                                                 sp[k], a32[k], s3[k]);
                 }
+            } else if (IPL == 1) {
+                int js = js0;
+                if (jt + js0 + RF_FLUSH <= j1)
+                    js = near_loop<MFLAG>(&sA[buf][js0], &sB[buf][js0], c[0], jt + js0, p.caph,
+                                          p.caps - BAND_SLOTS, nh[0], ns[0], hp[0], sp[0], a32[0],
+                                          s3[0]) - jt;
+#pragma unroll 1
+                for (int jj = js; jj < js0 + RF_FLUSH; jj++)
+                    pair_step<MFLAG, true>(p, c[0], sA[buf][jj], sB[buf][jj], jt + jj, j1, nh[0],
+                                           ns[0], hp[0], sp[0], a32[0], s3[0]);
             } else {
 #pragma unroll 2
                 for (int jj = js0; jj < js0 + RF_FLUSH; jj++) {
@@ -783,8 +952,11 @@ __global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
 
 // Persistent form for a batch of independent clusters: each work-group takes the
 // next work item from a queue (items are ordered longest first) until none is left.
+// Four wavefronts per SIMD: a cluster's longest items last nearly as long as the launch, and
+// each takes the shorter the fewer share its SIMD (64 clusters of 1024-16384: 3.86 ms
+// against 4.21 with five and 4.56 with six).
 template <int T, int IPL, bool MFLAG>
-__global__ __launch_bounds__(T, (regf_waves<T, IPL>())) void regf_items_kernel(TileParams p,
+__global__ __launch_bounds__(T, IPL == 1 ? 4 : 2) void regf_items_kernel(TileParams p,
                                                        const int4 *__restrict__ items,
                                                        int nitems, int *__restrict__ queue) {
     __shared__ float4 sA[2][T];
