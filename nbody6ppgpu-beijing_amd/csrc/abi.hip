@@ -282,7 +282,7 @@ void gpunb_send_(int *nj, double mj[], double xj[][3], double vj[][3]) {
     // AoS records (x y z m vx vy vz 0) in the caller's order, plus box, max mass and a
     // NaN check, in one pass spread over a few threads (one range each)
     double *h = static_cast<double *>(g.hj.get((size_t)8 * std::max(n, 1) * sizeof(double)));
-    const int nt = n > 65536 ? std::max(1, std::min(8, (int)std::thread::hardware_concurrency())) : 1;
+    const int nt = host_threads(n * 1.9e-3);
     double box[6];
     double mmax = 0.0;
     if (!pack_j_records(n, nt, mj, xj, vj, h, box, &mmax)) {
@@ -341,6 +341,9 @@ void gpunb_regf_(int *ni_, double h2[], double dtr[], double xi[][3], double vi[
     regf_finish(g, ni, di, lmax, nnbmax, *m_flag, acc, jrk, pot, list, s, t0);
 }
 
+// host time of one row's results (seven numbers and about 80 list entries), nanoseconds
+constexpr double ROW_NS = 60.0;
+
 // regf on a staged device i-block, results copied into the caller's arrays
 static void regf_finish(Gpunb &g, int ni, const double *di, int lmax, int nnbmax, int m_flag,
                         double acc[][3], double jrk[][3], double pot[], int *list, hipStream_t s,
@@ -379,7 +382,7 @@ static void regf_finish(Gpunb &g, int ni, const double *di, int lmax, int nnbmax
                 std::memcpy(list + (size_t)i * lmax, hp + hoff[i],
                             (size_t)(hoff[i + 1] - hoff[i]) * sizeof(int));
             }
-        });
+        }, ROW_NS);
         const double t2 = wtime();
         g.time_grav += t1 - t0;
         g.time_reduce += t2 - t1;
@@ -404,7 +407,7 @@ static void regf_finish(Gpunb &g, int ni, const double *di, int lmax, int nnbmax
             dst[0] = c;
             if (c > 0 && c <= nnbeff) std::memcpy(dst + 1, src + 1, (size_t)c * sizeof(int));
         }
-    });
+    }, ROW_NS);
     const double t2 = wtime();
     g.time_grav += t1 - t0;
     g.time_reduce += t2 - t1;

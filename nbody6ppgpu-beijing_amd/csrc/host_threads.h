@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <thread>
 #include <vector>
 
@@ -35,11 +36,19 @@ inline void run_ranges(int nt, int n, F f) {
     for (auto &x : th) x.join();
 }
 
-// A host loop over [0, n) in ranges f(a, b): up to 8 threads above 4,096 items.
+// Threads for host work that takes `us` microseconds on one: starting one and waiting for it
+// costs about 15 us, so us / nt + 15 nt is least at nt = sqrt(us / 15); at most 8.  (With
+// 8 threads from 4,097 items on, packing 10,007 particles took 140 us, and 10 on one thread;
+// 65,536 j records take 122 us on one, 85 on two, 72 on four, 140 on eight.)
+inline int host_threads(double us) {
+    const int hw = std::max(1, (int)std::thread::hardware_concurrency());
+    return std::max(1, std::min({8, hw, (int)std::sqrt(us / 15.0)}));
+}
+
+// A host loop over [0, n) in ranges f(a, b), an item of which takes about `ns` nanoseconds.
 template <class F>
-inline void par_for(int n, F f) {
-    const int nt = n > 4096 ? std::min(8, (int)std::thread::hardware_concurrency()) : 1;
-    run_ranges(nt, n, [&](int, int a, int b) { f(a, b); });
+inline void par_for(int n, F f, double ns = 2.0) {
+    run_ranges(host_threads(n * ns * 1e-3), n, [&](int, int a, int b) { f(a, b); });
 }
 
 // gpunb_send_'s host pass: AoS records (x y z m vx vy vz 0) of the caller's j
