@@ -351,11 +351,11 @@ static void regf_finish(Gpunb &g, int ni, const double *di, int lmax, int nnbmax
     double *dout = static_cast<double *>(g.dout.get((size_t)7 * ni * sizeof(double)));
     int *dlist = static_cast<int *>(g.dlist.get((size_t)ni * lmax * sizeof(int)));
     if (regf_launch(g.js, ni, ni, di, lmax, nnbmax, m_flag, dout, dlist, s) != OK) return;
-    double *ho = static_cast<double *>(g.hout.get((size_t)7 * ni * sizeof(double)));
-    NB6_HIP(hipMemcpyAsync(ho, dout, (size_t)7 * ni * sizeof(double), hipMemcpyDeviceToHost, s));
+    double *ho = static_cast<double *>(g.hout.get((size_t)8 * ni * sizeof(double)));
     const int nnbeff = std::max(0, std::min(nnbmax, lmax - 1));
     const size_t full = (size_t)ni * lmax * sizeof(int);
     if (full > ((size_t)2 << 20)) {
+        NB6_HIP(hipMemcpyAsync(ho, dout, (size_t)7 * ni * sizeof(double), hipMemcpyDeviceToHost, s));
         // large blocks: only the rows' used part crosses PCIe (about nnb + 1 of lmax ints
         // per row), packed on the device and spread into the caller's rows here
         int *len = static_cast<int *>(g.dlen.get((size_t)(ni + 1) * sizeof(int)));
@@ -389,18 +389,15 @@ static void regf_finish(Gpunb &g, int ni, const double *di, int lmax, int nnbmax
         return;
     }
     int *hl = static_cast<int *>(g.hlist.get(full));
-    NB6_HIP(hipMemcpyAsync(hl, dlist, full, hipMemcpyDeviceToHost, s));
+    deliver_rows(dout, dlist, ni, lmax, nnbeff, ho, hl, s);
     NB6_HIP(hipStreamSynchronize(s));
     const double t1 = wtime();
     par_for(ni, [&](int a, int b) {
         for (int i = a; i < b; i++) {
-            acc[i][0] = ho[0 * (size_t)ni + i];
-            acc[i][1] = ho[1 * (size_t)ni + i];
-            acc[i][2] = ho[2 * (size_t)ni + i];
-            jrk[i][0] = ho[3 * (size_t)ni + i];
-            jrk[i][1] = ho[4 * (size_t)ni + i];
-            jrk[i][2] = ho[5 * (size_t)ni + i];
-            pot[i] = ho[6 * (size_t)ni + i];
+            const double *o = ho + (size_t)8 * i;
+            acc[i][0] = o[0]; acc[i][1] = o[1]; acc[i][2] = o[2];
+            jrk[i][0] = o[3]; jrk[i][1] = o[4]; jrk[i][2] = o[5];
+            pot[i] = o[6];
             const int *src = hl + (size_t)i * lmax;
             int *dst = list + (size_t)i * lmax;
             const int c = src[0];

@@ -114,6 +114,8 @@ void jset_input_wait(JSet &js);
 // off[i] (n + 1 entries, off[n] = total) and pack[off[i] .. off[i + 1]) = the row's
 // 1 + count leading ints (only the count if it is negative or above maxc); len is
 // n + 1 ints of scratch (jset.hip).
+void deliver_rows(const double *res, const int *list, int ni, int lmax, int nnbmax, double *out,
+                  int *rows, hipStream_t s);
 void pack_rows(const int *list, int n, int lmax, int maxc, int *len, int *off, int *pack,
                DBuf &tmp, hipStream_t s);
 

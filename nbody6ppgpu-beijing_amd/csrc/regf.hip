@@ -94,7 +94,15 @@ struct TileParams {
     float fnear;                     // near field: r < fnear RS (soft candidates)
     int nseg_c;                      // partial-sum segments per chunk (part rows chunk * nseg_c
     int seg_tiles;                   // + s), each seg_tiles T-tiles long (0: the whole chunk)
+    int *__restrict__ zero;          // counters of the FP64 pass that the first work-group clears
+    int nzero;
 };
+
+// clears p.zero, for the kernels that follow (a launch of its own cost 4 us)
+__device__ __forceinline__ void clear_counters(const TileParams &p) {
+    if (p.zero && blockIdx.x == 0)
+        for (int k = threadIdx.x; k < p.nzero; k += blockDim.x) p.zero[k] = 0;
+}
 
 // per-lane constants that do not depend on the tile
 struct ILane {
@@ -778,6 +786,7 @@ __global__ __launch_bounds__(T, (regf_waves<T, IPL>())) void regf_tile_kernel(Ti
     __shared__ float4 sB[2][T];   // vx', vy', vz', 0
     // (chunk, i-block) items chunk-major, each XCD taking a contiguous run: the
     // work-groups resident on one XCD stream the same j-chunk through its L2
+    clear_counters(p);
     const int w = xcd_order(blockIdx.x, gridDim.x);
     const int chunk = w / p.nib;
     const int ib = w - chunk * p.nib;
@@ -828,6 +837,7 @@ __global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
     __shared__ float4 sA[JTILE], sB[JTILE];
     __shared__ PieceMask sM[4][64];
     __shared__ float sP[4][8][64];
+    clear_counters(p);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int b = xcd_order(blockIdx.x, gridDim.x);
     const int chunk = b / p.nib;
@@ -2736,8 +2746,6 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     if (refine) {
         nfix = ctr;
         g_nfix = ctr;
-        hipLaunchKernelGGL(zero_ints_kernel, dim3((6 + nseg + 255) / 256), dim3(256), 0, s, ctr,
-                           6 + nseg);
     }
     g_last_refine = refine;
 
@@ -2780,6 +2788,8 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         tp.fnear = cfg.near;
         tp.nseg_c = P;
         tp.seg_tiles = P > 1 ? seglen / T : 0;
+        tp.zero = b0 == 0 ? ctr : nullptr;   // (null without the FP64 pass)
+        tp.nzero = 6 + nseg;
         if (timed && b0 == 0) t1.start(s);
         if (small) {
             tp.nib = (nb + 63) / 64;
