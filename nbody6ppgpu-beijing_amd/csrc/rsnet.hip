@@ -24,6 +24,8 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "block_sort.h"
+
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -129,30 +131,33 @@ struct GradLds {
     float dy[GB];
 };
 
-// 64 x 64 x 64 products of the hidden layer on the matrix cores, rows 16 mt .. 16 mt + 15
-// by one wavefront: C[m][n] = sum_k A(m, k) B(k, n), A and B read through the callables
+// 64 x 64 x 64 products of the hidden layer on the matrix cores, NT blocks of 16 x 16 by
+// wavefront w: rows 16 mt .. 16 mt + 15, columns from 16 n0 on: C[m][n] = sum_k A(m, k) B(k, n), A and B read through the callables
 // (LDS), each element of C handed to out(m, n, c).  v_mfma_f32_16x16x4f32 (FP32 in, FP32
 // accumulate): lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] of a 16 x 4 and
 // a 4 x 16 block, and holds C[4 (l / 16) + i][l % 16], i = 0..3, of the 16 x 16 block.
 typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int GW = 8;
 template <class FA, class FB, class FO>
-__device__ __forceinline__ void gemm64(FA a, FB b, FO out, int lane, int mt) {
+__device__ __forceinline__ void gemm64(FA a, FB b, FO out, int lane, int w) {
+    constexpr int NT = 16 / GW;
     const int r = lane & 15, q = lane >> 4;
-    v4f acc[4];
+    const int mt = w * NT / 4, n0 = w * NT % 4;
+    v4f acc[NT];
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) acc[nt] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; nt++) acc[nt] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int kb = 0; kb < NH; kb += 4) {
         const float av = a(mt * 16 + r, kb + q);
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++)
-            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b(kb + q, nt * 16 + r), acc[nt], 0,
+        for (int nt = 0; nt < NT; nt++)
+            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b(kb + q, (n0 + nt) * 16 + r), acc[nt], 0,
                                                            0, 0);
     }
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
+    for (int nt = 0; nt < NT; nt++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) out(mt * 16 + q * 4 + i, nt * 16 + r, acc[nt][i]);
+        for (int i = 0; i < 4; i++) out(mt * 16 + q * 4 + i, (n0 + nt) * 16 + r, acc[nt][i]);
     }
 }
 
@@ -161,13 +166,13 @@ __device__ __forceinline__ void gemm64(FA a, FB b, FO out, int lane, int mt) {
 // GW wavefronts: the 8 -> 64 layer and the gradients of W1, b1, W3, b3 on the VALU, the
 // three 64 x 64 products of the hidden layer (forward, dW2, back-propagated delta) on
 // the matrix cores.  Bound by the latency of its chain of short LDS passes (a batch of
-// 8,192 is only 128 work-groups), so each pass is dealt to four wavefronts: wavefront w
-// takes rows 16 w .. of every product and outputs 16 w .. of the layer-1 loop, each sum
+// 8,192 is only 128 work-groups), so each pass is dealt to GW wavefronts: wavefront w takes
+// two of the 16 blocks of every product and outputs 8 w .. of the layer-1 loop, each sum
 // in the order that one wavefront would take it (same bits).  Batch of 8,192: 49.8 us
 // with one wavefront per work-group, 19.5 us with four, 15.6 us with the weights' loads
-// issued together (load_weights).
-constexpr int GW = 4;
-static_assert(GW * 16 == NH && GW * 16 == GB, "one 16-row tile per wavefront");
+// issued together (load_weights), 14.7 us with eight wavefronts.
+static_assert(NH == 64 && GB == 64 && NF == GW, "16 blocks of a product, one feature per wavefront");
+constexpr int NHW = NH / GW;         // outputs of a wavefront in the VALU passes
 __global__ __launch_bounds__(64 * GW) void rsnet_grad_kernel(
     int n, const float *__restrict__ feat, const float *__restrict__ tgt,
     const int *__restrict__ idx, int base, int fstride, const uint16_t *__restrict__ wbf,
@@ -185,10 +190,10 @@ __global__ __launch_bounds__(64 * GW) void rsnet_grad_kernel(
         for (int f = 0; f < NF; f++) x[f] = 0.f;
     load_weights<64 * GW>(L.w, wbf);
     __syncthreads();
-    // layer 1 (VALU): 16 of h1 of this lane's sample into LDS
+    // layer 1 (VALU): NHW of h1 of this lane's sample into LDS
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-        const int k = w * 16 + q;
+    for (int q = 0; q < NHW; q++) {
+        const int k = w * NHW + q;
         float z = L.w.b1[k];
 #pragma unroll
         for (int f = 0; f < NF; f++) z = fmaf(L.w.w1[k * NF + f], x[f], z);
@@ -236,8 +241,8 @@ __global__ __launch_bounds__(64 * GW) void rsnet_grad_kernel(
     __syncthreads();
     // delta2 = dy w3 [h2 > 0], in place of h2
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-        const int o = w * 16 + q;
+    for (int q = 0; q < NHW; q++) {
+        const int o = w * NHW + q;
         const float h2 = L.d2[t][o];
         L.d2[t][o] = h2 > 0.f ? dy * L.w.w3[o] : 0.f;
     }
@@ -259,19 +264,17 @@ __global__ __launch_bounds__(64 * GW) void rsnet_grad_kernel(
            [&](int o, int k) { return L.w.w2[o * (NH + 1) + k]; },
            [&](int m, int k, float v) { L.h1[m][k] = L.h1[m][k] > 0.f ? v : 0.f; }, t, w);
     __syncthreads();
-    // W1 (row k = t; wavefront w: features 2 w, 2 w + 1), b1
+    // W1 (row k = t; wavefront w: feature w), b1
     {
         const int k = t;
-        float a0 = 0.f, a1 = 0.f, gb = 0.f;
+        float a0 = 0.f, gb = 0.f;
 #pragma unroll 16
         for (int q = 0; q < GB; q++) {
             const float d = L.h1[q][k];
             gb += d;
-            a0 = fmaf(d, L.x[q][2 * w], a0);
-            a1 = fmaf(d, L.x[q][2 * w + 1], a1);
+            a0 = fmaf(d, L.x[q][w], a0);
         }
-        P[OFF_W1 + k * NF + 2 * w] = a0;
-        P[OFF_W1 + k * NF + 2 * w + 1] = a1;
+        P[OFF_W1 + k * NF + w] = a0;
         if (w == 0) P[OFF_B1 + k] = gb;
     }
 }
@@ -356,16 +359,27 @@ __global__ __launch_bounds__(256) void rsnet_sum_kernel(const float *__restrict_
 }
 
 // epoch shuffle: a random 32-bit key per sample (SplitMix64 of seed and index), sorted
-__global__ __launch_bounds__(256) void rsnet_keys_kernel(int n, unsigned long long seed,
+struct ShuffleKeys {
+    unsigned long long seed;
+    __device__ void begin() const {}
+    __device__ unsigned long long key(int k) const {
+        unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (unsigned long long)(k + 1);
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+        z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+        z ^= z >> 31;
+        return z >> 32;
+    }
+};
+struct PutPerm {
+    int *perm;
+    __device__ void put(int place, int e, unsigned long long) const { perm[place] = e; }
+};
+__global__ __launch_bounds__(256) void rsnet_keys_kernel(ShuffleKeys kf, int n,
                                                          unsigned *__restrict__ key,
                                                          int *__restrict__ val) {
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= n) return;
-    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (unsigned long long)(k + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    key[k] = (unsigned)(z >> 32);
+    key[k] = (unsigned)kf.key(k);
     val[k] = k;
 }
 
@@ -761,16 +775,26 @@ int rsnet_train_epoch(int n, const float *d_feat, const float *d_t, int batch, f
         return E_ARG;
     }
     NetState &g = g_net;
-    unsigned *key = static_cast<unsigned *>(g.keys.get((size_t)n * sizeof(unsigned)));
-    unsigned *skey = static_cast<unsigned *>(g.skeys.get((size_t)n * sizeof(unsigned)));
-    int *val = static_cast<int *>(g.vals.get((size_t)n * sizeof(int)));
     int *perm = static_cast<int *>(g.perm.get((size_t)n * sizeof(int)));
-    hipLaunchKernelGGL(rsnet_keys_kernel, dim3((n + 255) / 256), dim3(256), 0, s, n, seed, key, val);
-    NB6_HIP(hipGetLastError());
-    size_t tb = 0;
-    NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, key, skey, val, perm, n, 0, 32, s));
-    void *tmp = g.sort_tmp.get(tb);
-    NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, skey, val, perm, n, 0, 32, s));
+    const ShuffleKeys kf{seed};
+    if (n <= BSORT_MAX) {
+        // (the order of the library's sort, which takes eight launches; an epoch of 131,072
+        // samples in batches of 8,192: 490 us with it, 472 so)
+        unsigned long long *key = static_cast<unsigned long long *>(
+            g.keys.get((size_t)n * 2 * sizeof(unsigned long long)));
+        int *val = static_cast<int *>(g.vals.get((size_t)n * 2 * sizeof(int)));
+        bsort(kf, PutPerm{perm}, n, key, val, s);
+    } else {
+        unsigned *key = static_cast<unsigned *>(g.keys.get((size_t)n * sizeof(unsigned)));
+        unsigned *skey = static_cast<unsigned *>(g.skeys.get((size_t)n * sizeof(unsigned)));
+        int *val = static_cast<int *>(g.vals.get((size_t)n * sizeof(int)));
+        hipLaunchKernelGGL(rsnet_keys_kernel, dim3((n + 255) / 256), dim3(256), 0, s, kf, n, key, val);
+        NB6_HIP(hipGetLastError());
+        size_t tb = 0;
+        NB6_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, key, skey, val, perm, n, 0, 32, s));
+        void *tmp = g.sort_tmp.get(tb);
+        NB6_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, skey, val, perm, n, 0, 32, s));
+    }
     double *lacc = static_cast<double *>(g.lacc.get(sizeof(double)));
     hipLaunchKernelGGL(rsnet_zero_kernel, dim3(1), dim3(1), 0, s, lacc);
     const int nb = n / batch;
