@@ -1438,27 +1438,30 @@ __device__ __forceinline__ void wave_lds_sync() {
 // non-neighbour candidate's force is added to s.  SHARED: several wavefronts fill one
 // row, taking buffer positions from *nshared; otherwise this wavefront's nnb counts them.
 // The candidates of 64 chunks form one list (per chunk the hard slots, then the soft
-// ones), taken 64 at a time, one per lane: the slot entries of the next 64 are read while
-// the records of the current ones are fetched, and chunks with a few candidates each (or
-// a massive star each, with m_flag) cost no pass of their own.  Bound by FP64 issue
-// (about 55 % of the time) and by the latency of the gathers, which the number of resident
-// wavefronts hides: fetching 64 records ahead in a second LDS set left 16 wavefronts per CU
-// in place of 24 and took 2.41 ms where this takes 1.87 (64 clusters, 381,067 rows; 2.39
-// with a pass per chunk and every lane reading its own record).  N = 65,536, ni = N:
-// 1.28 -> 0.70 ms; N = 100,003, ni = 6007 with m_flag, whose massive stars lie in every
-// chunk: 0.56 -> 0.23 ms; N = 2^20, ni = 2^17: 2.06 -> 1.57 ms.  Listing all hard candidates
-// before all soft ones, so that most passes need no neighbour test, gained 1 % there and
-// lost 3 % on many chunks.
+// ones), taken 64 at a time, one per lane; chunks with a few candidates each (or a massive
+// star each, with m_flag) cost no pass of their own.  Bound by FP64 issue and by the latency
+// of the gathers: a pass waited for its records, then for the slot entries of the next
+// one, and computed after both; now it computes while both are under way (its own records
+// are in registers, so one set of them in LDS is enough and 24 wavefronts fit on a CU).
+// Finalize: 64 clusters (381,067 rows) 1.84 -> 1.41 ms, N = ni = 65,536 716 -> 645 us; N = 100,003,
+// ni = 6007 with m_flag 233 -> 215 us; N = 50,021, ni = 257 35.7 -> 34.2 us.
+// Listing all hard candidates before all soft ones, so that most passes need no
+// neighbour test, gained 1 % there and lost 3 % on many chunks.
+// cnt0: fin_counts of the first 64 chunks, which the callers load before all else.
+__device__ __forceinline__ int2 fin_counts(const FinParams &f, int i, int c) {
+    if (c >= f.nchunk) return make_int2(0, 0);
+    return make_int2(f.cnt[((size_t)c * 2 + 0) * f.ni + i], f.cnt[((size_t)c * 2 + 1) * f.ni + i]);
+}
 template <bool MFLAG, bool SHARED>
 __device__ __forceinline__ void fin_candidates(const FinParams &f, const IF64 &I, int i, int jb,
                                                int c0, int cstep, int lane, double *s, int *buf,
-                                               int cap, FinStage &st, int *nshared, int &nnb,
-                                               int &dropped, int &unres, bool &dropped_any) {
+                                               int cap, FinStage &st, int *nshared, int2 cnt0,
+                                               int &nnb, int &dropped, int &unres,
+                                               bool &dropped_any) {
     enum { HARD, SOFT, BAND, NONE };
     for (int cg = 0; c0 + cstep * cg < f.nchunk; cg += 64) {
-        const int c = c0 + cstep * (cg + lane);
-        const int nh = c < f.nchunk ? f.cnt[((size_t)c * 2 + 0) * f.ni + i] : 0;
-        const int ns = c < f.nchunk ? f.cnt[((size_t)c * 2 + 1) * f.ni + i] : 0;
+        const int2 hs = cg == 0 ? cnt0 : fin_counts(f, i, c0 + cstep * (cg + lane));
+        const int nh = hs.x, ns = hs.y;
         const int over = wave_sum_i(nh > f.caph ? nh - f.caph : 0);
         dropped += over;
         dropped_any = dropped_any || over > 0;
@@ -1470,10 +1473,11 @@ __device__ __forceinline__ void fin_candidates(const FinParams &f, const IF64 &I
         wave_lds_sync();                 // the last group's reads of pre are done
         st.pre[lane] = make_int2(end - nhc - nsr, nhc);
         wave_lds_sync();
-        // candidate e of the list: its slot entry and kind
-        auto entry = [&](int e, int &kind) {
+        // where candidate e of the list has its slot, and its kind (reads LDS)
+        auto place = [&](int e, int &kind) {
             kind = NONE;
-            if (e >= total) return 0;
+            const int *q = f.hslot;
+            if (e >= total) return q;
             int m = 0;
             if (f.nchunk > 1) {
 #pragma unroll
@@ -1484,48 +1488,74 @@ __device__ __forceinline__ void fin_candidates(const FinParams &f, const IF64 &I
             const int k = e - pr.x;
             const size_t rowc = (size_t)(c0 + cstep * (cg + m)) * f.ni + i;
             kind = k < pr.y ? HARD : SOFT;
-            return k < pr.y ? f.hslot[rowc * f.caph + k] : f.sslot[rowc * f.caps + (k - pr.y)];
+            return k < pr.y ? f.hslot + rowc * f.caph + k : f.sslot + rowc * f.caps + (k - pr.y);
         };
-        int kn, en = entry(lane, kn);
-        for (int e0 = 0; e0 < total; e0 += 64) {
-            int kind = kn;
-            int sj = en;
-            // soft slots hold near-field pairs (force only) and, marked ~j, band pairs
-            // beyond the hard slots of an overflowing row; those were counted in
-            // dropped and are re-counted by the FP64 test here
-            const bool band = kind == SOFT && sj < 0;
-            if (band) {
+        // an entry as read from its slot: the candidate and its kind.  Soft slots hold near-field
+        // pairs (force only) and, marked ~j, band pairs beyond the hard slots of an
+        // overflowing row; those were counted in dropped and are re-counted by the FP64
+        // test here.  Kinds NONE and out-of-range entries take record 0 and no part.
+        auto decode = [&](int &kind, int &sj) {
+            if (kind == SOFT && sj < 0) {
                 sj = ~sj;
                 kind = BAND;
             }
-            const bool ok = kind != NONE && (unsigned)sj < (unsigned)f.nj;
-            if (!ok) sj = 0;
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last records are read
-            stage_records(f.rec64, sj, lane, st.rec);
-            const int jo = ok && kind == HARD ? f.perm[sj] - jb : 0;
-            kn = NONE;
-            if (e0 + 64 < total) en = entry(e0 + 64 + lane, kn);
+            if (kind == NONE || (unsigned)sj >= (unsigned)f.nj) {
+                kind = NONE;
+                sj = 0;
+            }
+        };
+        // Pass e0 computes while the records of the next pass, its neighbours' caller indices and
+        // the slot entries of the one after are on their way.  LDS is only touched before
+        // the fetches are issued (the compiler waits for a fetch into LDS before any
+        // other access to it), so a pass's neighbours go to buf in the next one.
+        int kind, sj, kn, jo, jn = 0;
+        const int *q = place(lane, kind);
+        sj = *q;
+        q = place(64 + lane, kn);
+        decode(kind, sj);
+        stage_records(f.rec64, sj, lane, st.rec);
+        jo = f.perm[sj];
+        int sn = *q;
+        unsigned long long nbm = 0ull;   // lanes whose last candidate is a neighbour (index jn)
+        auto keep = [&]() {
+            if (!nbm) return;
+            int base = nnb;
+            if (SHARED) {
+                int t = 0;
+                if (lane == 0) t = atomicAdd(nshared, __popcll(nbm));
+                base = __builtin_amdgcn_readfirstlane(t);
+            }
+            const int pos = base + lane_prefix(nbm);
+            if ((nbm >> lane & 1ull) && pos < cap) buf[pos] = jn - jb;
+            nnb += __popcll(nbm);
+        };
+        for (int e0 = 0; e0 < total; e0 += 64) {
             lds_dma_wait();
+            double4 r0, r1;
+            staged_record(st.rec, lane, r0, r1);
+            keep();
+            const int kc = kind;
+            jn = jo;
+            int kq;
+            q = place(e0 + 128 + lane, kq);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the records are read
+            if (e0 + 64 < total) {
+                kind = kn;
+                sj = sn;
+                decode(kind, sj);
+                stage_records(f.rec64, sj, lane, st.rec);
+                jo = f.perm[sj];
+                sn = *q;
+                kn = kq;
+            }
             bool isnb = false;
-            if (ok) {
-                double4 r0, r1;
-                staged_record(st.rec, lane, r0, r1);
-                isnb = pair64<MFLAG>(r0, r1, I, kind != SOFT, s);
-            }
-            const unsigned long long b = __ballot(isnb && kind == HARD);
-            if (b) {
-                int base = nnb;
-                if (SHARED) {
-                    int t = 0;
-                    if (lane == 0) t = atomicAdd(nshared, __popcll(b));
-                    base = __shfl(t, 0, 64);
-                }
-                const int pos = base + lane_prefix(b);
-                if (isnb && kind == HARD && pos < cap) buf[pos] = jo;
-                nnb += __popcll(b);
-            }
-            dropped += __popcll(__ballot(isnb && band)) - __popcll(__ballot(band));
+            if (kc != NONE) isnb = pair64<MFLAG>(r0, r1, I, kc != SOFT, s);
+            nbm = __ballot(isnb && kc == HARD);
+            const unsigned long long bm = __ballot(kc == BAND);
+            if (bm) dropped += __popcll(__ballot(isnb && kc == BAND)) - __popcll(bm);
         }
+        keep();
+        nbm = 0ull;
     }
 }
 
@@ -1715,11 +1745,11 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
     extern __shared__ __align__(16) int nbuf[];   // [4][row_cap]
     __shared__ FinStage stage[4];
     const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = xcd_order(blockIdx.x, gridDim.x) * 4 + wid;   // slot
     if (i >= f.ni) return;   // whole wavefront leaves together
     const int r = f.imap ? f.imap[i] : i;   // caller row
-    if (r < 0) return;
+    const int2 cnt0 = fin_counts(f, i, lane);
     const int cap = row_cap(f.nnbmax);
     int *buf = nbuf + wid * cap;
 
@@ -1736,6 +1766,7 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
             for (int q = 0; q < NERR; q++) e[q] += pp[(size_t)(7 + q) * f.ni];
         }
     }
+    if (r < 0) return;   // (an empty slot's counts and sums are there too)
 
     // 2. FP64 work on the candidates
     const int is = f.ib_stride;
@@ -1749,8 +1780,8 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
     int dropped = 0;      // hard candidates beyond the slot capacity
     int unres = 0;        // band pairs of an overflowing row left without a slot
     bool dropped_any = false;
-    fin_candidates<MFLAG, false>(f, I, i, jb, 0, 1, lane, s, buf, cap, stage[wid], nullptr, nnb,
-                                 dropped, unres, dropped_any);
+    fin_candidates<MFLAG, false>(f, I, i, jb, 0, 1, lane, s, buf, cap, stage[wid], nullptr, cnt0,
+                                 nnb, dropped, unres, dropped_any);
 
 #pragma unroll
     for (int q = 0; q < 7; q++) s[q] = wave_sum(s[q]);
@@ -1809,7 +1840,7 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
 // the partial sums' lines they share.  Forces are combined in a fixed
 // order; the row is rank-sorted as in regf_finalize_kernel.
 template <bool MFLAG, int W>
-__global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f) {
+__global__ __launch_bounds__(64 * W, 6) void regf_finalize_wide_kernel(FinParams f) {
     extern __shared__ __align__(16) int buf[];   // [row_cap]
     __shared__ FinStage stage[W];
     __shared__ double red[W][NPART];
@@ -1818,9 +1849,10 @@ __global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f)
     __shared__ int flag;             // 1: chunk items, 2: whole-row pass
     __shared__ double vtot[NPART];
     const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = xcd_order(blockIdx.x, gridDim.x);   // slot
     const int r = f.imap ? f.imap[i] : i;
+    const int2 cnt0 = fin_counts(f, i, w + W * lane);
     if (r < 0) return;   // the whole work-group leaves together
     if (threadIdx.x == 0) {
         nshared = 0;
@@ -1849,7 +1881,7 @@ __global__ __launch_bounds__(64 * W) void regf_finalize_wide_kernel(FinParams f)
     int nnb = 0, dropped = 0, unres = 0;
     bool dropped_any = false;
     fin_candidates<MFLAG, true>(f, I, i, jb, w, W, lane, s, buf, row_cap(f.nnbmax), stage[w],
-                                &nshared, nnb, dropped, unres, dropped_any);
+                                &nshared, cnt0, nnb, dropped, unres, dropped_any);
 #pragma unroll
     for (int q = 0; q < NPART; q++) s[q] = wave_sum(s[q]);
     if (lane == 0) {
