@@ -448,7 +448,7 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
 // Tile kernel (the loop that the compiler made, then this one): N = 100,003, ni = 6007 with
 // m_flag, where 99 % of the tiles are tested, 640 -> 564 us; N = 65,536, ni = 1024
 // (all) 100 -> 86 us; send and force of N = 2^20, ni = 2^17 (9 %) 92.8 -> 89.5 ms.
-#define NEAR_PAIR(X, Y, Z0, M, U, V, W, Z, K, NEXT, THQ, TQ, THR)                           \
+#define NEAR_PAIR(X, Y, Z0, M, U, V, W, Z, K, NEXT, THQ, TQ, THR, REC)                      \
     "s_waitcnt lgkmcnt(0)\n" NEXT                                                           \
     "v_sub_f32 " X ", " X ", v24\n"                                                         \
     "v_sub_f32 " Y ", " Y ", v25\n"                                                         \
@@ -486,26 +486,7 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
     "s_or_b64 %[x], %[h], vcc\n"                                                            \
     "s_cbranch_scc0 .Lr" K "_%=\n"                                                          \
     "s_andn2_b64 %[f], vcc, %[h]\n"                                                         \
-    "s_add_i32 %[j], %[jb], " K "\n"                                                        \
-    "v_cmp_le_i32 vcc, %[caph], v46\n"                                                      \
-    "s_and_b64 vcc, vcc, %[h]\n"                                                            \
-    "s_cbranch_scc1 .Lx_%=\n"                                                               \
-    "v_cmp_le_i32 vcc, %[lim], v47\n"                                                       \
-    "s_and_b64 vcc, vcc, %[f]\n"                                                            \
-    "s_cbranch_scc1 .Lx_%=\n"                                                               \
-    "v_mov_b32 v23, %[j]\n"                                                                 \
-    "s_mov_b64 exec, %[h]\n"                                                                \
-    "s_cbranch_execz .Lf" K "_%=\n"                                                         \
-    "v_mad_u64_u32 v[54:55], vcc, v46, 4, v[48:49]\n"                                       \
-    "global_store_dword v[54:55], v23, off\n"                                               \
-    "v_add_u32 v46, 1, v46\n"                                                               \
-    ".Lf" K "_%=:\n"                                                                        \
-    "s_mov_b64 exec, %[f]\n"                                                                \
-    "s_cbranch_execz .Lh" K "_%=\n"                                                         \
-    "v_mad_u64_u32 v[54:55], vcc, v47, 4, v[50:51]\n"                                       \
-    "global_store_dword v[54:55], v23, off\n"                                               \
-    "v_add_u32 v47, 1, v47\n"                                                               \
-    ".Lh" K "_%=:\n"                                                                        \
+    REC                                                                                     \
     "s_mov_b64 exec, %[x]\n"                                                                \
     "v_mov_b32 v18, 0\n"                                                                    \
     ".Lr" K "_%=:\n"                                                                        \
@@ -527,21 +508,52 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
     "v_fmac_f32 v36, v16, " V "\n"                                                          \
     "v_fmac_f32 v33, v16, " W "\n"                                                          \
     "v_fmac_f32 v37, v20, v21\n"
-#define NEAR_A(K, NEXT, THQ, TQ, THR)                                                       \
-    NEAR_PAIR("v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", K, NEXT, THQ("v3"), TQ, THR("v3"))
-#define NEAR_B(K, NEXT, THQ, TQ, THR)                                                       \
+// a pair's candidates: to the lanes' next slots (leaving the loop where one has none) ...
+#define NEAR_SLOTS(K)                                                                       \
+    "s_add_i32 %[j], %[jb], " K "\n"                                                        \
+    "v_cmp_le_i32 vcc, %[caph], v46\n"                                                      \
+    "s_and_b64 vcc, vcc, %[h]\n"                                                            \
+    "s_cbranch_scc1 .Lx_%=\n"                                                               \
+    "v_cmp_le_i32 vcc, %[lim], v47\n"                                                       \
+    "s_and_b64 vcc, vcc, %[f]\n"                                                            \
+    "s_cbranch_scc1 .Lx_%=\n"                                                               \
+    "v_mov_b32 v23, %[j]\n"                                                                 \
+    "s_mov_b64 exec, %[h]\n"                                                                \
+    "s_cbranch_execz .Lf" K "_%=\n"                                                         \
+    "v_mad_u64_u32 v[54:55], vcc, v46, 4, v[48:49]\n"                                       \
+    "global_store_dword v[54:55], v23, off\n"                                               \
+    "v_add_u32 v46, 1, v46\n"                                                               \
+    ".Lf" K "_%=:\n"                                                                        \
+    "s_mov_b64 exec, %[f]\n"                                                                \
+    "s_cbranch_execz .Lh" K "_%=\n"                                                         \
+    "v_mad_u64_u32 v[54:55], vcc, v47, 4, v[50:51]\n"                                       \
+    "global_store_dword v[54:55], v23, off\n"                                               \
+    "v_add_u32 v47, 1, v47\n"                                                               \
+    ".Lh" K "_%=:\n"
+// ... or to bits of v46 (hard) and v47 (soft)
+#define NEAR_BITS(K)                                                                        \
+    "s_add_i32 %[j], %[jb], " K "\n"                                                        \
+    "s_lshl_b32 %[j], 1, %[j]\n"                                                            \
+    "s_mov_b64 exec, %[h]\n"                                                                \
+    "v_or_b32 v46, %[j], v46\n"                                                             \
+    "s_mov_b64 exec, %[f]\n"                                                                \
+    "v_or_b32 v47, %[j], v47\n"
+#define NEAR_A(K, NEXT, THQ, TQ, THR, REC)                                                       \
+    NEAR_PAIR("v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", K, NEXT, THQ("v3"), TQ, THR("v3"), \
+              REC(K))
+#define NEAR_B(K, NEXT, THQ, TQ, THR, REC)                                                       \
     NEAR_PAIR("v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", K, NEXT, THQ("v11"), TQ, \
-              THR("v11"))
-#define NEAR_LOOP(THQ, TQ, THR)                                                             \
+              THR("v11"), REC(K))
+#define NEAR_LOOP(THQ, TQ, THR, REC)                                                             \
     ".Ln%=:\n" FAR_LA("0")                                                                  \
-    NEAR_A("0", FAR_LB("16"), THQ, TQ, THR)                                                 \
-    NEAR_B("1", FAR_LA("32"), THQ, TQ, THR)                                                 \
-    NEAR_A("2", FAR_LB("48"), THQ, TQ, THR)                                                 \
-    NEAR_B("3", FAR_LA("64"), THQ, TQ, THR)                                                 \
-    NEAR_A("4", FAR_LB("80"), THQ, TQ, THR)                                                 \
-    NEAR_B("5", FAR_LA("96"), THQ, TQ, THR)                                                 \
-    NEAR_A("6", FAR_LB("112"), THQ, TQ, THR)                                                \
-    NEAR_B("7", "", THQ, TQ, THR)                                                           \
+    NEAR_A("0", FAR_LB("16"), THQ, TQ, THR, REC)                                                 \
+    NEAR_B("1", FAR_LA("32"), THQ, TQ, THR, REC)                                                 \
+    NEAR_A("2", FAR_LB("48"), THQ, TQ, THR, REC)                                                 \
+    NEAR_B("3", FAR_LA("64"), THQ, TQ, THR, REC)                                                 \
+    NEAR_A("4", FAR_LB("80"), THQ, TQ, THR, REC)                                                 \
+    NEAR_B("5", FAR_LA("96"), THQ, TQ, THR, REC)                                                 \
+    NEAR_A("6", FAR_LB("112"), THQ, TQ, THR, REC)                                                \
+    NEAR_B("7", "", THQ, TQ, THR, REC)                                                           \
     "v_add_u32 %[a], 0x80, %[a]\n"                                                          \
     "v_add_u32 %[b], 0x80, %[b]\n"                                                          \
     "s_add_i32 %[jb], %[jb], 8\n"                                                           \
@@ -572,7 +584,7 @@ __device__ __forceinline__ int near_loop(const float4 *sA, const float4 *sB, con
     unsigned long long mh, mf, mx;
     int j, jb = j0;
     if (MFLAG)
-        asm volatile(NEAR_LOOP(NEAR_TQ1, "v54", NEAR_TH1)
+        asm volatile(NEAR_LOOP(NEAR_TQ1, "v54", NEAR_TH1, NEAR_SLOTS)
                      : [a] "+&v"(a), [b] "+&v"(b), [jb] "+&s"(jb), [j] "=&s"(j), [h] "=&s"(mh),
                        [f] "=&s"(mf), [x] "=&s"(mx), "+{v46}"(nhk), "+{v47}"(nsk),
                        "+{v31}"(acc[0]), "+{v30}"(acc[1]), "+{v32}"(acc[2]), "+{v34}"(acc[3]),
@@ -584,7 +596,7 @@ __device__ __forceinline__ int near_loop(const float4 *sA, const float4 *sB, con
                        [caph] "s"(caph), [lim] "s"(lim), [je] "s"(j0 + RF_FLUSH)
                      : NEAR_CLOBBERS);
     else
-        asm volatile(NEAR_LOOP(NEAR_TQ0, "v40", NEAR_TH0)
+        asm volatile(NEAR_LOOP(NEAR_TQ0, "v40", NEAR_TH0, NEAR_SLOTS)
                      : [a] "+&v"(a), [b] "+&v"(b), [jb] "+&s"(jb), [j] "=&s"(j), [h] "=&s"(mh),
                        [f] "=&s"(mf), [x] "=&s"(mx), "+{v46}"(nhk), "+{v47}"(nsk),
                        "+{v31}"(acc[0]), "+{v30}"(acc[1]), "+{v32}"(acc[2]), "+{v34}"(acc[3]),
@@ -595,6 +607,38 @@ __device__ __forceinline__ int near_loop(const float4 *sA, const float4 *sB, con
                        [caph] "s"(caph), [lim] "s"(lim), [je] "s"(j0 + RF_FLUSH)
                      : NEAR_CLOBBERS);
     return j;
+}
+
+// near_loop over 32 j for callers that give out slots later: every candidate is left out of the
+// sums and marked in hard or soft (bit = j).
+template <bool MFLAG>
+__device__ __forceinline__ void near_mark(const float4 *sA, const float4 *sB, const IC &c,
+                                          unsigned &hard, unsigned &soft, float *__restrict__ acc,
+                                          float &s3) {
+    unsigned a = (unsigned)(uintptr_t)(lds_void *)sA, b = (unsigned)(uintptr_t)(lds_void *)sB;
+    unsigned long long mh, mf, mx;
+    int j, jb = 0;
+    if (MFLAG)
+        asm volatile(NEAR_LOOP(NEAR_TQ1, "v54", NEAR_TH1, NEAR_BITS)
+                     : [a] "+&v"(a), [b] "+&v"(b), [jb] "+&s"(jb), [j] "=&s"(j), [h] "=&s"(mh),
+                       [f] "=&s"(mf), [x] "=&s"(mx), "+{v46}"(hard), "+{v47}"(soft),
+                       "+{v31}"(acc[0]), "+{v30}"(acc[1]), "+{v32}"(acc[2]), "+{v34}"(acc[3]),
+                       "+{v35}"(acc[4]), "+{v36}"(acc[5]), "+{v33}"(acc[6]), "+{v37}"(s3)
+                     : "{v24}"(c.x), "{v25}"(c.y), "{v26}"(c.z), "{v27}"(c.u), "{v28}"(c.v),
+                       "{v29}"(c.w), "{v38}"(c.dt1), "{v39}"(c.dt2), "{v40}"(c.hQ), "{v41}"(c.hH),
+                       "{v42}"(c.hS), "{v43}"(c.dQ), "{v44}"(c.dH), "{v45}"(c.dS),
+                       [je] "s"(32)
+                     : NEAR_CLOBBERS);
+    else
+        asm volatile(NEAR_LOOP(NEAR_TQ0, "v40", NEAR_TH0, NEAR_BITS)
+                     : [a] "+&v"(a), [b] "+&v"(b), [jb] "+&s"(jb), [j] "=&s"(j), [h] "=&s"(mh),
+                       [f] "=&s"(mf), [x] "=&s"(mx), "+{v46}"(hard), "+{v47}"(soft),
+                       "+{v31}"(acc[0]), "+{v30}"(acc[1]), "+{v32}"(acc[2]), "+{v34}"(acc[3]),
+                       "+{v35}"(acc[4]), "+{v36}"(acc[5]), "+{v33}"(acc[6]), "+{v37}"(s3)
+                     : "{v24}"(c.x), "{v25}"(c.y), "{v26}"(c.z), "{v27}"(c.u), "{v28}"(c.v),
+                       "{v29}"(c.w), "{v38}"(c.dt1), "{v39}"(c.dt2), "{v40}"(c.hQ), "{v41}"(c.hH),
+                       "{v42}"(c.hS), [je] "s"(32)
+                     : NEAR_CLOBBERS);
 }
 
 // FP64 partial sums and error scales of this lane's i-particles to part row `row`
@@ -800,10 +844,12 @@ __global__ __launch_bounds__(T, (regf_waves<T, IPL>())) void regf_tile_kernel(Ti
 // pieces of each 256-j tile side by side.  Bound by latency: one wavefront walks 64 j in place
 // of 256.  Partial sums, error scales and candidate slots come out as the 256-wide form
 // leaves them, bit for bit: a piece is one FP32 partial sum there too, and wavefront 0 adds
-// the four in j order; which soft pairs still find a slot depends on the pieces before, so
-// the neighbour test runs first and leaves bit masks, from which every wavefront knows the
-// slots taken before its own, and the force loop leaves out the pairs that got one.
-// N = 50,021, ni = 257: 74 -> 42 us; N = 1024, ni = 40: 69 -> 32 us.
+// the four in j order.  Which soft pairs still find a slot depends on the pieces before, so
+// the loop leaves bit masks of its candidates, from which every wavefront knows the slots
+// taken before its own; where a row has too few for all of them, the piece is taken again
+// and the force loop leaves out only the pairs that got one.
+// N = 50,021, ni = 257: 74 -> 42 us, 36 with near_mark in place of a test loop and a masked force
+// loop; N = 1024, ni = 40: 69 -> 32 -> 23 us.
 struct PieceMask {
     unsigned long long hard, soft, band;   // band: hard pairs that the FP64 test has to decide
 };
@@ -866,10 +912,27 @@ __global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
         const bool near = !(p.far_test && lane_far<MFLAG>(c, ok, p.tbox + tt * TBOX));
         lds_dma_wait();                      // a wavefront reads only the records it staged
         PieceMask m = {0ull, 0ull, 0ull};
-        if (__ballot(near)) {
-#pragma unroll 4
+        float acc[NACC] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, s3 = 0.f;
+        const bool anear = __ballot(near) != 0ull;
+        const float4 *pA = &sA[w * 64], *pB = &sB[w * 64];
+        // sums without any candidate and the candidates' marks; pieces of rows with slots enough
+        // for all of them (the next step) need no more
+        const bool whole = jt + w * 64 + 64 <= j1;
+        if (!anear) {
+            far_loop(pA, pB, c, acc, s3);
+        } else if (whole) {
+            unsigned h0 = 0, h1 = 0, s0 = 0, s1 = 0;
+            near_mark<MFLAG>(pA, pB, c, h0, s0, acc, s3);
+            near_mark<MFLAG>(pA + 32, pB + 32, c, h1, s1, acc, s3);
+            m.hard = h0 | (unsigned long long)h1 << 32;
+            m.soft = s0 | (unsigned long long)s1 << 32;
+        }
+        // the marks alone, for the last piece of the j-set and for rows that run out of slots
+        auto marks = [&]() {
+            m = {0ull, 0ull, 0ull};
+#pragma unroll 1
             for (int jj = 0; jj < 64; jj++) {
-                const float4 ra = sA[w * 64 + jj], rb = sB[w * 64 + jj];
+                const float4 ra = pA[jj], rb = pB[jj];
                 const PairBase q = pair_base(c, ra, rb);
                 const float t1 = fmaf(c.dt2, fminf(q.rv, 0.f), q.r2);
                 const float thq = MFLAG ? fmaf(ra.w, c.hQ, c.dQ) : c.hQ;
@@ -887,9 +950,21 @@ __global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
                     }
                 }
             }
-        }
+        };
+        if (anear && !whole) marks();
         sM[w][lane] = m;
         __syncthreads();
+        // rows whose hard slots run out need the band marks too (every wavefront comes to the
+        // same answer)
+        int c4 = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) c4 += __popcll(sM[q][lane].hard);
+        if (__ballot(nh + c4 > p.caph)) {
+            __syncthreads();
+            if (anear) marks();
+            sM[w][lane] = m;
+            __syncthreads();
+        }
         // slots before this piece, then this piece's own, then the tile's
         unsigned long long kept = 0ull, left = 0ull;
         for (int q = 0; q < 4; q++) {
@@ -913,17 +988,18 @@ __global__ __launch_bounds__(256, 4) void regf_tile_small_kernel(TileParams p) {
                 }
             }
         }
-        float acc[NACC] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, s3 = 0.f;
-        if (__ballot(left != 0ull)) {
-#pragma unroll 4
+        // pieces with a candidate that got no slot, or without sums so far
+        if (anear && (!whole || __ballot(left != (m.hard | m.soft)))) {
+#pragma unroll
+            for (int q = 0; q < NACC; q++) acc[q] = 0.f;
+            s3 = 0.f;
+#pragma unroll 2
             for (int jj = 0; jj < 64; jj++) {
-                const float4 ra = sA[w * 64 + jj], rb = sB[w * 64 + jj];
+                const float4 ra = pA[jj], rb = pB[jj];
                 const PairBase q = pair_base(c, ra, rb);
                 const float rinv = (left >> jj) & 1ull ? 0.f : rinv_nr(q.r2);
                 pair_add(q, rinv, ra.w, acc, s3);
             }
-        } else {
-            far_loop(&sA[w * 64], &sB[w * 64], c, acc, s3);
         }
 #pragma unroll
         for (int q = 0; q < NACC; q++) sP[w][q][lane] = acc[q];
