@@ -2769,10 +2769,15 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     }
     // 64 i per work-group and the tile's four pieces side by side (the same bits) up to 1792
     // such work-groups, seven per CU; with more the 256-wide form fills the GPU by itself and
-    // runs the neighbour test and the force in one loop.  Whole call: N = 65,536, ni = 256
-    // (1024 of them) 244 -> 216 us, ni = 512 (2048) 248 and 250, ni = 700 (2816) 262 and 279
+    // adds up its pieces without LDS.  Whole call: N = 65,536, ni = 256 (1024 of them)
+    // 244 -> 216 us, ni = 512 (2048) 160 with it and 164 with 64, ni = 768 (3072) 174 and
+    // 189.  Above 1792 still where a 256-wide block would leave three eighths of its lanes
+    // empty: ni = 270 at N = 100,003 (1955) 197 -> 177 us, at 400,000 (7815) 496 -> 459;
+    // ni = 100 at 300,000 357 -> 328.  (A quarter empty: 540 at 65,536 170 and 174, 520 at
+    // 131,072 248 and 238.)
+    const long long n64 = (ni + 63) / 64, g64 = n64 * nchunk;
     const bool small = cfg.prec == 0 && cfg.threads == 256 && cfg.ipl == 1 && P == 1 &&
-                       (long long)((ni + 63) / 64) * nchunk <= 1792;
+                       (g64 <= 1792 || (g64 <= 8192 && 8 * n64 <= 5 * 4 * (long long)nib));
     const size_t rows = (size_t)nchunk * nbatch_i;
     // rows the finalize flags for the FP64 pass (FP32 production kernel only)
     const int fix_items = na ? na->fix_items : FIX_ITEMS;
