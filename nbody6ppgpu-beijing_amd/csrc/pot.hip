@@ -34,29 +34,48 @@ struct PotParams {
 
 // One LDS tile against this lane's i, compensated (Kahan) FP32 sums from zero: one close
 // pair (a tight binary) can dominate the tile sum.  CHECK: pairs with r2 = 0 (the particle
-// itself, coincident ones) and with values that are not finite add nothing.
+// itself, coincident ones) and with values that are not finite add nothing.  Four pairs at a
+// time, their reciprocal square roots together and at raised priority: without it the two
+// wavefronts that a SIMD issues side by side fall into step at these slow instructions and
+// take turns afterwards (n = 262,144: 20.7 -> 20.2 ms; the same order without priority 21.2).
 template <int IPL, bool CHECK>
 __device__ __forceinline__ void pot_tile(const double4 *sJ, const double *xi, const double *yi,
                                          const double *zi, float *a32, float *c32) {
 #pragma unroll
     for (int k = 0; k < IPL; k++) a32[k] = c32[k] = 0.f;
-#pragma unroll 4
-    for (int jj = 0; jj < PT_TJ; jj++) {
-        const double4 b = sJ[jj];
-        const float mj = __int_as_float(__double2loint(b.w));   // (stored as FP32)
+    constexpr int U = 4 / IPL;
+#pragma unroll 2
+    for (int j0 = 0; j0 < PT_TJ; j0 += U) {
+        float mj[U], r2[U][IPL], ri[U][IPL];
 #pragma unroll
-        for (int k = 0; k < IPL; k++) {
-            const float dx = (float)(b.x - xi[k]);
-            const float dy = (float)(b.y - yi[k]);
-            const float dz = (float)(b.z - zi[k]);
-            const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-            float ri = __builtin_amdgcn_rsqf(r2);
-            if (CHECK) ri = r2 > 0.f ? ri : 0.f;
-            const float y = fmaf(mj, ri, -c32[k]);
-            const float t = a32[k] + y;
-            c32[k] = (t - a32[k]) - y;
-            a32[k] = t;
+        for (int u = 0; u < U; u++) {
+            const double4 b = sJ[j0 + u];
+            mj[u] = __int_as_float(__double2loint(b.w));   // (stored as FP32)
+#pragma unroll
+            for (int k = 0; k < IPL; k++) {
+                const float dx = (float)(b.x - xi[k]);
+                const float dy = (float)(b.y - yi[k]);
+                const float dz = (float)(b.z - zi[k]);
+                r2[u][k] = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+            }
         }
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 0; k < IPL; k++) ri[u][k] = __builtin_amdgcn_rsqf(r2[u][k]);
+        __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 0; k < IPL; k++) {
+                float q = ri[u][k];
+                if (CHECK) q = r2[u][k] > 0.f ? q : 0.f;
+                const float y = fmaf(mj[u], q, -c32[k]);
+                const float t = a32[k] + y;
+                c32[k] = (t - a32[k]) - y;
+                a32[k] = t;
+            }
     }
 }
 
