@@ -1355,6 +1355,43 @@ __device__ __forceinline__ double wave_sum(double v) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
                             __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
+// Two lane arrays folded into one: sums of lanes l and l + 32 of a in the lower half, of b in
+// the upper (fold32); of rows of 16 lanes 0 + 1 and 2 + 3 of a in rows 0 and 2, of b in rows 1
+// and 3 (fold16).
+__device__ __forceinline__ double fold32(double a, double b) {
+    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+    const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+// v[q], q < NPART, summed over the wavefront (the same in every lane).  Folding pairs of values
+// before the sums within rows takes 85 instructions where eleven sums one by one take
+// 220 (finalize of 381,067 rows 1402 -> 1382 us; send and force at N = 50,021, ni = 257
+// 141.6 -> 140.7 us).
+__device__ __forceinline__ void wave_sums(double *v) {
+    static_assert(NPART == 11, "three groups of four values, one of them empty");
+    double w[3];
+#pragma unroll
+    for (int g = 0; g < 3; g++) {
+        const double d = 4 * g + 3 < NPART ? v[4 * g + 3] : 0.0;
+        w[g] = fold16(fold32(v[4 * g], v[4 * g + 1]), fold32(v[4 * g + 2], d));
+        w[g] += dpp0<0x111, 0xf>(w[g]);
+        w[g] += dpp0<0x112, 0xf>(w[g]);
+        w[g] += dpp0<0x114, 0xf>(w[g]);
+        w[g] += dpp0<0x118, 0xf>(w[g]);
+    }
+    // rows of w[g]: values 4 g, 4 g + 2, 4 g + 1, 4 g + 3
+#pragma unroll
+    for (int q = 0; q < NPART; q++) {
+        const int l = 15 + 16 * ((q & 1) * 2 + (q >> 1 & 1));
+        v[q] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(w[q >> 2]), l),
+                                __builtin_amdgcn_readlane(__double2loint(w[q >> 2]), l));
+    }
+}
 __device__ __forceinline__ int wave_sum_i(int v) {
     return __builtin_amdgcn_readlane(wave_last(v), 63);
 }
@@ -1830,9 +1867,10 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
     int *buf = nbuf + wid * cap;
 
     // 1. FP64 sum of the chunk partials (and of the error scales)
-    double s[7], e[NERR] = {0.0, 0.0, 0.0, 0.0};
+    double s[NPART];                 // sums, then the error scales e
+    double *e = s + 7;
 #pragma unroll
-    for (int q = 0; q < 7; q++) s[q] = 0.0;
+    for (int q = 0; q < NPART; q++) s[q] = 0.0;
     for (int c = lane; c < f.nprow; c += 64) {
         const double *pp = f.part + (size_t)c * NPART * f.ni + i;
 #pragma unroll
@@ -1859,12 +1897,7 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
     fin_candidates<MFLAG, false>(f, I, i, jb, 0, 1, lane, s, buf, cap, stage[wid], nullptr, cnt0,
                                  nnb, dropped, unres, dropped_any);
 
-#pragma unroll
-    for (int q = 0; q < 7; q++) s[q] = wave_sum(s[q]);
-    if (f.refine || f.dbg) {
-#pragma unroll
-        for (int q = 0; q < NERR; q++) e[q] = wave_sum(e[q]);
-    }
+    wave_sums(s);
     int *row = f.list + (size_t)r * f.lmax;
     const int tot = nnb + dropped;
     // a row whose hard slots overflowed reports -count, as any overflow does, even in
@@ -1893,12 +1926,7 @@ __global__ __launch_bounds__(256, 6) void regf_finalize_kernel(FinParams f) {
         if (unres > 0 || !f.items) {
             if (lane == 0) f.fix_rows[atomicAdd(f.nfix, 1)] = f.fix_slot ? i : r + f.row_base;
         } else {
-            double se[7 + NERR];
-#pragma unroll
-            for (int q = 0; q < 7; q++) se[q] = s[q];
-#pragma unroll
-            for (int q = 0; q < NERR; q++) se[7 + q] = e[q];
-            emit_chunks(f, i, r, se, lane);
+            emit_chunks(f, i, r, s, lane);
         }
     }
     if (!ovf && nnb > 0) {
@@ -1958,8 +1986,7 @@ __global__ __launch_bounds__(64 * W, 6) void regf_finalize_wide_kernel(FinParams
     bool dropped_any = false;
     fin_candidates<MFLAG, true>(f, I, i, jb, w, W, lane, s, buf, row_cap(f.nnbmax), stage[w],
                                 &nshared, cnt0, nnb, dropped, unres, dropped_any);
-#pragma unroll
-    for (int q = 0; q < NPART; q++) s[q] = wave_sum(s[q]);
+    wave_sums(s);
     if (lane == 0) {
 #pragma unroll
         for (int q = 0; q < NPART; q++) red[w][q] = s[q];
