@@ -220,7 +220,8 @@ int nb6_set_regf_debug_bounds(double *d_bounds);
  * reference, which holds one j-set per library instance).
  *   nb6_ens_send_device: offsets[nclusters+1] (host) index the concatenated SoA
  *     double[7][stride] (x,y,z,vx,vy,vz,m) on the device; cluster c owns
- *     [offsets[c], offsets[c+1]).
+ *     [offsets[c], offsets[c+1]).  Returns when the j-set is complete: the step may
+ *     follow on any stream.
  *   nb6_ens_regf_device: one regular step of every particle of every cluster
  *     against its own cluster: d_i SoA double[8][stride] (x,y,z,vx,vy,vz,h2,dtr)
  *     for all particles, d_out SoA double[7][stride], d_list int[ntot][lmax] with

@@ -280,7 +280,6 @@ int ens_send_device(int nc, const int *offsets, const double *d_soa, int stride,
     double *mmax = e.js.stat.as<double>() + 6;
     hipLaunchKernelGGL(ens_soa_to_aos, dim3((n + 255) / 256), dim3(256), 0, s, d_soa, n, stride, in64,
                        mmax);
-    jset_input_queued(e.js, s);
     hipLaunchKernelGGL(ens_bbox_kernel, dim3(nc), dim3(EB), 0, s, in64, e.d_off.as<int>(),
                        e.d_box.as<double>(), reinterpret_cast<unsigned long long *>(mmax));
     hipLaunchKernelGGL(ens_key_kernel, dim3((n + 255) / 256), dim3(256), 0, s, in64, n,
@@ -301,7 +300,9 @@ int ens_send_device(int nc, const int *offsets, const double *d_soa, int stride,
     // (padding sits at the end of a cluster's last tile)
     jset_build_clusters(e.js, e.npad, in64, e.d_svals.as<int>(), e.d_off.as<int>(),
                         e.d_padoff.as<int>(), nc, s);
-    jset_input_wait(e.js);
+    // The j-set is complete when the send returns: the step may run on another stream, also
+    // from a graph that the caller captured, where no event of this one could be waited for.
+    NB6_HIP(hipStreamSynchronize(s));
     const RegfConfig cfg = regf_effective(0);
     if (same_layout && e.items_bi == cfg.threads * cfg.ipl) return OK;
     const int rc = build_items(e, s);
