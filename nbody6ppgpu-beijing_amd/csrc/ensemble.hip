@@ -116,9 +116,9 @@ __global__ void ens_zero_kernel(int *q) { *q = 0; }
 
 struct GraphKey {
     const void *ptr[4] = {nullptr, nullptr, nullptr, nullptr};   // d_i, d_out, d_list, items
-    long long val[18] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    long long val[19] = {};
     bool operator==(const GraphKey &o) const {
-        return std::equal(ptr, ptr + 4, o.ptr) && std::equal(val, val + 18, o.val);
+        return std::equal(ptr, ptr + 4, o.ptr) && std::equal(val, val + 19, o.val);
     }
 };
 
@@ -332,17 +332,18 @@ int ens_regf_device(const double *d_i, int stride, int lmax, int nnbmax, int m_f
                                  nnbmax, m_flag, d_out, d_list, grid, e.work, st);
     };
     if (!use_graph) return step(s);
-    // The graph holds kernel arguments by value: pointers, sizes and the launch shape.  Any
-    // change there needs a new capture.
+    // The graph holds kernel arguments by value: pointers, sizes, the launch shape and what
+    // the clusters' number and longest one determine (segments, buckets).  Any change there
+    // needs a new capture.
     GraphKey key;
     key.ptr[0] = d_i; key.ptr[1] = d_out; key.ptr[2] = d_list; key.ptr[3] = e.d_items.p;
     int nbits = 0, kb[4] = {0, 0, 0, 0};
     std::memcpy(&nbits, &cfg.near, sizeof(nbits));
     std::memcpy(kb, cfg.kref_ens, sizeof(kb));
-    const long long v[18] = {stride, lmax, nnbmax, m_flag, cfg.threads, cfg.ipl, e.nitems, grid,
-                             e.ntot, e.npad, 0, cfg.far_test, cfg.refine, nbits,
+    const long long v[19] = {stride, lmax, nnbmax, m_flag, cfg.threads, cfg.ipl, e.nitems, grid,
+                             e.ntot, e.npad, e.nc, e.maxseg, cfg.far_test, cfg.refine, nbits,
                              kb[0], kb[1], kb[2], kb[3]};
-    std::copy(v, v + 18, key.val);
+    std::copy(v, v + 19, key.val);
     const bool same = e.exec && key == e.gkey;
     if (!same) {
         drop_graph();
