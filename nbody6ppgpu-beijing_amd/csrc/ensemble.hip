@@ -115,10 +115,14 @@ __global__ __launch_bounds__(256) void ens_soa_to_aos(const double *__restrict__
 __global__ void ens_zero_kernel(int *q) { *q = 0; }
 
 struct GraphKey {
-    const void *ptr[4] = {nullptr, nullptr, nullptr, nullptr};   // d_i, d_out, d_list, items
+    // d_i, d_out, d_list, items, error-scale output
+    const void *ptr[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+    // A buffer that a larger step outgrew is freed; where it lies at the same address again it is
+    // larger than the captured step needs.
+    std::array<const void *, 11> work = {};
     long long val[19] = {};
     bool operator==(const GraphKey &o) const {
-        return std::equal(ptr, ptr + 4, o.ptr) && std::equal(val, val + 19, o.val);
+        return std::equal(ptr, ptr + 5, o.ptr) && work == o.work && std::equal(val, val + 19, o.val);
     }
 };
 
@@ -337,6 +341,8 @@ int ens_regf_device(const double *d_i, int stride, int lmax, int nnbmax, int m_f
     // needs a new capture.
     GraphKey key;
     key.ptr[0] = d_i; key.ptr[1] = d_out; key.ptr[2] = d_list; key.ptr[3] = e.d_items.p;
+    key.ptr[4] = regf_debug_bounds();
+    key.work = e.work.batched();
     int nbits = 0, kb[4] = {0, 0, 0, 0};
     std::memcpy(&nbits, &cfg.near, sizeof(nbits));
     std::memcpy(kb, cfg.kref_ens, sizeof(kb));
@@ -356,6 +362,7 @@ int ens_regf_device(const double *d_i, int stride, int lmax, int nnbmax, int m_f
         NB6_HIP(hipStreamEndCapture(s, &e.graph));
         if (rc != OK) return rc;
         NB6_HIP(hipGraphInstantiate(&e.exec, e.graph, nullptr, nullptr, 0));
+        key.work = e.work.batched();   // (as the eager step sized them)
         e.gkey = key;
         return OK;   // the eager step already produced this call's results
     }

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -165,6 +166,11 @@ struct RegfWork {
     DBuf fixrows, nfix, fixpart;     // FP64 pass: whole rows, counters, chunk sums
     DBuf items, delta, rowsel;       // FP64 pass: (row, chunk) items, candidate terms, rows
     DBuf segitems, part64;           // FP64 pass: items by chunk, FP64 sums per sub-range
+    // the buffers of a batched step (regf_items_launch), which a captured one holds by address
+    std::array<const void *, 11> batched() const {
+        return {part.p, cnt.p, hslot.p, sslot.p, fixrows.p, nfix.p, segitems.p, items.p, delta.p,
+                part64.p, rowsel.p};
+    }
     void release() {
         part.release(); cnt.release(); hslot.release(); sslot.release();
         ikey.release(); ival.release(); itmp.release();
@@ -192,6 +198,7 @@ int regf_items_launch(const JSet &js, int nslots, const int *imap, int stride, c
 int regf_items_refined();     // rows of the last batched step's FP64 pass (synchronises)
 void regf_items_forget();     // the ensemble's work buffers are gone
 void regf_set_debug_bounds(double *d);   // rows' error scales to d[4][out_stride] (or null)
+const double *regf_debug_bounds();
 
 // streaming copy of bytes (multiple of 16) on stream s
 void device_copy(void *dst, const void *src, size_t bytes, hipStream_t s);

@@ -3266,6 +3266,7 @@ int regf_items_launch(const JSet &js, int nslots, const int *imap, int stride, c
 
 void regf_items_forget() { g_ens_nfix = nullptr; }
 void regf_set_debug_bounds(double *d) { g_dbg = d; }
+const double *regf_debug_bounds() { return g_dbg; }
 
 int regf_items_refined() {
     if (!g_ens_nfix) return 0;

@@ -79,3 +79,34 @@ def test_layout_of_equal_totals_and_another_longest_cluster():
     finally:
         e.L.nb6_set_ens_refine_weights(0.5, 0.5, 0.5, 0.0)
         e.close()
+
+
+def test_work_buffers_that_a_larger_step_outgrew():
+    """A step with longer rows between two graph steps takes larger work buffers, so the graph's
+    are gone; the same for the switched diagnostic output."""
+    e = Ens([[3000, 900, 1500]], 600)
+    dbg = lib.DeviceArray(4 * e.ntot * 8)
+    try:
+        e.send(0)
+        first = [e.step(1, 80, 60) for _ in range(2)]
+        e.step(0, 600, 560)
+        after = [e.step(1, 80, 60) for _ in range(3)]
+        want = e.step(0, 80, 60)
+        for out, lst in first + after:
+            assert np.array_equal(out, want[0])
+            assert _same_rows(lst, want[1])
+        # the error scales follow the switch, from eager and from replayed steps
+        ref = np.full((4, e.ntot), -1.0)
+        scales = []
+        for ptr in (dbg.ptr, None, dbg.ptr):
+            e.L.nb6_set_regf_debug_bounds(ptr)
+            e.L.nb6_memcpy_htod(dbg.ptr, ref.ctypes.data, ref.nbytes)
+            out, _ = e.step(1, 80, 60)
+            assert np.array_equal(out, want[0])
+            scales.append(dbg.to_host(np.float64, (4, e.ntot)))
+        assert (scales[0] >= 0).all() and np.array_equal(scales[0], scales[2])
+        assert (scales[1] == -1.0).all()
+    finally:
+        e.L.nb6_set_regf_debug_bounds(None)
+        dbg.free()
+        e.close()
