@@ -2192,9 +2192,8 @@ struct ChunkFixParams {
     const int *__restrict__ nrows;
     double *__restrict__ out;        // SoA [7][out_stride] (of the batch)
     int out_stride;
-    const int *__restrict__ padoff;  // batched form: segment c = cluster [padoff[c],
-    int maxseg;                      // padoff[c + 1]), work-array chunk 0; maxseg its
-};                                   // longest segment
+    const int *__restrict__ padoff;  // batched form: bucket c = segment c % nseg_c of cluster
+};                                   // c / nseg_c in [padoff[..], ..), work-array chunk 0
 
 __device__ __forceinline__ IF64 load_if64(const double *__restrict__ ib, int is, int r) {
     IF64 I;
@@ -2204,38 +2203,55 @@ __device__ __forceinline__ IF64 load_if64(const double *__restrict__ ib, int is,
     return I;
 }
 
-// Prefix sums over the buckets in LDS (spre[nchunk + 1], wtot[4]): spre[c] = sum over the
-// buckets before c of their items in groups of `grp`.  All 256 threads; nchunk <= SEGCNT_LDS.
-__device__ __forceinline__ void bucket_prefix(const ChunkFixParams &f, int grp, int *spre,
-                                              int *wtot) {
+// The items of all buckets, in groups of `grp` of one bucket, as one list: LDS prefix sums
+// over runs of `run` consecutive buckets, one entry per run (a bucket each up to SEGCNT_LDS of
+// them, as every plain call has; ensembles can have more).
+// A list that is dealt out whole keeps the work even however many buckets there are: bucket
+// by bucket, each from the first work-group on, 4200 clusters of 100 took 8.9 ms a step in
+// place of 1.4.
+struct BucketList {
+    const int *spre;                 // [entries + 1]: groups before each run, then their number
+    int run, entries;
+};
+__device__ __forceinline__ int bucket_groups(const ChunkFixParams &f, int c, int grp) {
+    return c < f.nchunk ? (f.seg_cnt[c] + grp - 1) / grp : 0;
+}
+// spre: LDS[SEGCNT_LDS + 1], wtot: LDS[4].  All 256 threads.
+__device__ __forceinline__ BucketList bucket_list(const ChunkFixParams &f, int grp, int *spre,
+                                                  int *wtot) {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int per = (f.nchunk + 255) / 256;
+    const int run = (f.nchunk + SEGCNT_LDS - 1) / SEGCNT_LDS;
+    const int entries = (f.nchunk + run - 1) / run;
+    const int per = (entries + 255) / 256;
     int n = 0;
-    for (int q = 0; q < per; q++) {
-        const int c = t * per + q;
-        n += c < f.nchunk ? (f.seg_cnt[c] + grp - 1) / grp : 0;
-    }
+    for (int q = 0; q < per * run; q++) n += bucket_groups(f, t * per * run + q, grp);
     const int incl = wave_last(n);
     if (lane == 63) wtot[w] = incl;
     __syncthreads();
     int base = incl - n;
     for (int q = 0; q < w; q++) base += wtot[q];
     for (int q = 0; q < per; q++) {
-        const int c = t * per + q;
-        if (c >= f.nchunk) break;
-        spre[c] = base;
-        base += (f.seg_cnt[c] + grp - 1) / grp;
+        const int e = t * per + q;
+        if (e >= entries) break;
+        spre[e] = base;
+        for (int r = 0; r < run; r++) base += bucket_groups(f, e * run + r, grp);
     }
-    if (t == 0) spre[f.nchunk] = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+    if (t == 0) spre[entries] = wtot[0] + wtot[1] + wtot[2] + wtot[3];
     __syncthreads();
+    return {spre, run, entries};
 }
-// the last bucket c with spre[c] <= g
-__device__ __forceinline__ int find_bucket(const int *spre, int n, int g) {
-    int c = 0, hi = n;
-    while (hi - c > 1) {
-        const int mid = (c + hi) >> 1;
-        if (spre[mid] <= g) c = mid; else hi = mid;
+// bucket of group g of the list, and the groups before that bucket's first
+__device__ __forceinline__ int find_bucket(const ChunkFixParams &f, const BucketList &l, int grp,
+                                           int g, int &first) {
+    int e = 0, hi = l.entries;           // the last run with spre[e] <= g
+    while (hi - e > 1) {
+        const int mid = (e + hi) >> 1;
+        if (l.spre[mid] <= g) e = mid; else hi = mid;
     }
+    first = l.spre[e];
+    int c = e * l.run;
+    if (l.run > 1)
+        for (int n; g >= first + (n = bucket_groups(f, c, grp)); c++) first += n;
     return c;
 }
 // bucket c's item list: one of ni entries, or (batched form: (cluster, segment) c) of its
@@ -2247,20 +2263,18 @@ __device__ __forceinline__ const int *bucket_of(const ChunkFixParams &f, int c) 
     return f.seg_items + (size_t)p0 * f.nseg_c + (size_t)sg * (f.padoff[cl + 1] - p0);
 }
 
-// one wavefront per item, the items of all buckets dealt evenly (spre: LDS[SEGCNT_LDS + 1],
-// wtot: LDS[4]); more buckets than that: every bucket in turn
+// one wavefront per item, the items of all buckets dealt evenly
 template <bool MFLAG>
 __device__ __forceinline__ void cand_body(const ChunkFixParams &f, int bid, int nblk, int *spre,
                                           int *wtot) {
     const int lane = threadIdx.x & 63;
     const int w0 = __builtin_amdgcn_readfirstlane(bid * 4 + (threadIdx.x >> 6)), nw = nblk * 4;
-    const bool cached = f.nchunk <= SEGCNT_LDS;
-    if (cached) bucket_prefix(f, 1, spre, wtot);
-    for (int cb = 0; cb < (cached ? 1 : f.nchunk); cb++) {
-    const int total = cached ? spre[f.nchunk] : f.seg_cnt[cb];
+    const BucketList bl = bucket_list(f, 1, spre, wtot);
+    const int total = spre[bl.entries];
     for (int w = w0; w < total; w += nw) {
-        const int cw = cached ? find_bucket(spre, f.nchunk, w) : cb;
-        const int k = bucket_of(f, cw)[cached ? w - spre[cw] : w];
+        int first;
+        const int cw = find_bucket(f, bl, 1, w, first);
+        const int k = bucket_of(f, cw)[w - first];
         const int2 it = f.items[k];
         const int i = it.x, c = f.padoff ? 0 : it.y / f.nseg_c;   // work-array chunk
         // the segment's j range (the batched form: segment it.y % nseg_c of cluster
@@ -2296,7 +2310,6 @@ __device__ __forceinline__ void cand_body(const ChunkFixParams &f, int bid, int 
             for (int q = 0; q < 7; q++) f.cand[(size_t)k * 7 + q] = cd[q];
         }
     }
-    }
 }
 
 template <bool MFLAG>
@@ -2317,18 +2330,13 @@ __device__ __forceinline__ void segfix_body(const ChunkFixParams &f, int bid, in
                                             double2 (*st)[256], int *spre, int *wtot) {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const bool cached = f.nchunk <= SEGCNT_LDS;
-    if (cached) bucket_prefix(f, 64, spre, wtot);
-    // (more buckets than LDS has room for: every group that a bucket could have in turn)
-    const int gmax = ((f.padoff ? f.maxseg : f.ni) + 63) / 64;
-    const long long groups = cached ? spre[f.nchunk] : (long long)f.nchunk * gmax;
-    for (long long u = bid; u < groups * f.nsub; u += nblk) {   // uniform per work-group
-        const long long gi = u / f.nsub;
-        const int sub = (int)(u - gi * f.nsub);
-        const int c = cached ? find_bucket(spre, f.nchunk, (int)gi) : (int)(gi / gmax);
-        const int i0 = 64 * (cached ? (int)gi - spre[c] : (int)(gi - (long long)c * gmax));
-        const int nc = f.seg_cnt[c];
-        if (i0 >= nc) continue;
+    const BucketList bl = bucket_list(f, 64, spre, wtot);
+    const long long units = (long long)spre[bl.entries] * f.nsub;
+    for (long long u = bid; u < units; u += nblk) {   // uniform per work-group
+        const int gi = (int)(u / f.nsub), sub = (int)(u - (long long)gi * f.nsub);
+        int first;
+        const int c = find_bucket(f, bl, 64, gi, first);
+        const int i0 = 64 * (gi - first), nc = f.seg_cnt[c];
         // (the last chunk or a short cluster: trailing sub-ranges are empty and write 0)
         int sb, se;
         if (f.padoff) {
@@ -2444,12 +2452,13 @@ template <bool MFLAG>
 __device__ __forceinline__ void segfix_small_body(const ChunkFixParams &f, int bid, int nblk,
                                                   double (*red)[4][7], int *wtot, int *spre) {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    bucket_prefix(f, 4, spre, wtot);
-    const long long units = (long long)spre[f.nchunk] * f.nsub;
+    const BucketList bl = bucket_list(f, 4, spre, wtot);
+    const long long units = (long long)spre[bl.entries] * f.nsub;
     for (long long u = bid; u < units; u += nblk) {   // uniform per work-group
         const int gi = (int)(u / f.nsub), sub = (int)(u - (long long)gi * f.nsub);
-        const int c = find_bucket(spre, f.nchunk, gi);
-        const int i0 = (gi - spre[c]) * 4, nc = f.seg_cnt[c];
+        int first;
+        const int c = find_bucket(f, bl, 4, gi, first);
+        const int i0 = (gi - first) * 4, nc = f.seg_cnt[c];
         const int *bucket = f.seg_items + (size_t)c * f.ni;
         const int im = i0 + (lane >> 4);
         const bool ok = im < nc;
@@ -3005,7 +3014,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
             cp.cand = cand; cp.part64 = part64;
             cp.rowsel = rowsel; cp.nrows = nrows;
             cp.out = bout; cp.out_stride = ni_stride;
-            cp.padoff = nullptr; cp.maxseg = 0;
+            cp.padoff = nullptr;
             if (timed && b0 == 0) t4.start(s);
             // whole-row FP64 pass (rows with NaN sums, rows with more segments than
             // they may store; their count stays on the device) with the last batch,
@@ -3234,7 +3243,7 @@ int regf_items_launch(const JSet &js, int nslots, const int *imap, int stride, c
         cp.cand = cand; cp.part64 = part64;
         cp.rowsel = rowsel; cp.nrows = ctr + 2;
         cp.out = d_out; cp.out_stride = stride;
-        cp.padoff = padoff; cp.maxseg = maxseg;
+        cp.padoff = padoff;
         if (m_flag) {
             hipLaunchKernelGGL(regf_cand_kernel<true>, dim3(CHUNKFIX_GROUPS), dim3(256), 0, s, cp);
             hipLaunchKernelGGL(regf_segfix_kernel<true>, dim3(CHUNKFIX_GROUPS), dim3(256), 0, s, cp);
