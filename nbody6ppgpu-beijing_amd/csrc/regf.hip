@@ -443,8 +443,10 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
 // takes r2 - |2 dtr rv|, which is no larger than r2 + 2 dtr min(rv, 0) and needs no minimum (an
 // instruction of half the rate), and a branch to the full test where a lane passes it.  The
 // full test decides, so candidates, their order and the sums are pair_step's, bit for bit.
-// Returns the first j not done: that of a pair for which a lane has no slot left (the caller
-// goes on with pair_step, which knows overflowing rows), or j0 + RF_FLUSH.
+// Returns the first j not done: that of a hard pair for which a lane has no slot left (the
+// caller goes on with pair_step, which knows overflowing rows), or j0 + RF_FLUSH.  A soft pair
+// without a slot stays in the sums here: leaving at each of them took the dense rows of few
+// long chunks out of the loop (one cluster of 65,536 in an ensemble 17.8 ms, 14.1 so).
 // Tile kernel (the loop that the compiler made, then this one): N = 100,003, ni = 6007 with
 // m_flag, where 99 % of the tiles are tested, 640 -> 564 us; N = 65,536, ni = 1024
 // (all) 100 -> 86 us; send and force of N = 2^20, ni = 2^17 (9 %) 92.8 -> 89.5 ms.
@@ -508,15 +510,15 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
     "v_fmac_f32 v36, v16, " V "\n"                                                          \
     "v_fmac_f32 v33, v16, " W "\n"                                                          \
     "v_fmac_f32 v37, v20, v21\n"
-// a pair's candidates: to the lanes' next slots (leaving the loop where one has none) ...
+// a pair's candidates: to the lanes' next slots (leaving the loop where a hard one has none)
 #define NEAR_SLOTS(K)                                                                       \
     "s_add_i32 %[j], %[jb], " K "\n"                                                        \
     "v_cmp_le_i32 vcc, %[caph], v46\n"                                                      \
     "s_and_b64 vcc, vcc, %[h]\n"                                                            \
     "s_cbranch_scc1 .Lx_%=\n"                                                               \
-    "v_cmp_le_i32 vcc, %[lim], v47\n"                                                       \
-    "s_and_b64 vcc, vcc, %[f]\n"                                                            \
-    "s_cbranch_scc1 .Lx_%=\n"                                                               \
+    "v_cmp_gt_i32 vcc, %[lim], v47\n"                                                       \
+    "s_and_b64 %[f], %[f], vcc\n"                                                           \
+    "s_or_b64 %[x], %[h], %[f]\n"                                                           \
     "v_mov_b32 v23, %[j]\n"                                                                 \
     "s_mov_b64 exec, %[h]\n"                                                                \
     "s_cbranch_execz .Lf" K "_%=\n"                                                         \
