@@ -2765,17 +2765,6 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     // a chunk cannot hold more candidates than records
     const int caph = std::min(nnbeff + 8, clen);
     const int caps = std::min(CAP_SOFT, clen);
-    // the finalize form depends on the whole call, never on the batching below, so a
-    // batched call gives the same bits as an unbatched one
-    // one wavefront per i where there are enough i to fill the GPU (N = 65,536: 703 us with
-    // one and 1034 us with four at ni = 65,536, 448 and 601 at 40,000; N = 100,003,
-    // ni = 20,011: 247 and 292); below that each i's chunks are dealt to four wavefronts
-    // (N = 65,536: 225 us against 257 at ni = 16,000, 117 against 225 at 6,000), and to
-    // eight in the smallest calls, where even those leave wavefront slots free (53 us
-    // against 59 with four at ni = 1024, 105 against 93 at 3,000)
-    const int fin_form = ni > FIN_WIDE_NI || nchunk < 2 ? 1
-                                                        : (ni <= FIN_WIDEST_NI && nchunk >= 16 ? 8 : 4);
-
     // Work arrays hold one row per (i, chunk): FP64 partials, counts and the hard and
     // soft candidate slots.  Calls whose rows would exceed the slot budget run in
     // batches of i (whole i-blocks); chunks and results do not change.
@@ -2805,6 +2794,21 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
         nbatch_i = (int)std::max<size_t>((size_t)nbi, rows_max / (size_t)nchunk / nbi * nbi);
         nbatch_i = std::min(nbatch_i, ni);
     }
+    // The finalize form depends on the whole call, never on the batching, so a batched call
+    // gives the same bits as an unbatched one; only with caller work memory, where the chunks
+    // differ from those of the unbatched call anyway, the batch's size decides:
+    // one wavefront per i where there are enough i to fill the GPU (N = 65,536: 703 us with
+    // one and 1034 us with four at ni = 65,536, 448 and 601 at 40,000; N = 100,003,
+    // ni = 20,011: 247 and 292); below that each i's chunks are dealt to four wavefronts
+    // (N = 65,536: 225 us against 257 at ni = 16,000, 117 against 225 at 6,000), and to
+    // eight in the smallest calls, where even those leave wavefront slots free (53 us
+    // against 59 with four at ni = 1024, 105 against 93 at 3,000; ni = 65,536 in caller work
+    // memory, 512 at a time: 34.7 ms a call with eight, 54.8 with one).
+    const int fin_ni = na ? nbatch_i : ni;
+    const int fin_form = fin_ni > FIN_WIDE_NI || nchunk < 2
+                             ? 1
+                             : (fin_ni <= FIN_WIDEST_NI && nchunk >= 16 ? 8 : 4);
+
     // 64 i per work-group and the tile's four pieces side by side (the same bits) up to 1792
     // such work-groups, seven per CU; with more the 256-wide form fills the GPU by itself and
     // adds up its pieces without LDS.  Whole call: N = 65,536, ni = 256 (1024 of them)
