@@ -133,7 +133,11 @@ int nb6_regf_device(int ni, int ni_stride, const double *d_i, int lmax, int nnbm
 int nb6_regf_device_noalloc(int ni, int ni_stride, const double *d_i, int lmax, int nnbmax,
                             int m_flag, double *d_out, int *d_list, void *stream);
 
-/* Device-resident j upload: d_j is SoA double[7][nj_stride] (x,y,z,vx,vy,vz,m). */
+/* Device-resident j upload: d_j is SoA double[7][nj_stride] (x,y,z,vx,vy,vz,m).  Returns
+ * when d_j has been read; the j-set is then being built on `stream`, and this library's
+ * later calls that use it wait for that, also on another stream.  A call that still runs
+ * (asynchronously, on another stream) when a new j-set is sent, and a graph that the caller
+ * captured and replays, are the caller's to order. */
 int nb6_send_device(int nj, int nj_stride, const double *d_j, void *stream);
 
 /* Device-resident potential: d_x SoA double[4][n_stride] (x,y,z,m) for all n

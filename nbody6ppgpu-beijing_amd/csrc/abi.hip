@@ -291,11 +291,13 @@ void gpunb_send_(int *nj, double mj[], double xj[][3], double vj[][3]) {
     }
     g.time_send -= tstart;   // the pack counts as send time
     g.isend++;
+    jset_ready(g.js, d.stream);
     if (n > 0)
         NB6_HIP(hipMemcpyAsync(g.js.in64.p, h, (size_t)8 * n * sizeof(double),
                                hipMemcpyHostToDevice, d.stream));
     jset_build(g.js, n, box, mmax, d.stream);
     NB6_HIP(hipStreamSynchronize(d.stream));
+    g.js.pending = false;
     g.time_send += wtime();
 }
 
@@ -703,6 +705,7 @@ void nb6_jp_predict_send_(double *time, int *nj) {
     if (n < 0 || n > g.nbmax) { set_error(E_ARG, "nb6_jp_predict_send: nj outside [0, nbmax]"); return; }
     const double t0 = wtime();
     Device &d = device();
+    jset_ready(g.js, d.stream);
     if (jp_predict(*time, n, g.js.in64.as<double>(), d.stream) != OK) return;
     jset_build(g.js, n, nullptr, 0.0, d.stream);
     g.isend++;

@@ -449,6 +449,7 @@ const int *irr_order(int ni, const int *d_addr, const int **oaddr, hipStream_t s
     const JSet *js = gpunb_jset();
     *oaddr = d_addr;
     if (!g_irrcfg.sort_i || ni < 2048 || !js || js->n <= 0) return nullptr;
+    jset_ready(*js, s);
     unsigned long long *kb =
         static_cast<unsigned long long *>(g.d_okey.get((size_t)ni * 2 * sizeof(unsigned long long)));
     int *v0 = static_cast<int *>(g.d_oval.get((size_t)ni * 4 * sizeof(int)));

@@ -343,16 +343,54 @@ void jset_release(JSet &js) {
     js.sort_tmp.release(); js.tbox.release();
     js.cap = 0; js.n = 0; js.ntile = 0;
     if (js.read) (void)hipEventDestroy(js.read);
-    js.read = nullptr;
+    if (js.built) (void)hipEventDestroy(js.built);
+    js.read = js.built = nullptr;
+    js.pending = js.recorded = false;
 }
 
-// The caller's input has been read once the work queued so far is done; a send returns after
-// that (its caller may then reuse the memory, on any stream), not after the whole build.
+// The caller's input has been read, and in64 written, once the work queued so far is done; a
+// send returns after that (its caller may then reuse the memory, on any stream), not after the
+// whole build.
 void jset_input_queued(JSet &js, hipStream_t s) {
     if (!js.read) NB6_HIP(hipEventCreateWithFlags(&js.read, hipEventDisableTiming));
     NB6_HIP(hipEventRecord(js.read, s));
 }
 void jset_input_wait(JSet &js) { NB6_HIP(hipEventSynchronize(js.read)); }
+
+// A build is queued when its send returns.  Work on its own stream follows it there; work on
+// another stream waits for an event after it.  The library's stream lives as long as the
+// library, so there the event is recorded when another stream asks; a caller's stream can be
+// gone by then and gets it at once.
+namespace {
+void record_built(const JSet &js) {
+    if (!js.built) NB6_HIP(hipEventCreateWithFlags(&js.built, hipEventDisableTiming));
+    NB6_HIP(hipEventRecord(js.built, js.stream));
+    js.recorded = true;
+}
+void build_queued(JSet &js, hipStream_t s) {
+    js.stream = s;
+    js.pending = true;
+    js.recorded = false;
+    if (s != device().stream) record_built(js);
+}
+}  // namespace
+void jset_ready(const JSet &js, hipStream_t s) {
+    if (!js.pending || s == js.stream) return;
+    // A captured call runs when its graph does, which the caller orders; a stream under capture
+    // can neither wait for an event from outside nor may the thread wait for one meanwhile.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    NB6_HIP(hipStreamIsCapturing(s, &cs));
+    if (cs != hipStreamCaptureStatusNone) return;
+    if (!js.recorded) record_built(js);
+    const hipError_t e = hipEventQuery(js.built);
+    if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+        NB6_HIP(hipStreamWaitEvent(s, js.built, 0));
+        return;
+    }
+    NB6_HIP(e);
+    js.pending = false;
+}
 
 namespace {
 int stat_groups(int n) { return std::min(STATS_GROUPS, (n + 255) / 256); }
@@ -382,6 +420,7 @@ void build(JSet &js, int n, int groups, const JStat &host, hipStream_t s) {
                        v1, nullptr, nullptr, nullptr, 0, js.rec64.as<double>(), js.torg.as<double>(),
                        js.rec32.as<float4>(), js.tbox.as<float>());
     NB6_HIP(hipGetLastError());
+    build_queued(js, s);
 }
 }  // namespace
 
@@ -397,8 +436,10 @@ void jset_build(JSet &js, int n, const double *box, double mmax, hipStream_t s) 
         hipLaunchKernelGGL(aos_stats_kernel, dim3(groups), dim3(256), 0, s, nullptr, n, 0,
                            js.in64.as<double>(), js.stat.as<double>() + 8);
         NB6_HIP(hipGetLastError());
+        jset_input_queued(js, s);
     }
     build(js, n, groups, host, s);
+    if (groups > 0) jset_input_wait(js);     // in64 is written
 }
 
 void jset_build_clusters(JSet &js, int npad, const double *in, const int *sorted, const int *off,
@@ -502,6 +543,7 @@ void jset_from_soa(JSet &js, int n, int stride, const double *d_soa, hipStream_t
         build(js, n, 0, JStat{}, s);
         return;
     }
+    jset_ready(js, s);
     const int groups = stat_groups(n);
     hipLaunchKernelGGL(aos_stats_kernel, dim3(groups), dim3(256), 0, s, d_soa, n, stride,
                        js.in64.as<double>(), js.stat.as<double>() + 8);

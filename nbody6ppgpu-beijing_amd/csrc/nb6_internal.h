@@ -88,6 +88,10 @@ struct JSet {
     int cap = 0;
     int ntile = 0;
     hipEvent_t read = nullptr;   // the caller's input has been read (jset_input_queued)
+    // the last build: its stream, and until it is known to be done (jset_ready) an event after it
+    hipStream_t stream = nullptr;
+    mutable hipEvent_t built = nullptr;
+    mutable bool pending = false, recorded = false;
     DBuf in64, rec64, rec32, torg, perm, keys, vals, stat, sort_tmp, tbox;
 };
 // Work-group b of G -> position in the work order such that XCD x (work-groups are
@@ -111,6 +115,8 @@ void jset_build_clusters(JSet &js, int npad, const double *in, const int *sorted
 // a send's input is read by the work queued on s up to here / wait for that
 void jset_input_queued(JSet &js, hipStream_t s);
 void jset_input_wait(JSet &js);
+// work queued on s from here on finds the j-set complete, whichever stream it was built on
+void jset_ready(const JSet &js, hipStream_t s);
 // Rows [count, entries...] of a [n][lmax] list array packed end to end on the device:
 // off[i] (n + 1 entries, off[n] = total) and pack[off[i] .. off[i + 1]) = the row's
 // 1 + count leading ints (only the count if it is negative or above maxc); len is

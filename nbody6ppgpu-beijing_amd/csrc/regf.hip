@@ -2904,6 +2904,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     }
     g_last_refine = refine;
 
+    jset_ready(js, s);
     // Morton-ordered i: a wavefront's particles are neighbours in space, so their
     // candidates fall on the same j and most tiles are far from all of them
     const int *imap = !na && cfg.isort_min > 0 && ni >= cfg.isort_min

@@ -867,6 +867,7 @@ int rs_kth(const JSet &js, int ni, int ib_stride, const double *ib, const int *l
            double *rs_out, hipStream_t s) {
     if (ni <= 0) return OK;
     if (k < 1 || lmax < 2) { set_error(E_ARG, "nb6_rs_kth_device: need k >= 1 and lmax >= 2"); return E_ARG; }
+    jset_ready(js, s);
     hipLaunchKernelGGL(rs_kth_kernel, dim3((ni + 3) / 4), dim3(256), 0, s, ni, ib_stride, ib, list,
                        lmax, k, js.in64.as<double>(), js.n, rs_out);
     NB6_HIP(hipGetLastError());
