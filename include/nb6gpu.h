@@ -231,8 +231,8 @@ int nb6_set_regf_debug_bounds(double *d_bounds);
  *     for all particles, d_out SoA double[7][stride], d_list int[ntot][lmax] with
  *     0-based indices relative to the particle's own cluster.  One persistent
  *     launch over (cluster, i-block) work items; use_graph=1 captures the step
- *     into a hipGraph on the first call and replays it while the pointers and
- *     sizes stay the same.  Results equal gpunb_send_ + gpunb_regf_ per cluster. */
+ *     into a hipGraph on the first call and replays it while the pointers, the
+ *     cluster layout's sizes and the settings stay the same.  Results equal gpunb_send_ + gpunb_regf_ per cluster. */
 int nb6_ens_open(int max_clusters, int max_particles);
 int nb6_ens_close(void);
 int nb6_ens_send_device(int nclusters, const int *offsets, const double *d_soa, int stride,
@@ -247,7 +247,7 @@ int nb6_ens_last_refined(void);
 /* Autotuners (run on the caller's own, already sent, inputs; outputs are
  * overwritten).  They time every combination of work-group size = LDS j-tile
  * (128, 256, 512), i-particles per lane (1, 2; i-block 128..1024) and occupancy
- * (regf: minimum work-groups 1024/2048/4096 through j-chunking; ensemble: 8, 16
+ * (regf: minimum work-groups 2048/4096/8192 through j-chunking; ensemble: 8, 16
  * or 32 wavefronts per CU in the persistent launch), keep the fastest as the
  * library's configuration and report best = {threads, i_per_lane, min_groups or
  * work-groups per CU, time in microseconds}. */

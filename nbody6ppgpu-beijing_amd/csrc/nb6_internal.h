@@ -121,10 +121,12 @@ void jset_ready(const JSet &js, hipStream_t s);
 // off[i] (n + 1 entries, off[n] = total) and pack[off[i] .. off[i + 1]) = the row's
 // 1 + count leading ints (only the count if it is negative or above maxc); len is
 // n + 1 ints of scratch (jset.hip).
-void deliver_rows(const double *res, const int *list, int ni, int lmax, int nnbmax, double *out,
-                  int *rows, hipStream_t s);
 void pack_rows(const int *list, int n, int lmax, int maxc, int *len, int *off, int *pack,
                DBuf &tmp, hipStream_t s);
+// SoA results res[7][ni] and the used part of each row of list[ni][lmax] into pinned host
+// memory: out[ni][8] and rows[ni][lmax] (jset.hip).
+void deliver_rows(const double *res, const int *list, int ni, int lmax, int nnbmax, double *out,
+                  int *rows, hipStream_t s);
 
 struct RegfConfig {
     int threads = 0;      // work-group size = LDS j-tile (128, 256 or 512; 0: by ni)

@@ -2154,9 +2154,10 @@ __global__ __launch_bounds__(256) void regf_fix_reduce_kernel(FixParams f) {
 // (pair64, the finalize's test), minus the candidates the finalize already added in
 // FP64 (the same slots and tests as fin_candidates), minus the chunk's FP32 partials.
 //  * regf_cand_kernel: one wavefront per item, the candidate terms -> cand[k];
-//  * regf_segfix_kernel: work units (chunk c, up to 256 of its items, sub-range s of
-//    FIX_SUB j): the sub-range's records pass through LDS once for all the unit's items,
-//    one thread per item -> part64[k][s];
+//  * regf_segfix_kernel: work units (chunk c, up to 64 of its items, sub-range s of FIX_SUB
+//    j): a lane per item, each of four wavefronts with a quarter of the sub-range, whose records
+//    it takes through LDS -> part64[k][s]; small calls: up to four items, 16 lanes each
+//    (segfix_small_body);
 //  * regf_segapply_kernel: each row adds, in item and sub-range order,
 //    sum_s part64 - cand - FP32 partial of every one of its items.
 // Every value depends only on (i, c, s), so results do not depend on the order in which
@@ -2164,7 +2165,7 @@ __global__ __launch_bounds__(256) void regf_fix_reduce_kernel(FixParams f) {
 constexpr int FIX_SUB = 1024;          // j per sub-range
 constexpr int SEG_MIN = 8192;          // shortest partial-sum segment
 constexpr int SEG_ENS = 4096;          // partial-sum segment of a cluster (batched form)
-constexpr int SEGCNT_LDS = 4096;       // bucket sizes the segment-sum kernel keeps in LDS
+constexpr int SEGCNT_LDS = 4096;       // entries of the bucket lists in LDS (bucket_list)
 constexpr size_t ITEM_BUDGET = 4ull << 30;   // FP64-pass item memory aimed at per call
 constexpr int MIN_ROW_ITEMS = 8;
 constexpr int PASS_MERGE_NI = 16384;   // batches up to this many i: the FP64 pass in two launches
@@ -2183,13 +2184,10 @@ struct ChunkFixParams {
     const int *__restrict__ sslot;
     int caps;
     const int2 *__restrict__ items;
-    const int *__restrict__ nitems;
-    int item_cap;
-    int row_items;                   // most items of one row entry (1 in the batched form)
     const int *__restrict__ seg_items;
     const int *__restrict__ seg_cnt;
-    double *__restrict__ cand;       // [item_cap][7]
-    double *__restrict__ part64;     // [item_cap][nsub][7]
+    double *__restrict__ cand;       // [items][7]
+    double *__restrict__ part64;     // [items][nsub][7]
     const int4 *__restrict__ rowsel;
     const int *__restrict__ nrows;
     double *__restrict__ out;        // SoA [7][out_stride] (of the batch)
@@ -2765,6 +2763,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     // a chunk cannot hold more candidates than records
     const int caph = std::min(nnbeff + 8, clen);
     const int caps = std::min(CAP_SOFT, clen);
+
     // Work arrays hold one row per (i, chunk): FP64 partials, counts and the hard and
     // soft candidate slots.  Calls whose rows would exceed the slot budget run in
     // batches of i (whole i-blocks); chunks and results do not change.
@@ -2803,7 +2802,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     // (N = 65,536: 225 us against 257 at ni = 16,000, 117 against 225 at 6,000), and to
     // eight in the smallest calls, where even those leave wavefront slots free (53 us
     // against 59 with four at ni = 1024, 105 against 93 at 3,000; ni = 65,536 in caller work
-    // memory, 512 at a time: 34.7 ms a call with eight, 54.8 with one).
+    // memory, 512 at a time: 34.6 ms a call with eight, 54.8 with one).
     const int fin_ni = na ? nbatch_i : ni;
     const int fin_form = fin_ni > FIN_WIDE_NI || nchunk < 2
                              ? 1
@@ -3015,8 +3014,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
             cp.ni = nb; cp.nsub = nsub; cp.nseg_c = P;
             cp.part = part; cp.cnt = cnt; cp.hslot = hslot; cp.caph = caph;
             cp.sslot = sslot; cp.caps = caps;
-            cp.items = items; cp.nitems = nitems; cp.item_cap = fp.item_cap;
-            cp.row_items = std::max(row_items, 1);
+            cp.items = items;
             cp.seg_items = seg_items; cp.seg_cnt = seg_cnt;
             cp.cand = cand; cp.part64 = part64;
             cp.rowsel = rowsel; cp.nrows = nrows;
@@ -3037,7 +3035,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
             // grids no larger than the work there can be (small calls launch small
             // grids); whole rows: at most (ni / 256 row groups) x (j tiles) items
             const int gc = (int)std::min<size_t>(CHUNKFIX_GROUPS,
-                                                 ((size_t)nb * cp.row_items + 3) / 4);
+                                                 ((size_t)nb * std::max(row_items, 1) + 3) / 4);
             // (by the whole call's size: a batched call gives the same bits)
             const bool few = ni <= PASS_MERGE_NI && nseg <= SEGCNT_LDS;
             const size_t ig = few ? 4 : 64;           // items per work unit
@@ -3236,16 +3234,15 @@ int regf_items_launch(const JSet &js, int nslots, const int *imap, int stride, c
         hipLaunchKernelGGL(regf_finalize_kernel<false>, fgrid, dim3(256), 4 * rl, s, fp);
     NB6_HIP(hipGetLastError());
     if (refine) {
-        // FP64 pass of the flagged rows: items bucketed by cluster, each cluster's records
-        // through LDS once per 256 of its rows
+        // FP64 pass of the flagged rows: items bucketed by cluster and segment, a segment's
+        // records through LDS once per 64 of its items
         ChunkFixParams cp{};
         cp.ib = d_i; cp.ib_stride = stride; cp.imap = imap;
         cp.rec64 = js.rec64.as<double>(); cp.nj = js.n; cp.clen = sege; cp.nchunk = (int)nbk;
         cp.ni = nslots; cp.nsub = nsub; cp.nseg_c = nsegc;
         cp.part = part; cp.cnt = cnt; cp.hslot = hslot; cp.caph = caph;
         cp.sslot = sslot; cp.caps = caps;
-        cp.items = fitems; cp.nitems = ctr + 1; cp.item_cap = fp.item_cap;
-        cp.row_items = nsegc;            // a row's items: at most one per segment
+        cp.items = fitems;
         cp.seg_items = seg_items; cp.seg_cnt = ctr + 6;
         cp.cand = cand; cp.part64 = part64;
         cp.rowsel = rowsel; cp.nrows = ctr + 2;

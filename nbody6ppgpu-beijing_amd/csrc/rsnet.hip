@@ -131,11 +131,12 @@ struct GradLds {
     float dy[GB];
 };
 
-// 64 x 64 x 64 products of the hidden layer on the matrix cores, NT blocks of 16 x 16 by
-// wavefront w: rows 16 mt .. 16 mt + 15, columns from 16 n0 on: C[m][n] = sum_k A(m, k) B(k, n), A and B read through the callables
-// (LDS), each element of C handed to out(m, n, c).  v_mfma_f32_16x16x4f32 (FP32 in, FP32
-// accumulate): lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] of a 16 x 4 and
-// a 4 x 16 block, and holds C[4 (l / 16) + i][l % 16], i = 0..3, of the 16 x 16 block.
+// 64 x 64 x 64 products of the hidden layer on the matrix cores: C[m][n] = sum_k A(m, k)
+// B(k, n), A and B read through the callables (LDS), each element of C handed to out(m, n, c).
+// Wavefront w takes NT blocks of 16 x 16: rows 16 mt .. 16 mt + 15, columns from 16 n0 on.
+// v_mfma_f32_16x16x4f32 (FP32 in, FP32 accumulate): lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16] of a 16 x 4 and a 4 x 16 block, and holds C[4 (l / 16) + i][l % 16],
+// i = 0..3, of the 16 x 16 block.
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int GW = 8;
 template <class FA, class FB, class FO>
