@@ -195,6 +195,16 @@ __device__ __forceinline__ IC tile_ic(const ILane &L, const double *__restrict__
     return c;
 }
 
+// For a row without a soft slot left: a soft pair stays in the sums, so only hard pairs need
+// to be found, and the soft thresholds (also those of lane_far and of the cheap test, which bounds
+// any threshold) fall to the hard ones, from the next tile on.  Otherwise near_loop is left at
+// every further soft pair of the chunk: one cluster of 65,536 in an ensemble 17.8 -> 10.4 ms
+// (17.3 with the loop that the compiler makes), four of 65,536 26.2 -> 19.0.
+__device__ __forceinline__ void only_hard(IC &c) {
+    c.hS = c.hH; c.dS = c.dH;
+    c.hQ = c.hH * (1.0f + Q_REL); c.dQ = c.dH * (1.0f + Q_REL);
+}
+
 // True when no pair of this lane's i with the 256-j tile whose bounds are B can be a
 // hard or soft candidate, so the per-pair test can be skipped for the whole tile.
 // The loop records a candidate only if min(r2, r2p - KAPPA_P r2) < ths, with
@@ -443,10 +453,8 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
 // takes r2 - |2 dtr rv|, which is no larger than r2 + 2 dtr min(rv, 0) and needs no minimum (an
 // instruction of half the rate), and a branch to the full test where a lane passes it.  The
 // full test decides, so candidates, their order and the sums are pair_step's, bit for bit.
-// Returns the first j not done: that of a hard pair for which a lane has no slot left (the
-// caller goes on with pair_step, which knows overflowing rows), or j0 + RF_FLUSH.  A soft pair
-// without a slot stays in the sums here: leaving at each of them took the dense rows of few
-// long chunks out of the loop (one cluster of 65,536 in an ensemble 17.8 ms, 14.1 so).
+// Returns the first j not done: that of a pair for which a lane has no slot left (the caller
+// goes on with pair_step, which knows overflowing rows), or j0 + RF_FLUSH.
 // Tile kernel (the loop that the compiler made, then this one): N = 100,003, ni = 6007 with
 // m_flag, where 99 % of the tiles are tested, 640 -> 564 us; N = 65,536, ni = 1024
 // (all) 100 -> 86 us; send and force of N = 2^20, ni = 2^17 (9 %) 92.8 -> 89.5 ms.
@@ -516,9 +524,9 @@ __device__ __forceinline__ void far_loop(const float4 *sA, const float4 *sB, con
     "v_cmp_le_i32 vcc, %[caph], v46\n"                                                      \
     "s_and_b64 vcc, vcc, %[h]\n"                                                            \
     "s_cbranch_scc1 .Lx_%=\n"                                                               \
-    "v_cmp_gt_i32 vcc, %[lim], v47\n"                                                       \
-    "s_and_b64 %[f], %[f], vcc\n"                                                           \
-    "s_or_b64 %[x], %[h], %[f]\n"                                                           \
+    "v_cmp_le_i32 vcc, %[lim], v47\n"                                                       \
+    "s_and_b64 vcc, vcc, %[f]\n"                                                            \
+    "s_cbranch_scc1 .Lx_%=\n"                                                               \
     "v_mov_b32 v23, %[j]\n"                                                                 \
     "s_mov_b64 exec, %[h]\n"                                                                \
     "s_cbranch_execz .Lf" K "_%=\n"                                                         \
@@ -703,6 +711,7 @@ __device__ __forceinline__ void tile_work(const TileParams &p, int ibase, int ie
     }
 
     const int ntile = (j1 - j0 + T - 1) / T;
+    const bool longc = p.chunk_len > CAP_SOFT;   // (else slots for nearly every record)
     int segw = 0;                    // partial-sum segment being summed
 
     // Tile t goes straight from HBM into LDS buffer t & 1 (global_load_lds_dwordx4:
@@ -739,6 +748,7 @@ __device__ __forceinline__ void tile_work(const TileParams &p, int ibase, int ie
 #pragma unroll
                 for (int k = 0; k < IPL; k++) {
                     c[k] = tile_ic<MFLAG>(L[k], p.torg + tt * 8, p.tbox + tt * TBOX);
+                    if (longc && ns[k] >= p.caps - BAND_SLOTS) only_hard(c[k]);
                     if (p.far_test) far = far && lane_far<MFLAG>(c[k], L[k].ok, p.tbox + tt * TBOX);
                 }
                 allfar = __ballot(!far) == 0ull;
