@@ -2812,7 +2812,7 @@ int regf_launch_impl(const JSet &js, int ni, int ni_stride, const double *d_i, i
     // (N = 65,536: 225 us against 257 at ni = 16,000, 117 against 225 at 6,000), and to
     // eight in the smallest calls, where even those leave wavefront slots free (53 us
     // against 59 with four at ni = 1024, 105 against 93 at 3,000; ni = 65,536 in caller work
-    // memory, 512 at a time: 34.6 ms a call with eight, 54.8 with one).
+    // memory, 512 at a time: 36.0 ms a call with eight, 59.2 with one).
     const int fin_ni = na ? nbatch_i : ni;
     const int fin_form = fin_ni > FIN_WIDE_NI || nchunk < 2
                              ? 1
